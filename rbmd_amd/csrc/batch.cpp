@@ -2,7 +2,7 @@
 // include/rbmdx.h: many independent periodic boxes of one force field
 // (RBMD's JSON surface, LJ/CUT or LJ/CUT/COUL/LONG with RBL or a full pair
 // set and RBE k-space) evaluated together.  One evaluation of every replica
-// is one captured hipGraph (seven stage kernels over the whole batch, plus a
+// is one captured hipGraph (six stage kernels over the whole batch, plus a
 // one-thread epoch update launched before it); the same kernels launched one
 // replica at a time are the per-replica path.  Launch shapes come from a
 // measuring autotuner whose choice is cached as JSON per device and batch
@@ -239,8 +239,12 @@ class Batch {
       pc_.t_core = pc_.rs2 - e;
       pc_.t_shell = pc_.rc2 - e;
       pc_.eps_min = e;
-      pc_.a_lo = -1.f;
-      pc_.a_hi = pc_.rclj2;
+      // one interval for LJ pairs without shell pairs, as the single-system
+      // engine forms it
+      float hi = std::min(pc_.rclj2, pc_.rc2);
+      if (rbl) hi = std::min(hi, std::min(pc_.t_core, pc_.rs2));
+      pc_.a_hi = hi;
+      pc_.a_lo = rbl ? e : -1.f;
       pc_.alpha = (float)cfg_.alpha;
       pc_.g = (float)std::sqrt(cfg_.alpha);
       pc_.qqr2e = (float)cfg_.qqr2e;
@@ -278,21 +282,28 @@ class Batch {
     d_.gid = upload(std::vector<int>(id, id + N_));
     d_.charge = upload(qf);
     d_.lj = upload(lj);
-    d_.cnt = alloc<int>(ncell_);
-    d_.cntq = alloc<int>(ncell_);
-    HIPCHK(hipMemset(d_.cnt, 0, sizeof(int) * ncell_));
-    HIPCHK(hipMemset(d_.cntq, 0, sizeof(int) * ncell_));
+    d_.cnt = alloc<unsigned long long>(ncell_);
+    HIPCHK(hipMemset(d_.cnt, 0, sizeof(unsigned long long) * ncell_));
     d_.start = alloc<int>(ncell_ + 1);
     d_.qstart = alloc<int>(ncell_ + 1);
     d_.cell_of = alloc<int>(N_);
     d_.slot = alloc<int>(N_);
     d_.tmp = alloc<int>(N_);
     d_.xs = alloc<float4>(N_);
-    d_.tg = alloc<int2>(N_);
-    d_.hj = alloc<unsigned long long>(N_);
+    d_.gid_s = alloc<int>(N_);
     d_.perm = alloc<int>(N_);
-    d_.qidx = alloc<int>(std::max(1, NQ_));
+    {
+      std::vector<int> qp(N_, -1);
+      int k = 0;
+      for (int i = 0; i < N_; ++i)
+        if (qf[i] != 0.f) qp[i] = k++;
+      d_.qpos = upload(qp);
+    }
+    d_.xqc = alloc<float4>(NQ_);
+    d_.qi = alloc<int4>(NQ_);
     d_.fs = alloc<float4>(N_);
+    d_.fq = alloc<float4>(NQ_);
+    d_.fk = alloc<float4>(NQ_);
     d_.racc = alloc<double>((size_t)R * kBatchAcc);
     d_.kacc = alloc<double>((size_t)R * kBatchKAcc);
     HIPCHK(hipMemset(d_.racc, 0, sizeof(double) * R * kBatchAcc));
@@ -302,10 +313,13 @@ class Batch {
     size_t wmax = 0;
     for (const RepInfo& p : rep_) wmax += (size_t)p.nc[0] * p.nc[1] * p.nc[2];
     work_dev_ = alloc<BatchWork>(wmax);
+    // charged runs sized for one lane per thread and charged atom
+    qwork_dev_ = alloc<BatchWork>((size_t)NQ_ + R);
     rep_dev_ = alloc<RepInfo>(R);
     d_.work = work_dev_;
+    d_.qwork = qwork_dev_;
     d_.rep = rep_dev_;
-    layout(tune_.bw);
+    layout(tune_);
     ready_ = true;
   }
 
@@ -347,23 +361,34 @@ class Batch {
     drop_graphs();
   }
 
-  // Bricks of width bw: per-replica brick counts and the replica-major work
-  // list (one item per brick).
-  void layout(int bw) {
+  // The work lists of a launch shape, replica-major: the bricks of every
+  // replica (of width t.bw, or 1 where the neighbourhood of such a brick, its
+  // mean occupancy with margin, would overfill the LDS stage) and runs of
+  // pair_block / qlanes charged atoms.
+  void layout(const BatchTune& t) {
     w0_.assign(R_ + 1, 0);
-    std::vector<BatchWork> work;
+    x0_.assign(R_ + 1, 0);
+    std::vector<BatchWork> work, qwork;
+    const int per = t.pair_block / t.qlanes;
     for (int r = 0; r < R_; ++r) {
       RepInfo& p = rep_[r];
-      for (int d = 0; d < 3; ++d) p.nb[d] = (p.nc[d] + bw - 1) / bw;
+      const double apc = (double)p.n / ((double)p.nc[0] * p.nc[1] * p.nc[2]);
+      p.bw = 64.0 * apc * 1.1 <= kBatchStageCap ? t.bw : 1;
+      for (int d = 0; d < 3; ++d) p.nb[d] = (p.nc[d] + p.bw - 1) / p.bw;
       const int nb = p.nb[0] * p.nb[1] * p.nb[2];
       for (int b = 0; b < nb; ++b) work.push_back(BatchWork{r, b});
       w0_[r + 1] = w0_[r] + nb;
+      for (int c = 0; c < p.nq; c += per) qwork.push_back(BatchWork{r, p.q0 + c});
+      x0_[r + 1] = (int)qwork.size();
     }
     HIPCHK(hipMemcpy(rep_dev_, rep_.data(), sizeof(RepInfo) * R_, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(work_dev_, work.data(), sizeof(BatchWork) * work.size(),
                      hipMemcpyHostToDevice));
+    if (!qwork.empty())
+      HIPCHK(hipMemcpy(qwork_dev_, qwork.data(), sizeof(BatchWork) * qwork.size(),
+                       hipMemcpyHostToDevice));
     d_.nwork = (int)work.size();
-    layout_bw_ = bw;
+    layout_ = t;
     drop_graphs();
   }
 
@@ -377,7 +402,8 @@ class Batch {
     g.c1 = c0_[r1];
     g.w0 = w0_[r0];
     g.w1 = w0_[r1];
-    g.q0 = q0_[r0];
+    g.x0 = x0_[r0];
+    g.x1 = x0_[r1];
     return g;
   }
 
@@ -459,9 +485,10 @@ class Batch {
         t.qlanes > t.pair_block)
       throw Error(RBMDX_E_ARG, "launch shape out of range");
     tune_ = t;
-    if (ready_ && t.bw != layout_bw_) {
+    if (ready_ && (t.bw != layout_.bw || t.pair_block / t.qlanes !=
+                                             layout_.pair_block / layout_.qlanes)) {
       if (last_stream_set_) HIPCHK(hipStreamSynchronize(last_stream_));
-      layout(t.bw);
+      layout(t);
     }
     drop_graphs();
   }
@@ -692,11 +719,12 @@ class Batch {
   bool ready_ = false;
   int R_ = 0, N_ = 0, NQ_ = 0, ncell_ = 0, P_ = 0, ntypes_ = 0;
   std::vector<RepInfo> rep_;
-  std::vector<int> a0_, q0_, c0_, w0_;
+  std::vector<int> a0_, q0_, c0_, w0_, x0_;
   std::vector<double> self_;
   RepInfo* rep_dev_ = nullptr;
   BatchWork* work_dev_ = nullptr;
-  int layout_bw_ = 0;
+  BatchWork* qwork_dev_ = nullptr;
+  BatchTune layout_{};  // the shape the work lists are laid out for
   PairConst<float> pc_{};
   BatchDev d_{};
   BatchTune tune_{};

@@ -1,27 +1,29 @@
 // Replica-batch kernels: one force evaluation of many independent periodic
 // boxes of one force field (LJ + erfc Coulomb pairs with RBL or a full pair
-// set, RBE k-space), every stage one launch over a range of replicas:
+// set, sampled or Ewald k-space), every stage one launch over a range of
+// replicas:
 //
 //   kb_bin       wrap, cell of every atom, per-cell counts (atomics)
-//   kb_scan      per-cell offsets of atoms and charged atoms (one workgroup)
+//   kb_scan      per-cell offsets of atoms and charged atoms (a workgroup per
+//                replica)
 //   kb_scatter   cell buckets in arrival order
 //   kb_cellsort  per cell: charged atoms first, then by caller index (a
-//                deterministic order); sorted positions, types, ids, hashes
-//   kb_pair      persistent over the (replica, brick) work list: the brick's
-//                neighbourhood staged in LDS; LJ for every pair with a
-//                neutral atom, LJ + Coulomb for charged pairs (stencil of
-//                ext_c cells); FP64 energy, virial and force sum per replica
-//   kb_kspace    persistent over replicas: S(k) over the replica's charged
-//                atoms (FP64 across tiles), RBE energy and virial, and the
-//                k-space force of every charged atom
-//   kb_finish    mean pair force removed (RBL), forces to caller order
+//                deterministic order); sorted positions, types, ids, and the
+//                charged atoms' compact copy
+//   kb_eval      three kinds of workgroups in one launch: the k-space of a
+//                replica (S(k), energy, virial, force of its charged atoms),
+//                the LJ pairs of a brick (persistent over the (replica, brick)
+//                work list, the brick's neighbourhood staged in LDS) and the
+//                Coulomb pairs of a run of charged atoms; FP64 energy, virial
+//                and force sum per replica
+//   kb_finish    the three force rows added in caller order, mean pair force
+//                removed (RBL)
 //
 // Cells are rebuilt every evaluation (no skin, no stored lists), so an
 // evaluation has no host-side decisions and the whole sequence replays as
-// one captured graph.  Small boxes (fewer than three cells in a dimension)
-// are handled exactly: such a dimension is staged once and pairs take the
-// minimum image; elsewhere stage coordinates are shifted across the box
-// edges and the minimum image is the identity.
+// one captured graph.  A dimension of fewer than three cells is staged once
+// and pairs take the minimum image; elsewhere stage coordinates are shifted
+// across the box edges.
 #include <hip/hip_runtime.h>
 
 #include "batch.hpp"
@@ -65,98 +67,78 @@ __global__ __launch_bounds__(256) void kb_bin(BatchDev d, BatchRange rg) {
   float w[3];
   const int cell = batch_cell(p, d.px[i], d.py[i], d.pz[i], w);
   d.cell_of[i] = cell;
-  d.slot[i] = atomicAdd(&d.cnt[cell], 1);
-  if (d.charge[i] != 0.f) atomicAdd(&d.cntq[cell], 1);
+  // one atomic for both counts: atoms in the low half, charged in the high
+  const unsigned long long one = d.charge[i] != 0.f ? (1ull << 32) + 1ull : 1ull;
+  d.slot[i] = (int)(unsigned)atomicAdd(&d.cnt[cell], one);
 }
 
-// Exclusive offsets of the range's cells (atoms from rg.a0, charged atoms from
-// rg.q0); the counters are cleared for the next evaluation.  One workgroup.
-__global__ __launch_bounds__(1024) void kb_scan(BatchDev d, BatchRange rg) {
+// Exclusive offsets of one replica's cells, a workgroup each (atoms from a0,
+// charged atoms from q0: both are known per replica, so no scan crosses
+// replicas); the counters are cleared for the next evaluation.  One workgroup
+// over all cells took 240 us for the 49,000 cells of 256 replicas, this 5.
+__global__ __launch_bounds__(256) void kb_scan(BatchDev d, BatchRange rg) {
   __shared__ int sm[33];
-  const int nc = rg.c1 - rg.c0;
-  const int per = (nc + blockDim.x - 1) / blockDim.x;
-  const int s0 = rg.c0 + threadIdx.x * per, s1 = min(rg.c1, s0 + per);
-  int a = 0, q = 0;
-  for (int c = s0; c < s1; ++c) {
-    a += d.cnt[c];
-    q += d.cntq[c];
+  const RepInfo& p = d.rep[rg.r0 + blockIdx.x];
+  const int c0 = p.c0, nc = p.nc[0] * p.nc[1] * p.nc[2];
+  int ra = p.a0, rq = p.q0;
+  for (int base = 0; base < nc; base += blockDim.x) {
+    const int c = base + (int)threadIdx.x;
+    const unsigned long long v = c < nc ? d.cnt[c0 + c] : 0ull;
+    int ta, tq;
+    const int ea = block_excl_scan((int)(unsigned)v, ta, sm);
+    const int eq = block_excl_scan((int)(v >> 32), tq, sm);
+    if (c < nc) {
+      d.start[c0 + c] = ra + ea;
+      d.qstart[c0 + c] = rq + eq;
+      d.cnt[c0 + c] = 0ull;
+    }
+    ra += ta;
+    rq += tq;
   }
-  int ta, tq;
-  int ra = block_excl_scan(a, ta, sm) + rg.a0;
-  int rq = block_excl_scan(q, tq, sm) + rg.q0;
-  for (int c = s0; c < s1; ++c) {
-    d.start[c] = ra;
-    d.qstart[c] = rq;
-    ra += d.cnt[c];
-    rq += d.cntq[c];
-    d.cnt[c] = 0;
-    d.cntq[c] = 0;
-  }
+  // (the next replica's first cell: the same values its own workgroup writes)
   if (threadIdx.x == 0) {
-    d.start[rg.c1] = rg.a0 + ta;
-    d.qstart[rg.c1] = rg.q0 + tq;
+    d.start[c0 + nc] = ra;
+    d.qstart[c0 + nc] = rq;
   }
 }
 
+// Sort key of a caller atom inside its cell: charged first, then by index.
+constexpr int kNeutralKey = 1 << 30;
 __global__ __launch_bounds__(256) void kb_scatter(BatchDev d, BatchRange rg) {
   const int i = rg.a0 + blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= rg.a1) return;
-  d.tmp[d.start[d.cell_of[i]] + d.slot[i]] = i;
+  d.tmp[d.start[d.cell_of[i]] + d.slot[i]] = (d.charge[i] != 0.f ? 0 : kNeutralKey) + i;
 }
 
-// 32 lanes per cell: order the bucket (charged first, then caller index) by
-// ranking every atom's key within the cell, and write the sorted arrays in
-// parallel; a cell of more than 32 atoms is ordered by its first lane.
-__device__ __forceinline__ void batch_sorted_write(const BatchDev& d, int i, int k,
-                                                   int qslot) {
+// One thread per atom: its rank among the keys of its cell (the lanes of a
+// wave read the same few buckets), then its rows of the sorted arrays and,
+// for a charged atom, of the compact charged copy.
+__global__ __launch_bounds__(256) void kb_cellsort(BatchDev d, BatchRange rg) {
+  const int b = rg.a0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= rg.a1) return;
+  const int kv = d.tmp[b], i = kv & (kNeutralKey - 1);
+  const int c = d.cell_of[i];
+  const int s0 = d.start[c], s1 = d.start[c + 1];
+  int r = 0;
+  for (int q = s0; q < s1; ++q) r += d.tmp[q] < kv ? 1 : 0;
+  const int k = s0 + r;
   const RepInfo& p = d.rep[d.rep_of[i]];
   float w[3];
   batch_cell(p, d.px[i], d.py[i], d.pz[i], w);
-  const float qi = d.charge[i];
-  d.xs[k] = make_float4(w[0], w[1], w[2], qi);
   const int g = d.gid[i];
-  d.tg[k] = make_int2(d.type[i], g);
-  d.hj[k] = rbl_hj(g);
+  // .w: the byte offset of the type's entry in one row of the LJ table
+  d.xs[k] = make_float4(w[0], w[1], w[2], __int_as_float(d.type[i] << 4));
+  d.gid_s[k] = g;
   d.perm[k] = i;
-  if (qslot >= 0) d.qidx[qslot] = k;
-}
-
-__global__ __launch_bounds__(256) void kb_cellsort(BatchDev d, BatchRange rg) {
-  const int lane = threadIdx.x & 31;
-  const int c = rg.c0 + (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 5);
-  if (c >= rg.c1) return;  // whole 32-lane groups leave together
-  const int s0 = d.start[c], s1 = d.start[c + 1], len = s1 - s0;
-  auto key = [&](int i) { return (d.charge[i] != 0.f ? 0 : (1 << 30)) + i; };
-  if (len <= 32) {
-    const int i = lane < len ? d.tmp[s0 + lane] : 0;
-    const int kv = lane < len ? key(i) : 0x7fffffff;
-    int r = 0;
-    for (int q = 0; q < len; ++q) r += __shfl(kv, q, 32) < kv ? 1 : 0;
-    if (lane < len) {
-      const int q0 = d.qstart[c];
-      batch_sorted_write(d, i, s0 + r, kv < (1 << 30) ? q0 + r : -1);
-    }
-    return;
-  }
-  if (lane != 0) return;
-  for (int k = s0 + 1; k < s1; ++k) {
-    const int v = d.tmp[k], kv = key(v);
-    int j = k - 1;
-    while (j >= s0 && key(d.tmp[j]) > kv) {
-      d.tmp[j + 1] = d.tmp[j];
-      --j;
-    }
-    d.tmp[j + 1] = v;
-  }
-  int q = d.qstart[c];
-  for (int k = s0; k < s1; ++k) {
-    const int i = d.tmp[k];
-    batch_sorted_write(d, i, k, d.charge[i] != 0.f ? q++ : -1);
+  if (kv < kNeutralKey) {
+    const int q = d.qstart[c] + r;
+    d.xqc[q] = make_float4(w[0], w[1], w[2], d.charge[i]);
+    d.qi[q] = make_int4(g, d.qpos[i], c, i);
   }
 }
 
-// Slot tables of one brick's neighbourhood (the brick widened by one cell,
-// a dimension that would wrap onto itself taken whole).
+// Slot tables of one brick's neighbourhood (the brick widened by one cell;
+// a dimension of fewer than three cells taken whole).
 struct BrickNb {
   int o[3], w[3];      // brick cells [o, o + w)
   int rs[3], rn[3];    // neighbourhood start (may be -1) and count
@@ -165,14 +147,19 @@ struct BrickNb {
   int mi;
 };
 
-__device__ __forceinline__ BrickNb batch_brick(const RepInfo& p, int b, int bw) {
+// With three cells or more, every owner's window of three cells holds each
+// cell once, shifted by +-L across the edges.  For a pair two cells apart of
+// a three-cell dimension the shifted distance may exceed L/2, but then its
+// other image is at least one cell away, beyond the cutoff, as is this one:
+// every pair inside the cutoff is met exactly once, at its minimum image.
+__device__ __forceinline__ BrickNb batch_brick(const RepInfo& p, int b) {
   BrickNb h;
   const int bc[3] = {b % p.nb[0], (b / p.nb[0]) % p.nb[1], b / (p.nb[0] * p.nb[1])};
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    h.o[d] = bc[d] * bw;
-    h.w[d] = min(bw, p.nc[d] - h.o[d]);
-    h.full[d] = h.w[d] + 2 >= p.nc[d];
+    h.o[d] = bc[d] * p.bw;
+    h.w[d] = min(p.bw, p.nc[d] - h.o[d]);
+    h.full[d] = p.nc[d] < 3;
     h.rs[d] = h.full[d] ? 0 : h.o[d] - 1;
     h.rn[d] = h.full[d] ? p.nc[d] : h.w[d] + 2;
   }
@@ -181,103 +168,11 @@ __device__ __forceinline__ BrickNb batch_brick(const RepInfo& p, int b, int bw) 
   return h;
 }
 
-// LJ interaction of a pair that involves a neutral atom (interact_a's
-// scalars and energy convention).
-template <bool RBL, bool EFLAG, bool MI, bool SPECIAL>
-__device__ __forceinline__ void batch_lj(const PairConst<float>& pc, const Box<float>& b,
-                                         const float* s_lj, int ti, const float4& xi,
-                                         unsigned long long hi, const float4& xj, int tj,
-                                         int gj, float& fx, float& fy, float& fz,
-                                         Acc<float>& a, const SpecRow& sr) {
-  float dx, dy, dz;
-  const float d2 = pair_d2<float, MI>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
-  if (!(d2 < pc.rclj2) || !(d2 < pc.rc2)) return;
-  const int tt = 4 * (ti * pc.ntypes + tj);
-  const float m24 = s_lj[tt], sig2 = s_lj[tt + 1], eps = s_lj[tt + 2];
-  const float inv = pair_rcp(d2);
-  const float s2 = sig2 * inv;
-  const float s6 = s2 * s2 * s2;
-  // CVFF: the owner's special-bond weight scales the LJ term
-  const float ws = SPECIAL ? special_w<float>(sr, gj, pc) : 1.f;
-  const float flj = ws * (m24 * (2.f * s6 - 1.f) * s6 * inv);
-  // the neighbour's hash enters only for shell pairs
-  const float w = pair_weight<float, RBL>(pc, d2, hi, [&] { return rbl_hj(gj); });
-  const float f = w * flj;
-  fx += f * dx;
-  fy += f * dy;
-  fz += f * dz;
-  if (EFLAG) {
-    a.e_lj += (double)(ws * (2.f * eps * (s6 - 1.f) * s6));
-    add_virial<float, EFLAG>(a, dx, dy, dz, flj);
-  }
-}
-
-// batch_lj over the staged candidates [l0, l1) of one stencil row without
-// energies or special bonds, with no branch per candidate: the owner itself
-// and (for a charged owner) charged candidates are masked, the cutoffs and
-// the RBL weight are selects, and only a shell candidate (rare at an LJ cutoff
-// at or below r_core) forms its selection hash.  Per pair the same terms in
-// the same order as batch_lj.
-template <bool RBL, bool MI>
-__device__ __forceinline__ void batch_lj_row(const PairConst<float>& pc, const Box<float>& b,
-                                             const float* s_lj, int ti, const float4& xi,
-                                             unsigned long long hi, bool qi, int li,
-                                             const float4* sx, const int2* stg, int l0,
-                                             int l1, float& fx, float& fy, float& fz) {
-  const int row = 4 * ti * pc.ntypes;
-  for (int l = l0; l < l1; ++l) {
-    const float4 xj = sx[l];
-    const int2 tgj = stg[l];
-    float dx, dy, dz;
-    const float d2 = pair_d2<float, MI>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
-    const bool in = (l != li) & !(qi & (xj.w != 0.f)) & (d2 < pc.rclj2) & (d2 < pc.rc2);
-    float w = 1.f;
-    if (RBL) {
-      const bool core = d2 < pc.t_core;
-      const float wc = ((d2 < pc.rs2) & (d2 > pc.eps_min)) ? 1.f : 0.f;
-      float wsh = 0.f;
-      if (in & !core & (d2 < pc.t_shell) & (d2 > pc.rs2))
-        wsh = rbl_keep(pc.ifreq, pc.fmask, pc.c32, pc.epoch, hi, rbl_hj(tgj.y)) ? pc.freq
-                                                                               : 0.f;
-      w = core ? wc : wsh;
-    }
-    const int tt = row + 4 * tgj.x;
-    const float m24 = s_lj[tt], sig2 = s_lj[tt + 1];
-    const float inv = pair_rcp(d2);
-    const float s2 = sig2 * inv;
-    const float s6 = s2 * s2 * s2;
-    const float flj = m24 * (2.f * s6 - 1.f) * s6 * inv;
-    const float f = (in & (w != 0.f)) ? w * flj : 0.f;
-    fx += f * dx;
-    fy += f * dy;
-    fz += f * dz;
-  }
-}
-
-// LJ + erfc Coulomb of a charged pair (interact_b's terms: eval_b, with the
-// owner's special-bond weight under CVFF; minimum image).
-template <bool RBL, bool EFLAG, bool MI, bool SPECIAL>
-__device__ __forceinline__ void batch_charged(const PairConst<float>& pc,
-                                              const Box<float>& b, const float* s_lj,
-                                              int ti, const float4& xi,
-                                              unsigned long long hi, const float4& xj,
-                                              int tj, int gj, Acc<float>& a,
-                                              const SpecRow& sr) {
-  float dx, dy, dz;
-  const float d2 = pair_d2<float, MI>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
-  if (!(d2 < pc.rc2)) return;
-  const float w = pair_weight<float, RBL>(pc, d2, hi, [&] { return rbl_hj(gj); });
-  const float ws = SPECIAL ? special_w<float>(sr, gj, pc) : 1.f;
-  eval_b<float, EFLAG, SPECIAL>(pc, s_lj, ti, tj, xi.w * xj.w, dx, dy, dz, d2, w, a, ws);
-}
-
-// The CVFF special-bond row of sorted atom s (counts and partner ids in
-// caller order).
-template <bool SPECIAL>
-__device__ __forceinline__ SpecRow batch_spec_row(const BatchDev& d, int ms, int s) {
+// The CVFF special-bond row of caller atom i.
+template <bool GEN>
+__device__ __forceinline__ SpecRow batch_spec_row(const BatchDev& d, int ms, int i) {
   SpecRow r;
-  if (SPECIAL) {
-    const int i = d.perm[s];
+  if (GEN && ms > 0) {
     const int4 c = d.spn[i];
     r.n12 = c.x;
     r.n13 = c.y;
@@ -287,24 +182,585 @@ __device__ __forceinline__ SpecRow batch_spec_row(const BatchDev& d, int ms, int
   return r;
 }
 
-template <bool RBL, bool EFLAG, bool SPECIAL>
-__global__ __launch_bounds__(256) void kb_pair(BatchDev d, PairConst<float> pc_arg,
-                                               BatchRange rg, int bw, int qlanes) {
-  __shared__ float4 sx[kBatchStageCap];
-  __shared__ int2 stg[kBatchStageCap];
-  // slot tables of the staged neighbourhood: up to kBatchMaxSlots cells for
-  // the LJ pass, up to kBatchQSlots for the charged pass
-  __shared__ int soff[kBatchQSlots + 1];
-  __shared__ int sfirst[kBatchQSlots];
-  __shared__ int sedge[kBatchQSlots];
-  __shared__ int sscan[33];
+// LDS of kb_eval's workgroups: one buffer for the three roles.
+//   LJ: the stage (position and LJ-row offset), 64 entries of padding that
+//       the unrolled tests may read past a row, the sentinel, then the
+//       per-lane lists of accepted stage positions [kLjList][block] and, with
+//       GEN, the staged global ids;
+//   Coulomb: per-lane lists of accepted charged atoms [kQList][block];
+//   k-space: the atom tile, per-k coefficients and rho, and partial sums.
+constexpr int kEvalBlock = 256;
+constexpr int kLjList = 44;
+constexpr int kStagePad = 64;
+constexpr int kQList = 8;
+constexpr int kKsTile = 256;
+constexpr size_t kStageBytes = (size_t)(kBatchStageCap + kStagePad + 1) * sizeof(float4);
+constexpr size_t kListBytes = (size_t)kLjList * kEvalBlock * sizeof(unsigned short);
+constexpr size_t kGidBytes = (size_t)kBatchStageCap * sizeof(int);
+constexpr size_t kKsBytes = kKsTile * sizeof(float4) + 2 * (size_t)kBatchMaxK * sizeof(float4) +
+                            (size_t)kBatchMaxK * sizeof(double2) +
+                            2 * (size_t)kEvalBlock * sizeof(double);
+static_assert(kKsBytes <= kStageBytes + kListBytes, "k-space LDS");
+
+// LJ pairs of one owner lane over the part [w0, w1) of the neighbourhood that
+// the stage holds.  Two phases, so that the pair terms run on lanes that hold
+// a pair: the candidates of each stencil row are tested 8 at a time without
+// branches (d^2 - r^2's sign shifted into a mask: eight VALU instructions a
+// test), the accepted stage positions go to the lane's list, and the list is
+// evaluated at the end of the window (or when it would overflow).  The lpo
+// lanes of an owner each take a contiguous part of every row.
+// Bound by VALU issue.  256 electrolytes (777,841 atoms): 3352 us with every
+// candidate's terms evaluated in one pass at the default shape.
+template <bool RBL, bool EFLAG, bool GEN, bool MI>
+__device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<float>& b,
+                                        const float* s_lj, const float4* sx,
+                                        const int* sgid, const int* soff,
+                                        unsigned short* list, int T, const int lo3[3],
+                                        const int hi3[3], int rn0, int rn1, int w0, int w1,
+                                        bool live, const float4& xi, int li, int sub,
+                                        int lsh, bool shell, unsigned long long hi,
+                                        const SpecRow& sr, float& fx, float& fy, float& fz,
+                                        Acc<float>& a) {
+  const float r2 = (EFLAG || GEN) ? fminf(pc.rclj2, pc.rc2) : pc.a_hi;
+  const char* lj_row =
+      reinterpret_cast<const char*>(s_lj) + (__float_as_int(xi.w) * pc.ntypes);
+  constexpr int kSent = kBatchStageCap + kStagePad;
+  auto d2_of = [&](const float4& xj, float& dx, float& dy, float& dz) {
+    return MI ? pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz)
+              : pair_d2<float, false>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
+  };
+  int cnt = 0;
+  auto eval = [&](int l) {
+    const float4 xj = sx[l];
+    float dx, dy, dz;
+    const float d2 = d2_of(xj, dx, dy, dz);
+    const float2 lj = *reinterpret_cast<const float2*>(lj_row + __float_as_int(xj.w));
+    const float inv = pair_rcp(d2);
+    const float s2 = lj.y * inv;
+    const float s6 = s2 * s2 * s2;
+    float flj = lj.x * (2.f * s6 - 1.f) * s6 * inv;
+    if (!EFLAG && !GEN) {
+      // the list's test was d^2 < a_hi; the sentinel and coincident atoms go
+      const float f = ((d2 < r2) & (d2 > pc.a_lo)) ? flj : 0.f;
+      fx = fma_r(f, dx, fx);
+      fy = fma_r(f, dy, fy);
+      fz = fma_r(f, dz, fz);
+      return;
+    }
+    const bool in = d2 < r2;
+    float ws = 1.f;
+    if (GEN && in && sr.n14 > 0) ws = special_w<float>(sr, sgid[l], pc);
+    flj *= ws;
+    float w = 1.f;
+    if (RBL) {
+      const bool core = d2 < pc.t_core;
+      w = (core && d2 < pc.rs2 && d2 > pc.eps_min) ? 1.f : 0.f;
+      if (GEN && shell && in && !core && d2 < pc.t_shell && d2 > pc.rs2 &&
+          rbl_keep(pc.ifreq, pc.fmask, pc.c32, pc.epoch, hi, rbl_hj(sgid[l])))
+        w = pc.freq;
+    }
+    const float f = (in && w != 0.f) ? w * flj : 0.f;
+    fx = fma_r(f, dx, fx);
+    fy = fma_r(f, dy, fy);
+    fz = fma_r(f, dz, fz);
+    if (EFLAG) {
+      const float eps = *reinterpret_cast<const float*>(lj_row + __float_as_int(xj.w) + 8);
+      a.e_lj += in ? (double)(ws * (2.f * eps * (s6 - 1.f) * s6)) : 0.0;
+      add_virial<float, EFLAG>(a, dx, dy, dz, in ? flj : 0.f);
+    }
+  };
+  auto drain = [&]() {
+    for (int k = 0; __any(k < cnt); k += 2) {
+      const int l0 = k < cnt ? list[k * T] : kSent;
+      const int l1 = k + 1 < cnt ? list[(k + 1) * T] : kSent;
+      eval(l0);
+      eval(l1);
+    }
+    cnt = 0;
+  };
+  for (int kz = lo3[2]; kz <= hi3[2]; ++kz)
+    for (int ky = lo3[1]; ky <= hi3[1]; ++ky) {
+      const int srow = (kz * rn1 + ky) * rn0;
+      const int l0 = max(soff[srow + lo3[0]], w0) - w0;
+      const int l1 = min(soff[srow + hi3[0] + 1], w1) - w0;
+      const int len = max(l1 - l0, 0), part = (len + (1 << lsh) - 1) >> lsh;
+      const int b0 = l0 + sub * part;
+      const int n = live ? min(part, len - sub * part) : 0;
+      for (int k0 = 0; __any(k0 < n); k0 += 32) {
+        unsigned m = 0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          if (!__any(k0 + 8 * g < n)) {
+            m <<= 8;
+            continue;
+          }
+          // a lane whose row is over reads its row's start (masked below)
+          const float4* xp = sx + (k0 + 8 * g < n ? b0 + k0 + 8 * g : 0);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            float dx, dy, dz;
+            const float s = d2_of(xp[u], dx, dy, dz) - r2;
+            m = __builtin_amdgcn_alignbit(m, __float_as_uint(s), 31);
+          }
+        }
+        // candidates past the row's part and the owner itself
+        const int rem = min(max(n - k0, 0), 32);
+        m &= (unsigned)(0xffffffff00000000ull >> rem);
+        const int so = li - b0 - k0;
+        if ((unsigned)so < 32u) m &= ~(0x80000000u >> so);
+        if (__any(cnt + __popc(m) > kLjList)) drain();
+        while (m) {
+          const int u = __clz((int)m);
+          m &= ~(0x80000000u >> u);
+          list[cnt * T] = (unsigned short)(b0 + k0 + u);
+          ++cnt;
+        }
+      }
+    }
+  drain();
+}
+
+// LJ pairs of one brick: every atom of the brick against its 27 cells.
+template <bool RBL, bool EFLAG, bool GEN>
+__device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<float>& pc,
+                                         const RepInfo& p, int brick, const float* s_lj,
+                                         char* buf, int* soff, int* sfirst, int* sedge,
+                                         float fs[3], Acc<float>& a) {
+  float4* sx = reinterpret_cast<float4*>(buf);
+  unsigned short* list = reinterpret_cast<unsigned short*>(buf + kStageBytes) + threadIdx.x;
+  int* sgid = reinterpret_cast<int*>(buf + kStageBytes + kListBytes);
+  const Box<float> b = p.box;
+  const BrickNb h = batch_brick(p, brick);
+  if (threadIdx.x < 64) {
+    int cnt = 0;
+    const int s = threadIdx.x;
+    if (s < h.nslots) {
+      const int k[3] = {s % h.rn[0], (s / h.rn[0]) % h.rn[1], s / (h.rn[0] * h.rn[1])};
+      int cw[3], e = 0;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int u = h.rs[q] + k[q];
+        cw[q] = wrapi(u, p.nc[q]);
+        e |= (u < 0 ? 0 : (u >= p.nc[q] ? 2 : 1)) << (2 * q);
+      }
+      const int cell = p.c0 + (cw[2] * p.nc[1] + cw[1]) * p.nc[0] + cw[0];
+      sfirst[s] = d.start[cell];
+      cnt = d.start[cell + 1] - d.start[cell];
+      sedge[s] = e;
+    }
+    const int inc = wave_incl_scan(cnt);
+    if (s < h.nslots) soff[s] = inc - cnt;
+    if (s == 63) soff[h.nslots] = inc;
+  }
+  if (threadIdx.x == 0)
+    sx[kBatchStageCap + kStagePad] = make_float4(1e18f, 1e18f, 1e18f, 0.f);
+  __syncthreads();
+  const int total = soff[h.nslots];
+  // the brick's own cells u = 0..own_n-1 (x-fastest within the brick) and
+  // their atoms' running offsets (at most 8 cells)
+  const int own_n = h.w[0] * h.w[1] * h.w[2];
+  int own_end[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    int len = 0;
+    if (u < own_n) {
+      const int k[3] = {u % h.w[0], (u / h.w[0]) % h.w[1], u / (h.w[0] * h.w[1])};
+      const int s = ((h.o[2] - h.rs[2] + k[2]) * h.rn[1] + (h.o[1] - h.rs[1] + k[1])) *
+                        h.rn[0] +
+                    (h.o[0] - h.rs[0] + k[0]);
+      len = soff[s + 1] - soff[s];
+    }
+    own_end[u] = (u > 0 ? own_end[u - 1] : 0) + len;
+  }
+  const int nown = own_end[7];
+  // lpo adjacent lanes per owner (up to 8, as many as the block leaves idle)
+  int lsh = 0;
+  while (lsh < 3 && (nown << (lsh + 1)) <= (int)blockDim.x) ++lsh;
+  const int lpo = 1 << lsh;
+  const bool shell = RBL && pc.rclj2 > pc.rs2;
+  // a neighbourhood beyond the stage goes in windows of kBatchStageCap atoms
+  // (staged again for every pass over the owners)
+  const bool one = total <= kBatchStageCap;
+  for (int t0 = 0; t0 < (nown << lsh); t0 += blockDim.x) {
+    const int tt = t0 + (int)threadIdx.x;
+    const bool live = tt < (nown << lsh);
+    const int t = live ? tt >> lsh : 0, sub = tt & (lpo - 1);
+    int u = 0, ub = 0;
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+      if (own_end[q] <= t) {
+        u = q + 1;
+        ub = own_end[q];
+      }
+    const int j0 = t - ub;
+    const int k[3] = {u % h.w[0], (u / h.w[0]) % h.w[1], u / (h.w[0] * h.w[1])};
+    int ko[3], lo3[3], hi3[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      ko[q] = h.o[q] - h.rs[q] + k[q];
+      lo3[q] = h.full[q] ? 0 : ko[q] - 1;
+      hi3[q] = h.full[q] ? h.rn[q] - 1 : ko[q] + 1;
+    }
+    const int s_own = (ko[2] * h.rn[1] + ko[1]) * h.rn[0] + ko[0];
+    const int i = sfirst[s_own] + j0;
+    const int li = soff[s_own] + j0;
+    const float4 xi = d.xs[i];
+    const int ci = d.perm[i];
+    const unsigned long long hi = (RBL && GEN) ? rbl_hi(d.gid_s[i]) : 0ull;
+    const SpecRow sr = batch_spec_row<GEN>(d, pc.ms, ci);
+    float fx = 0.f, fy = 0.f, fz = 0.f;
+    for (int w0 = 0; w0 < total; w0 += kBatchStageCap) {
+      const int w1 = min(total, w0 + kBatchStageCap);
+      if (!one || t0 == 0) {
+        if (!one) __syncthreads();  // the previous window's readers are done
+        const int lane = threadIdx.x & 15;
+        for (int s = threadIdx.x >> 4; s < h.nslots; s += blockDim.x >> 4) {
+          const int o = soff[s], f = sfirst[s], e = sedge[s];
+          float sh[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const int c = (e >> (2 * q)) & 3;
+            sh[q] = c == 0 ? -b.L[q] : (c == 2 ? b.L[q] : 0.f);
+          }
+          const int le = min(soff[s + 1], w1);
+          for (int l = max(o, w0) + lane; l < le; l += 16) {
+            float4 v = d.xs[f + (l - o)];
+            v.x += sh[0];
+            v.y += sh[1];
+            v.z += sh[2];
+            sx[l - w0] = v;
+            if (GEN) sgid[l - w0] = d.gid_s[f + (l - o)];
+          }
+        }
+        __syncthreads();
+      }
+      if (h.mi)
+        lj_lane<RBL, EFLAG, GEN, true>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3,
+                                       hi3, h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, sub,
+                                       lsh, shell, hi, sr, fx, fy, fz, a);
+      else
+        lj_lane<RBL, EFLAG, GEN, false>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3,
+                                        hi3, h.rn[0], h.rn[1], w0, w1, live, xi, li - w0,
+                                        sub, lsh, shell, hi, sr, fx, fy, fz, a);
+    }
+    fs[0] += fx;
+    fs[1] += fy;
+    fs[2] += fz;
+    for (int o = lpo / 2; o > 0; o >>= 1) {
+      fx += __shfl_xor(fx, o, 64);
+      fy += __shfl_xor(fy, o, 64);
+      fz += __shfl_xor(fz, o, 64);
+    }
+    if (live && sub == 0) d.fs[ci] = make_float4(fx, fy, fz, 0.f);
+  }
+}
+
+// Coulomb pairs of the charged atoms [c0, c0 + block / qlanes) of a replica,
+// qlanes lanes per atom, over the charged atoms of the cells within ext_c:
+// the cells of one stencil row are consecutive in the compact charged order
+// (two runs where the row wraps), read from cache.  Tested first, then the
+// accepted ones (per-lane list) take the erfc terms and the RBL hash.
+template <bool RBL, bool EFLAG, bool GEN>
+__device__ __forceinline__ void coul_run(const BatchDev& d, const PairConst<float>& pc,
+                                         const RepInfo& p, int c0, int qlanes, char* buf,
+                                         float fs[3], Acc<float>& a) {
+  int* list = reinterpret_cast<int*>(buf) + threadIdx.x;
+  const int T = (int)blockDim.x;
+  const Box<float> b = p.box;
+  const int grp = threadIdx.x / qlanes, gl = threadIdx.x % qlanes;
+  const int c = c0 + grp;
+  const bool live = c < p.q0 + p.nq;
+  const int cc = live ? c : p.q0 + p.nq - 1;
+  const float4 xi = d.xqc[cc];
+  const int4 qi = d.qi[cc];
+  const unsigned long long hi = RBL ? rbl_hi(qi.x) : 0ull;
+  const SpecRow sr = batch_spec_row<GEN>(d, pc.ms, qi.w);
+  const int cl = qi.z - p.c0;
+  const int cx = cl % p.nc[0], cy = (cl / p.nc[0]) % p.nc[1], cz = cl / (p.nc[0] * p.nc[1]);
+  const Span sy = make_span(cy, p.ext_c[1], p.nc[1]), sz = make_span(cz, p.ext_c[2], p.nc[2]);
+  // x cells of a row: [x0, x1] and, where the window wraps, [y0, y1]
+  const Span sxs = make_span(cx, p.ext_c[0], p.nc[0]);
+  const int x0 = max(sxs.start, 0), x1 = min(sxs.start + sxs.count, p.nc[0]) - 1;
+  int y0 = 0, y1 = -1;
+  if (sxs.start < 0) {
+    y0 = sxs.start + p.nc[0];
+    y1 = p.nc[0] - 1;
+  } else if (sxs.start + sxs.count > p.nc[0]) {
+    y1 = sxs.start + sxs.count - 1 - p.nc[0];
+  }
+  const int nrow = sy.count * sz.count;
+  // lanes over candidates within a row (cw) and over rows, by the mean run
+  int cw = 1;
+  const float run = (float)p.nq * (float)sxs.count / (float)(p.nc[0] * p.nc[1] * p.nc[2]);
+  while (cw < qlanes && run > 8.f * (float)cw) cw *= 2;
+  const int rw = qlanes / cw, rl = gl / cw, ql = gl % cw;
+  float fx = 0.f, fy = 0.f, fz = 0.f;
+  int cnt = 0;
+  auto drain = [&]() {
+    for (int k = 0; __any(k < cnt); ++k) {
+      if (k < cnt) {
+        const int j = list[k * T];
+        const float4 xj = d.xqc[j];
+        float dx, dy, dz;
+        const float d2 =
+            pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
+        float w = 1.f, ws = 1.f;
+        if (RBL || GEN) {
+          const int gj = d.qi[j].x;
+          w = pair_weight<float, RBL>(pc, d2, hi, [&] { return rbl_hj(gj); });
+          if (GEN && sr.n14 > 0) ws = special_w<float>(sr, gj, pc);
+        }
+        const float qq = xi.w * xj.w;
+        const float rinv = pair_rsqrt(d2), inv = pair_rcp(d2);
+        float fc, ec;
+        coul<float>(pc, d2, rinv, inv, qq, fc, ec);
+        // a special pair removes (1 - ws) of the full Coulomb force from
+        // every kept pair, without the RBL multiplier
+        const float corr = GEN ? (1.f - ws) * (-pc.qqr2e * qq * rinv * rinv * rinv) : 0.f;
+        const float f = w * fc - (w != 0.f ? corr : 0.f);
+        fx = fma_r(f, dx, fx);
+        fy = fma_r(f, dy, fy);
+        fz = fma_r(f, dz, fz);
+        if (EFLAG) {
+          a.e_c += (double)(ec - (GEN ? (1.f - ws) * (0.5f * pc.qqr2e * qq * rinv) : 0.f));
+          add_virial<float, EFLAG>(a, dx, dy, dz, fc - corr);
+        }
+      }
+    }
+    cnt = 0;
+  };
+  for (int r = rl; __any(r < nrow); r += rw) {
+    const int row = p.c0 + (sz.at(min(r, nrow - 1) / sy.count) * p.nc[1] +
+                            sy.at(min(r, nrow - 1) % sy.count)) * p.nc[0];
+    for (int seg = 0; seg < 2; ++seg) {
+      const int e0 = seg ? y0 : x0, e1 = seg ? y1 : x1;
+      if (!__any(e1 >= e0)) break;
+      const bool on = live && r < nrow && e1 >= e0;
+      const int j0 = on ? d.qstart[row + e0] : 0;
+      const int j1 = on ? d.qstart[row + e1 + 1] : 0;
+      for (int j = j0 + ql; __any(j < j1); j += 4 * cw) {
+        float4 xj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xj[u] = d.xqc[j + u * cw < j1 ? j + u * cw : cc];
+        if (__any(cnt + 4 > kQList)) drain();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float dx, dy, dz;
+          const float d2 = pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj[u].x, xj[u].y, xj[u].z,
+                                               dx, dy, dz);
+          if (j + u * cw < j1 && j + u * cw != c && d2 < pc.rc2) {
+            list[cnt * T] = j + u * cw;
+            ++cnt;
+          }
+        }
+      }
+    }
+  }
+  drain();
+  fs[0] += fx;
+  fs[1] += fy;
+  fs[2] += fz;
+  for (int o = qlanes / 2; o > 0; o >>= 1) {
+    fx += __shfl_xor(fx, o, 64);
+    fy += __shfl_xor(fy, o, 64);
+    fz += __shfl_xor(fz, o, 64);
+  }
+  if (live && gl == 0) d.fq[qi.y] = make_float4(fx, fy, fz, 0.f);
+}
+
+// k-space of one replica: S(k) (one k per thread; with K at most half the
+// block, the atoms of a tile split over block / K groups; FP32 within a tile
+// and FP64 across), the energy and virial (FP64), then the force on every
+// charged atom (several lanes per atom, each a part of the k's, when the
+// replica has few).  RBE and EWALD: the k's of m, weights kw or
+// exp(-k^2 / 4 alpha), virial E_k (delta_ab - 2 k_a k_b (1/(4 alpha) + 1/k^2)).
+// RBSOG: the P sampled k's (weight kw) and the nd direct vectors (per-replica
+// weights kwd), every k in the RBE form E_k = qqr2e (2 pi / V) w |rho|^2 / k^2;
+// virial W_aa += E_k and W_ab += tau_k |rho_s|^2 k_s,a k_s,b with s the
+// virial-chain source of a sampled k (tau = ktau, over |k_s|^4) or the direct
+// vector itself (tau = kvd) (kspace_calculator_op.hip.cu:1133-1222, :1308-1352).
+template <bool EFLAG>
+__device__ __forceinline__ void kspace_replica(const BatchDev& d, const PairConst<float>& pc,
+                                               const RepInfo& p, int r, char* buf,
+                                               double* smem) {
+  float4* sa = reinterpret_cast<float4*>(buf);
+  float4* kf0 = sa + kKsTile;
+  float4* kf1 = kf0 + kBatchMaxK;
+  double2* srho = reinterpret_cast<double2*>(kf1 + kBatchMaxK);
+  double* spart = reinterpret_cast<double*>(srho + kBatchMaxK);  // [2 * block]
+  const double two_pi = 6.283185307179586476925;
+  const int P = d.P, T = (int)blockDim.x;
+  const bool sog = d.kmode == 2;
+  const int K = P + (sog ? d.nd : 0);
+  const int* m = d.m + (size_t)r * d.mstride;
+  // integer vector of k: sampled (replica's m) or direct (shared table)
+  auto mvec = [&](int k) { return k < P ? m + 3 * k : d.dm + 3 * (k - P); };
+  double kv[kBatchKAcc] = {0, 0, 0, 0, 0, 0, 0};
+  int kw = T;  // threads over k; T / kw groups over the atoms
+  while (K <= kw / 2 && kw > 32) kw /= 2;
+  const int ng = T / kw, grp = (int)threadIdx.x / kw, kt = (int)threadIdx.x % kw;
+  for (int k0 = 0; k0 < K; k0 += kw) {
+    const int k = k0 + kt;
+    const int* mk = mvec(k < K ? k : 0);
+    const float mx = (float)mk[0], my = (float)mk[1], mz = (float)mk[2];
+    double re = 0.0, im = 0.0;
+    for (int t0 = 0; t0 < p.nq; t0 += kKsTile) {
+      const int tn = min(kKsTile, p.nq - t0);
+      __syncthreads();
+      for (int j = threadIdx.x; j < tn; j += T) {
+        const float4 x = d.xqc[p.q0 + t0 + j];
+        sa[j] = make_float4((x.x - p.box.lo[0]) * p.box.invL[0],
+                            (x.y - p.box.lo[1]) * p.box.invL[1],
+                            (x.z - p.box.lo[2]) * p.box.invL[2], x.w);
+      }
+      __syncthreads();
+      float fr = 0.f, fi = 0.f;
+#pragma unroll 4
+      for (int j = grp; j < tn; j += ng) {
+        const float4 a = sa[j];
+        float sn, cs;
+        sincos_rev(fma_r(mx, a.x, fma_r(my, a.y, mz * a.z)), sn, cs);
+        fr = fma_r(a.w, cs, fr);
+        fi = fma_r(a.w, sn, fi);
+      }
+      re += (double)fr;
+      im += (double)fi;
+    }
+    if (ng > 1) {  // K <= kw: a single pass
+      spart[2 * threadIdx.x] = re;
+      spart[2 * threadIdx.x + 1] = im;
+      __syncthreads();
+      re = im = 0.0;
+      for (int g = 0; g < ng; ++g) {
+        re += spart[2 * (g * kw + kt)];
+        im += spart[2 * (g * kw + kt) + 1];
+      }
+    }
+    if (k < K && grp == 0) {
+      const double kx = two_pi * mk[0] / (double)p.box.L[0];
+      const double ky = two_pi * mk[1] / (double)p.box.L[1];
+      const double kz = two_pi * mk[2] / (double)p.box.L[2];
+      const double k2 = kx * kx + ky * ky + kz * kz;
+      const double wk = d.kmode == 1 ? exp(-k2 / (4.0 * (double)pc.alpha))
+                        : (k < P ? p.kw : d.kwd[(size_t)r * d.nd + (k - P)]);
+      const double A = wk * (-4.0 * 3.141592653589793238463 * (double)pc.qqr2e) /
+                       (p.volume * k2);
+      kf0[k] = make_float4((float)mk[0], (float)mk[1], (float)mk[2], (float)(A * re));
+      kf1[k] = make_float4((float)kx, (float)ky, (float)kz, (float)(A * im));
+      srho[k] = make_double2(re, im);
+      if (EFLAG) {
+        const double base =
+            (double)pc.qqr2e * two_pi / p.volume * wk * (re * re + im * im) / k2;
+        kv[0] += base;
+        if (sog) {
+          kv[1] += base;
+          kv[2] += base;
+          kv[3] += base;
+        } else {
+          const double cc = 2.0 * (1.0 / (4.0 * (double)pc.alpha) + 1.0 / k2);
+          kv[1] += base * (1.0 - cc * kx * kx);
+          kv[2] += base * (1.0 - cc * ky * ky);
+          kv[3] += base * (1.0 - cc * kz * kz);
+          kv[4] += base * (-cc * kx * ky);
+          kv[5] += base * (-cc * kx * kz);
+          kv[6] += base * (-cc * ky * kz);
+        }
+      }
+    }
+  }
+  __syncthreads();  // srho of every k is written
+  if (EFLAG) {
+    if (sog)
+      for (int k = threadIdx.x; k < K; k += T) {
+        const int src = k < P ? m[3 * P + k] : k;
+        const int* ms = mvec(src);
+        const double kx = two_pi * ms[0] / (double)p.box.L[0];
+        const double ky = two_pi * ms[1] / (double)p.box.L[1];
+        const double kz = two_pi * ms[2] / (double)p.box.L[2];
+        const double2 rs = srho[src];
+        double t = (k < P ? p.ktau : d.kvd[(size_t)r * d.nd + (k - P)]) *
+                   (rs.x * rs.x + rs.y * rs.y);
+        if (k < P) {
+          const double k2 = kx * kx + ky * ky + kz * kz;
+          t /= k2 * k2;
+        }
+        kv[1] += t * kx * kx;
+        kv[2] += t * ky * ky;
+        kv[3] += t * kz * kz;
+        kv[4] += t * kx * ky;
+        kv[5] += t * kx * kz;
+        kv[6] += t * ky * kz;
+      }
+    block_sum<kBatchKAcc>(kv, smem);
+    if (threadIdx.x == 0)
+      for (int q = 0; q < kBatchKAcc; ++q) d.kacc[(size_t)r * kBatchKAcc + q] = kv[q];
+  }
+  // nl lanes per atom, lane s the k's s, s + nl, ...
+  int nl = 1;
+  while (nl < 16 && 2 * nl * p.nq <= T) nl *= 2;
+  const int s = (int)threadIdx.x % nl, per = T / nl;
+  for (int c0 = 0; c0 < p.nq; c0 += per) {
+    const int c = c0 + (int)threadIdx.x / nl;
+    const bool live = c < p.nq;
+    const float4 x = d.xqc[p.q0 + (live ? c : 0)];
+    const float sx = (x.x - p.box.lo[0]) * p.box.invL[0];
+    const float sy = (x.y - p.box.lo[1]) * p.box.invL[1];
+    const float sz = (x.z - p.box.lo[2]) * p.box.invL[2];
+    float fx = 0.f, fy = 0.f, fz = 0.f;
+#pragma unroll 4
+    for (int k = s; k < K; k += nl) {
+      const float4 a = kf0[k];
+      const float4 e = kf1[k];
+      float sn, cs;
+      sincos_rev(fma_r(a.x, sx, fma_r(a.y, sy, a.z * sz)), sn, cs);
+      const float gg = fma_r(cs, e.w, -sn * a.w);
+      fx = fma_r(gg, e.x, fx);
+      fy = fma_r(gg, e.y, fy);
+      fz = fma_r(gg, e.z, fz);
+    }
+    for (int o = nl / 2; o > 0; o >>= 1) {
+      fx += __shfl_xor(fx, o, 64);
+      fy += __shfl_xor(fy, o, 64);
+      fz += __shfl_xor(fz, o, 64);
+    }
+    if (live && s == 0)
+      d.fk[d.qi[p.q0 + c].y] = make_float4(x.w * fx, x.w * fy, x.w * fz, 0.f);
+  }
+}
+
+// Blocks [0, nk): the k-space of one replica each (first, since a large
+// replica's takes longest); [nk, nk + npg): LJ, persistent over the bricks of
+// the range; the rest: Coulomb, one run of charged atoms each.  Nothing
+// depends on another block's result, so the k-space latency and the short
+// Coulomb runs fill the machine beside the LJ bricks.
+// GEN: CVFF special bonds, or an LJ cutoff beyond r_core (RBL shell pairs in
+// the LJ pass), which need the candidates' global ids.
+template <bool RBL, bool EFLAG, bool GEN>
+__global__ __launch_bounds__(kEvalBlock) void kb_eval(BatchDev d, PairConst<float> pc_arg,
+                                                      BatchRange rg, int nk, int npg,
+                                                      int qlanes) {
+  __shared__ __align__(16) char buf[kStageBytes + kListBytes + (GEN ? kGidBytes : 0)];
+  __shared__ int soff[kBatchMaxSlots + 1];
+  __shared__ int sfirst[kBatchMaxSlots];
+  __shared__ int sedge[kBatchMaxSlots];
   __shared__ float s_lj[4 * kBatchMaxTypes * kBatchMaxTypes];
-  __shared__ double smem[16 * kBatchAcc];
-  const int nt = pc_arg.ntypes;
-  for (int q = threadIdx.x; q < 4 * nt * nt; q += blockDim.x) s_lj[q] = d.lj[q];
+  __shared__ double smem[(kEvalBlock / 64) * kBatchAcc];
+  const int blk = (int)blockIdx.x;
+  if (blk < nk) {
+    const int r = rg.r0 + blk;
+    kspace_replica<EFLAG>(d, pc_arg, d.rep[r], r, buf, smem);
+    return;
+  }
+  const bool lj = blk < nk + npg;
+  if (lj) {
+    const int nt = pc_arg.ntypes;
+    for (int q = threadIdx.x; q < 4 * nt * nt; q += blockDim.x) s_lj[q] = d.lj[q];
+  }
   const long long epoch = *d.epoch;
-  for (int wi = rg.w0 + blockIdx.x; wi < rg.w1; wi += gridDim.x) {
-    const BatchWork wk = d.work[wi];
+  const int w1 = lj ? rg.w1 : rg.x1;
+  for (int wi = lj ? rg.w0 + (blk - nk) : rg.x0 + (blk - nk - npg); wi < w1;
+       wi += lj ? npg : w1) {
+    const BatchWork wk = lj ? d.work[wi] : d.qwork[wi];
     const RepInfo& p = d.rep[wk.rep];
     PairConst<float> pc = pc_arg;
     if (RBL) {
@@ -314,493 +770,39 @@ __global__ __launch_bounds__(256) void kb_pair(BatchDev d, PairConst<float> pc_a
       pc.fmask = p.fmask;
       pc.c32 = p.c32;
     }
-    const Box<float> b = p.box;
-    const BrickNb h = batch_brick(p, wk.brick, bw);
-    __syncthreads();  // the previous item's readers of the tables are done
-    if (threadIdx.x < 64) {
-      int cnt = 0;
-      const int s = threadIdx.x;
-      if (s < h.nslots) {
-        const int k[3] = {s % h.rn[0], (s / h.rn[0]) % h.rn[1], s / (h.rn[0] * h.rn[1])};
-        int cw[3], e = 0;
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          const int u = h.rs[q] + k[q];
-          cw[q] = wrapi(u, p.nc[q]);
-          e |= (u < 0 ? 0 : (u >= p.nc[q] ? 2 : 1)) << (2 * q);
-        }
-        const int cell = p.c0 + (cw[2] * p.nc[1] + cw[1]) * p.nc[0] + cw[0];
-        sfirst[s] = d.start[cell];
-        cnt = d.start[cell + 1] - d.start[cell];
-        sedge[s] = e;
-      }
-      const int inc = wave_incl_scan(cnt);
-      if (s < h.nslots) soff[s] = inc - cnt;
-      if (s == 63) soff[h.nslots] = inc;
-    }
-    __syncthreads();
-    const int total = soff[h.nslots];
-    const bool staged = total <= kBatchStageCap;
-    if (staged) {
-      const int lane = threadIdx.x & 15;
-      for (int s = threadIdx.x >> 4; s < h.nslots; s += blockDim.x >> 4) {
-        const int o = soff[s], len = soff[s + 1] - o, f = sfirst[s], e = sedge[s];
-        float sh[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          const int c = (e >> (2 * q)) & 3;
-          sh[q] = c == 0 ? -b.L[q] : (c == 2 ? b.L[q] : 0.f);
-        }
-        for (int j = lane; j < len; j += 16) {
-          float4 v = d.xs[f + j];
-          v.x += sh[0];
-          v.y += sh[1];
-          v.z += sh[2];
-          sx[o + j] = v;
-          stg[o + j] = d.tg[f + j];
-        }
-      }
-    }
-    __syncthreads();
     Acc<float> a;
-    float fsx = 0.f, fsy = 0.f, fsz = 0.f;  // this thread's share of the force sum
-    // owners: the atoms of the brick's own cells, one per thread
-    // own cells u = 0..own_n-1 (x-fastest within the brick) and their
-    // atoms' running offsets (at most 8 cells)
-    const int own_n = h.w[0] * h.w[1] * h.w[2];
-    int own_end[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      int len = 0;
-      if (u < own_n) {
-        const int k[3] = {u % h.w[0], (u / h.w[0]) % h.w[1], u / (h.w[0] * h.w[1])};
-        const int s = ((h.o[2] - h.rs[2] + k[2]) * h.rn[1] + (h.o[1] - h.rs[1] + k[1])) *
-                          h.rn[0] +
-                      (h.o[0] - h.rs[0] + k[0]);
-        len = soff[s + 1] - soff[s];
-      }
-      own_end[u] = (u > 0 ? own_end[u - 1] : 0) + len;
+    float fs[3] = {0.f, 0.f, 0.f};  // this thread's share of the force sum
+    if (lj) {
+      __syncthreads();  // the previous item's readers of the tables are done
+      lj_brick<RBL, EFLAG, GEN>(d, pc, p, wk.brick, s_lj, buf, soff, sfirst, sedge, fs, a);
+    } else {
+      coul_run<RBL, EFLAG, GEN>(d, pc, p, wk.brick, qlanes, buf, fs, a);
     }
-    const int nown = own_end[7];
-    // lpo adjacent lanes per owner (up to 4, as many as the block leaves
-    // idle); lane `sub` takes every lpo-th row of the owner's stencil
-    int lpo = 1;
-    while (lpo < 4 && nown * lpo * 2 <= (int)blockDim.x) lpo *= 2;
-    for (int tt = threadIdx.x; tt < nown * lpo; tt += blockDim.x) {
-      const int t = tt / lpo, sub = tt % lpo;
-      int u = 0, ub = 0;
-#pragma unroll
-      for (int q = 0; q < 7; ++q)
-        if (own_end[q] <= t) {
-          u = q + 1;
-          ub = own_end[q];
-        }
-      const int j0 = t - ub;
-      const int k[3] = {u % h.w[0], (u / h.w[0]) % h.w[1], u / (h.w[0] * h.w[1])};
-      int ko[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) ko[q] = h.o[q] - h.rs[q] + k[q];
-      const int s_own = (ko[2] * h.rn[1] + ko[1]) * h.rn[0] + ko[0];
-      const int i = sfirst[s_own] + j0;
-      const int li = soff[s_own] + j0;
-      const float4 xi = d.xs[i];
-      const int2 tgi = d.tg[i];
-      const unsigned long long hi = RBL ? rbl_hi(tgi.y) : 0ull;
-      const bool qi = xi.w != 0.f;
-      const SpecRow sr = batch_spec_row<SPECIAL>(d, pc.ms, i);
-      float fx = 0.f, fy = 0.f, fz = 0.f;
-      int lo3[3], hi3[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        lo3[q] = h.full[q] ? 0 : ko[q] - 1;
-        hi3[q] = h.full[q] ? h.rn[q] - 1 : ko[q] + 1;
-      }
-      const int nyr = hi3[1] - lo3[1] + 1;
-      const int nrow = (hi3[2] - lo3[2] + 1) * nyr;
-      for (int row = sub; row < nrow; row += lpo) {
-        const int kz = lo3[2] + row / nyr, ky = lo3[1] + row % nyr;
-        const int srow = (kz * h.rn[1] + ky) * h.rn[0];
-        if (staged) {
-          const int l0 = soff[srow + lo3[0]], l1 = soff[srow + hi3[0] + 1];
-          if (!EFLAG && !SPECIAL) {
-            // the force pass: every candidate's terms as selects (the same
-            // pairs, weights and arithmetic as batch_lj)
-            if (h.mi)
-              batch_lj_row<RBL, true>(pc, b, s_lj, tgi.x, xi, hi, qi, li, sx, stg, l0, l1, fx,
-                                      fy, fz);
-            else
-              batch_lj_row<RBL, false>(pc, b, s_lj, tgi.x, xi, hi, qi, li, sx, stg, l0, l1,
-                                       fx, fy, fz);
-          } else {
-            for (int l = l0; l < l1; ++l) {
-              const float4 xj = sx[l];
-              if (l == li || (qi && xj.w != 0.f)) continue;
-              const int2 tgj = stg[l];
-              if (h.mi)
-                batch_lj<RBL, EFLAG, true, SPECIAL>(pc, b, s_lj, tgi.x, xi, hi, xj, tgj.x,
-                                                    tgj.y, fx, fy, fz, a, sr);
-              else
-                batch_lj<RBL, EFLAG, false, SPECIAL>(pc, b, s_lj, tgi.x, xi, hi, xj, tgj.x,
-                                                     tgj.y, fx, fy, fz, a, sr);
-            }
-          }
-        } else {
-          // beyond the stage: the same cells from global memory, minimum image
-          for (int kx = lo3[0]; kx <= hi3[0]; ++kx) {
-            const int s = srow + kx;
-            const int f = sfirst[s], len = soff[s + 1] - soff[s];
-            for (int j = 0; j < len; ++j) {
-              const float4 xj = d.xs[f + j];
-              if (f + j == i || (qi && xj.w != 0.f)) continue;
-              const int2 tgj = d.tg[f + j];
-              batch_lj<RBL, EFLAG, true, SPECIAL>(pc, b, s_lj, tgi.x, xi, hi, xj, tgj.x,
-                                                  tgj.y, fx, fy, fz, a, sr);
-            }
-          }
-        }
-      }
-      fsx += fx;
-      fsy += fy;
-      fsz += fz;
-      for (int o = lpo / 2; o > 0; o >>= 1) {
-        fx += __shfl_xor(fx, o, lpo);
-        fy += __shfl_xor(fy, o, lpo);
-        fz += __shfl_xor(fz, o, lpo);
-      }
-      if (sub == 0) d.fs[i] = make_float4(fx, fy, fz, 0.f);
-    }
-    // charged owners: LJ + Coulomb with the charged atoms of the ext_c
-    // stencil, qlanes lanes per owner.  The charged atoms of the brick
-    // widened by ext_c (a dimension that would wrap onto itself taken whole)
-    // are restaged into the LJ stage buffers, edge-shifted; a neighbourhood
-    // beyond the tables or the stage is read from global memory.
-    __syncthreads();
-    {
-      int qs[3], qn[3], qfull[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        qfull[q] = h.w[q] + 2 * p.ext_c[q] >= p.nc[q];
-        qs[q] = qfull[q] ? 0 : h.o[q] - p.ext_c[q];
-        qn[q] = qfull[q] ? p.nc[q] : h.w[q] + 2 * p.ext_c[q];
-      }
-      const int qslots = qn[0] * qn[1] * qn[2];
-      const bool qmi = qfull[0] | qfull[1] | qfull[2];
-      bool qstaged = false;
-      if (qslots <= kBatchQSlots) {
-        const int per = (qslots + blockDim.x - 1) / blockDim.x;
-        const int s0 = threadIdx.x * per, s1 = min(qslots, s0 + per);
-        int sum = 0;
-        for (int s = s0; s < s1; ++s) {
-          const int kk[3] = {s % qn[0], (s / qn[0]) % qn[1], s / (qn[0] * qn[1])};
-          int cw[3], e = 0;
-#pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            const int u = qs[q] + kk[q];
-            cw[q] = wrapi(u, p.nc[q]);
-            e |= (u < 0 ? 0 : (u >= p.nc[q] ? 2 : 1)) << (2 * q);
-          }
-          const int cell = p.c0 + (cw[2] * p.nc[1] + cw[1]) * p.nc[0] + cw[0];
-          sfirst[s] = d.start[cell];
-          sedge[s] = e;
-          const int cnt = d.qstart[cell + 1] - d.qstart[cell];
-          soff[s] = cnt;
-          sum += cnt;
-        }
-        __syncthreads();
-        int tot;
-        int run = block_excl_scan(sum, tot, sscan);
-        for (int s = s0; s < s1; ++s) {
-          const int c = soff[s];
-          soff[s] = run;
-          run += c;
-        }
-        if (threadIdx.x == 0) soff[qslots] = tot;
-        __syncthreads();
-        qstaged = tot <= kBatchStageCap;
-        if (qstaged) {
-          const int lane = threadIdx.x & 15;
-          for (int s = threadIdx.x >> 4; s < qslots; s += blockDim.x >> 4) {
-            const int o = soff[s], len = soff[s + 1] - o, f = sfirst[s], ec = sedge[s];
-            float sh[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-              const int cc = (ec >> (2 * q)) & 3;
-              sh[q] = cc == 0 ? -b.L[q] : (cc == 2 ? b.L[q] : 0.f);
-            }
-            for (int j = lane; j < len; j += 16) {
-              float4 v = d.xs[f + j];
-              v.x += sh[0];
-              v.y += sh[1];
-              v.z += sh[2];
-              sx[o + j] = v;
-              stg[o + j] = d.tg[f + j];
-            }
-          }
-        }
-        __syncthreads();
-      }
-      const int grp = threadIdx.x / qlanes, gl = threadIdx.x % qlanes;
-      const int ngrp = blockDim.x / qlanes;
-      int qend[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        int len = 0;
-        if (u < own_n) {
-          const int k[3] = {u % h.w[0], (u / h.w[0]) % h.w[1], u / (h.w[0] * h.w[1])};
-          const int cell = p.c0 + ((h.o[2] + k[2]) * p.nc[1] + h.o[1] + k[1]) * p.nc[0] +
-                           h.o[0] + k[0];
-          len = d.qstart[cell + 1] - d.qstart[cell];
-        }
-        qend[u] = (u > 0 ? qend[u - 1] : 0) + len;
-      }
-      const int nqo = qend[7];
-      for (int t0 = 0; t0 < nqo; t0 += ngrp) {
-        const int t = t0 + grp;
-        float fx = 0.f, fy = 0.f, fz = 0.f;
-        int i = -1;
-        if (t < nqo) {
-          int u = 0, ub = 0;
-#pragma unroll
-          for (int q = 0; q < 7; ++q)
-            if (qend[q] <= t) {
-              u = q + 1;
-              ub = qend[q];
-            }
-          const int k[3] = {u % h.w[0], (u / h.w[0]) % h.w[1], u / (h.w[0] * h.w[1])};
-          const int c[3] = {h.o[0] + k[0], h.o[1] + k[1], h.o[2] + k[2]};
-          const int cell = p.c0 + (c[2] * p.nc[1] + c[1]) * p.nc[0] + c[0];
-          i = d.start[cell] + (t - ub);
-          const float4 xi = d.xs[i];
-          const int ti = d.tg[i].x;
-          const unsigned long long hi = RBL ? rbl_hi(d.tg[i].y) : 0ull;
-          const SpecRow sr = batch_spec_row<SPECIAL>(d, pc.ms, i);
-          Acc<float> ac;
-          if (qstaged) {
-            // rows of the stencil in the restaged neighbourhood
-            int lo3[3], nn[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-              lo3[q] = qfull[q] ? 0 : c[q] - h.o[q];
-              nn[q] = qfull[q] ? qn[q] : 2 * p.ext_c[q] + 1;
-            }
-            const int li = soff[((c[2] - qs[2]) * qn[1] + (c[1] - qs[1])) * qn[0] +
-                                (c[0] - qs[0])] + (t - ub);
-            for (int row = gl; row < nn[1] * nn[2]; row += qlanes) {
-              const int ky = lo3[1] + row % nn[1], kz = lo3[2] + row / nn[1];
-              const int srow = (kz * qn[1] + ky) * qn[0];
-              const int l1 = soff[srow + lo3[0] + nn[0]];
-              for (int l = soff[srow + lo3[0]]; l < l1; ++l) {
-                if (l == li) continue;
-                const int2 tgj = stg[l];
-                if (qmi)
-                  batch_charged<RBL, EFLAG, true, SPECIAL>(pc, b, s_lj, ti, xi, hi, sx[l],
-                                                           tgj.x, tgj.y, ac, sr);
-                else
-                  batch_charged<RBL, EFLAG, false, SPECIAL>(pc, b, s_lj, ti, xi, hi, sx[l],
-                                                            tgj.x, tgj.y, ac, sr);
-              }
-            }
-          } else {
-            const Span spx = make_span(c[0], p.ext_c[0], p.nc[0]);
-            const Span spy = make_span(c[1], p.ext_c[1], p.nc[1]);
-            const Span spz = make_span(c[2], p.ext_c[2], p.nc[2]);
-            const int nst = spx.count * spy.count * spz.count;
-            for (int s = gl; s < nst; s += qlanes) {
-              const int kx = s % spx.count, ky = (s / spx.count) % spy.count,
-                        kz = s / (spx.count * spy.count);
-              const int cj =
-                  p.c0 + (spz.at(kz) * p.nc[1] + spy.at(ky)) * p.nc[0] + spx.at(kx);
-              const int j0 = d.start[cj], j1 = j0 + (d.qstart[cj + 1] - d.qstart[cj]);
-              for (int j = j0; j < j1; ++j) {
-                if (j == i) continue;
-                batch_charged<RBL, EFLAG, true, SPECIAL>(pc, b, s_lj, ti, xi, hi, d.xs[j],
-                                                         d.tg[j].x, d.tg[j].y, ac, sr);
-              }
-            }
-          }
-          fx = ac.fx;
-          fy = ac.fy;
-          fz = ac.fz;
-          a.e_lj += ac.e_lj;
-          a.e_c += ac.e_c;
-#pragma unroll
-          for (int q = 0; q < 6; ++q) a.v[q] += ac.v[q];
-        }
-        for (int o = qlanes / 2; o > 0; o >>= 1) {
-          fx += __shfl_xor(fx, o, qlanes);
-          fy += __shfl_xor(fy, o, qlanes);
-          fz += __shfl_xor(fz, o, qlanes);
-        }
-        if (i >= 0 && gl == 0) {
-          float4 f = d.fs[i];
-          f.x += fx;
-          f.y += fy;
-          f.z += fz;
-          d.fs[i] = f;
-          fsx += fx;
-          fsy += fy;
-          fsz += fz;
-        }
-      }
-    }
-    double v[kBatchAcc] = {(double)fsx, (double)fsy, (double)fsz, a.e_lj, a.e_c,
-                           a.v[0],      a.v[1],      a.v[2],      a.v[3], a.v[4],
-                           a.v[5]};
-    block_sum<kBatchAcc>(v, smem);
-    if (threadIdx.x == 0)
-      for (int q = 0; q < (EFLAG ? kBatchAcc : 3); ++q)
-        if (v[q] != 0.0) atomicAdd(&d.racc[(size_t)wk.rep * kBatchAcc + q], v[q]);
-  }
-}
-
-// k-space of one replica per workgroup pass: S(k) (one k per thread,
-// charged atoms staged in tiles, FP32 within a tile and FP64 across), the
-// energy and virial (FP64), then the force on every charged atom.  RBE and
-// EWALD: the k's of m, weights kw or exp(-k^2 / 4 alpha), virial
-// E_k (delta_ab - 2 k_a k_b (1/(4 alpha) + 1/k^2)).  RBSOG: the P sampled k's
-// (weight kw) and the nd direct vectors (per-replica weights kwd), every k in
-// the RBE form E_k = qqr2e (2 pi / V) w |rho|^2 / k^2; virial W_aa += E_k and
-// W_ab += tau_k |rho_s|^2 k_s,a k_s,b with s the virial-chain source of a
-// sampled k (tau = ktau, over |k_s|^4) or the direct vector itself (tau = kvd)
-// (kspace_calculator_op.hip.cu:1133-1222, :1308-1352).
-constexpr int kKsTile = 256;
-template <bool EFLAG>
-__global__ __launch_bounds__(256) void kb_kspace(BatchDev d, PairConst<float> pc,
-                                                 BatchRange rg) {
-  __shared__ float4 sa[kKsTile];
-  __shared__ float4 kf0[kBatchMaxK];
-  __shared__ float4 kf1[kBatchMaxK];
-  __shared__ double2 srho[kBatchMaxK];
-  __shared__ double smem[16 * kBatchKAcc];
-  const double two_pi = 6.283185307179586476925;
-  const int P = d.P;
-  const bool sog = d.kmode == 2;
-  const int K = P + (sog ? d.nd : 0);
-  for (int r = rg.r0 + blockIdx.x; r < rg.r1; r += gridDim.x) {
-    const RepInfo& p = d.rep[r];
-    const int* m = d.m + (size_t)r * d.mstride;
-    // integer vector of k: sampled (replica's m) or direct (shared table)
-    auto mvec = [&](int k) { return k < P ? m + 3 * k : d.dm + 3 * (k - P); };
-    double kv[kBatchKAcc] = {0, 0, 0, 0, 0, 0, 0};
-    for (int k0 = 0; k0 < K; k0 += blockDim.x) {
-      const int k = k0 + threadIdx.x;
-      const int* mk = mvec(k < K ? k : 0);
-      const float mx = (float)mk[0], my = (float)mk[1], mz = (float)mk[2];
-      double re = 0.0, im = 0.0;
-      for (int t0 = 0; t0 < p.nq; t0 += kKsTile) {
-        const int tn = min(kKsTile, p.nq - t0);
-        __syncthreads();
-        for (int j = threadIdx.x; j < tn; j += blockDim.x) {
-          const float4 x = d.xs[d.qidx[p.q0 + t0 + j]];
-          sa[j] = make_float4((x.x - p.box.lo[0]) * p.box.invL[0],
-                              (x.y - p.box.lo[1]) * p.box.invL[1],
-                              (x.z - p.box.lo[2]) * p.box.invL[2], x.w);
-        }
-        __syncthreads();
-        float fr = 0.f, fi = 0.f;
-        for (int j = 0; j < tn; ++j) {
-          const float4 a = sa[j];
-          float sn, cs;
-          sincos_rev(fma_r(mx, a.x, fma_r(my, a.y, mz * a.z)), sn, cs);
-          fr = fma_r(a.w, cs, fr);
-          fi = fma_r(a.w, sn, fi);
-        }
-        re += (double)fr;
-        im += (double)fi;
-      }
-      if (k < K) {
-        const double kx = two_pi * mk[0] / (double)p.box.L[0];
-        const double ky = two_pi * mk[1] / (double)p.box.L[1];
-        const double kz = two_pi * mk[2] / (double)p.box.L[2];
-        const double k2 = kx * kx + ky * ky + kz * kz;
-        const double wk = d.kmode == 1 ? exp(-k2 / (4.0 * (double)pc.alpha))
-                          : (k < P ? p.kw : d.kwd[(size_t)r * d.nd + (k - P)]);
-        const double A = wk * (-4.0 * 3.141592653589793238463 * (double)pc.qqr2e) /
-                         (p.volume * k2);
-        kf0[k] = make_float4((float)mk[0], (float)mk[1], (float)mk[2], (float)(A * re));
-        kf1[k] = make_float4((float)kx, (float)ky, (float)kz, (float)(A * im));
-        srho[k] = make_double2(re, im);
-        if (EFLAG) {
-          const double base =
-              (double)pc.qqr2e * two_pi / p.volume * wk * (re * re + im * im) / k2;
-          kv[0] += base;
-          if (sog) {
-            kv[1] += base;
-            kv[2] += base;
-            kv[3] += base;
-          } else {
-            const double cc = 2.0 * (1.0 / (4.0 * (double)pc.alpha) + 1.0 / k2);
-            kv[1] += base * (1.0 - cc * kx * kx);
-            kv[2] += base * (1.0 - cc * ky * ky);
-            kv[3] += base * (1.0 - cc * kz * kz);
-            kv[4] += base * (-cc * kx * ky);
-            kv[5] += base * (-cc * kx * kz);
-            kv[6] += base * (-cc * ky * kz);
-          }
-        }
-      }
-    }
-    __syncthreads();  // srho of every k is written
     if (EFLAG) {
-      if (sog)
-        for (int k = threadIdx.x; k < K; k += blockDim.x) {
-          const int src = k < P ? m[3 * P + k] : k;
-          const int* ms = mvec(src);
-          const double kx = two_pi * ms[0] / (double)p.box.L[0];
-          const double ky = two_pi * ms[1] / (double)p.box.L[1];
-          const double kz = two_pi * ms[2] / (double)p.box.L[2];
-          const double2 rs = srho[src];
-          double t = (k < P ? p.ktau : d.kvd[(size_t)r * d.nd + (k - P)]) *
-                     (rs.x * rs.x + rs.y * rs.y);
-          if (k < P) {
-            const double k2 = kx * kx + ky * ky + kz * kz;
-            t /= k2 * k2;
-          }
-          kv[1] += t * kx * kx;
-          kv[2] += t * ky * ky;
-          kv[3] += t * kz * kz;
-          kv[4] += t * kx * ky;
-          kv[5] += t * kx * kz;
-          kv[6] += t * ky * kz;
-        }
-      block_sum<kBatchKAcc>(kv, smem);
+      double v[kBatchAcc] = {(double)fs[0], (double)fs[1], (double)fs[2], a.e_lj, a.e_c,
+                             a.v[0],        a.v[1],        a.v[2],        a.v[3], a.v[4],
+                             a.v[5]};
+      block_sum<kBatchAcc>(v, smem);
       if (threadIdx.x == 0)
-        for (int q = 0; q < kBatchKAcc; ++q) d.kacc[(size_t)r * kBatchKAcc + q] = kv[q];
+        for (int q = 0; q < kBatchAcc; ++q)
+          if (v[q] != 0.0) atomicAdd(&d.racc[(size_t)wk.rep * kBatchAcc + q], v[q]);
+    } else if (RBL) {  // the mean pair force
+      double v[3] = {(double)fs[0], (double)fs[1], (double)fs[2]};
+      block_sum<3>(v, smem);
+      if (threadIdx.x == 0)
+        for (int q = 0; q < 3; ++q)
+          if (v[q] != 0.0) atomicAdd(&d.racc[(size_t)wk.rep * kBatchAcc + q], v[q]);
     }
-    __syncthreads();
-    for (int c = threadIdx.x; c < p.nq; c += blockDim.x) {
-      const int s = d.qidx[p.q0 + c];
-      const float4 x = d.xs[s];
-      const float sx = (x.x - p.box.lo[0]) * p.box.invL[0];
-      const float sy = (x.y - p.box.lo[1]) * p.box.invL[1];
-      const float sz = (x.z - p.box.lo[2]) * p.box.invL[2];
-      float fx = 0.f, fy = 0.f, fz = 0.f;
-      for (int k = 0; k < K; ++k) {
-        const float4 a = kf0[k];
-        const float4 e = kf1[k];
-        float sn, cs;
-        sincos_rev(fma_r(a.x, sx, fma_r(a.y, sy, a.z * sz)), sn, cs);
-        const float gg = fma_r(cs, e.w, -sn * a.w);
-        fx = fma_r(gg, e.x, fx);
-        fy = fma_r(gg, e.y, fy);
-        fz = fma_r(gg, e.z, fz);
-      }
-      float4 f = d.fs[s];
-      f.x += x.w * fx;
-      f.y += x.w * fy;
-      f.z += x.w * fz;
-      d.fs[s] = f;
-    }
-    __syncthreads();
   }
 }
 
-// Forces to caller order; the RBL mean pair force of each replica removed.
-__global__ __launch_bounds__(256) void kb_finish(BatchDev d, BatchRange rg, int mean_fix) {
-  const int s = rg.a0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= rg.a1) return;
-  const int i = d.perm[s];
-  float4 f = d.fs[s];
+// The force rows added in caller order; the RBL mean pair force of each
+// replica removed.
+__global__ __launch_bounds__(256) void kb_finish(BatchDev d, BatchRange rg, int mean_fix,
+                                                 int has_q, int has_k) {
+  const int i = rg.a0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= rg.a1) return;
+  float4 f = d.fs[i];
   if (mean_fix) {
     const int r = d.rep_of[i];
     const double* acc = d.racc + (size_t)r * kBatchAcc;
@@ -808,6 +810,19 @@ __global__ __launch_bounds__(256) void kb_finish(BatchDev d, BatchRange rg, int 
     f.x -= (float)(acc[0] * inv);
     f.y -= (float)(acc[1] * inv);
     f.z -= (float)(acc[2] * inv);
+  }
+  const int q = has_q ? d.qpos[i] : -1;
+  if (q >= 0) {
+    const float4 c = d.fq[q];
+    f.x += c.x;
+    f.y += c.y;
+    f.z += c.z;
+    if (has_k) {
+      const float4 k = d.fk[q];
+      f.x += k.x;
+      f.y += k.y;
+      f.z += k.z;
+    }
   }
   d.fx[i] = f.x;
   d.fy[i] = f.y;
@@ -828,40 +843,37 @@ hipError_t batch_set_epoch(long long* epoch, long long step, hipStream_t s) {
 hipError_t batch_launch(const BatchDev& d, const PairConst<float>& pc, int rbl,
                         int coulomb, int eflag, int special, const BatchRange& rg,
                         const BatchTune& t, int num_cu, hipStream_t s) {
-  const int na = rg.a1 - rg.a0, ncl = rg.c1 - rg.c0, nw = rg.w1 - rg.w0;
+  const int na = rg.a1 - rg.a0, nw = rg.w1 - rg.w0;
   if (na <= 0) return hipSuccess;
   hipLaunchKernelGGL(kb_bin, dim3(cdiv(na, 256)), dim3(256), 0, s, d, rg);
-  hipLaunchKernelGGL(kb_scan, dim3(1), dim3(1024), 0, s, d, rg);
+  hipLaunchKernelGGL(kb_scan, dim3(rg.r1 - rg.r0), dim3(256), 0, s, d, rg);
   hipLaunchKernelGGL(kb_scatter, dim3(cdiv(na, 256)), dim3(256), 0, s, d, rg);
-  hipLaunchKernelGGL(kb_cellsort, dim3(cdiv(ncl, 8)), dim3(256), 0, s, d, rg);
-  const int pg = std::max(1, std::min(nw, t.grid_per_cu * num_cu));
-#define RBMDX_KB_PAIR(RB, EF, SP)                                                      \
-  hipLaunchKernelGGL((kb_pair<RB, EF, SP>), dim3(pg), dim3(t.pair_block), 0, s, d, pc, rg, \
-                     t.bw, t.qlanes)
-#define RBMDX_KB_PAIR2(RB, EF)   \
-  if (special)                   \
-    RBMDX_KB_PAIR(RB, EF, true); \
+  hipLaunchKernelGGL(kb_cellsort, dim3(cdiv(na, 256)), dim3(256), 0, s, d, rg);
+  const int npg = std::max(1, std::min(nw, t.grid_per_cu * num_cu));
+  const int nk = coulomb && d.P > 0 ? rg.r1 - rg.r0 : 0;
+  const int nq = coulomb ? rg.x1 - rg.x0 : 0;
+  const bool gen = special || (rbl && pc.rclj2 > pc.rs2);
+#define RBMDX_KB_EVAL(RB, EF, GE)                                                        \
+  hipLaunchKernelGGL((kb_eval<RB, EF, GE>), dim3(nk + npg + nq), dim3(t.pair_block), 0, s, \
+                     d, pc, rg, nk, npg, t.qlanes)
+#define RBMDX_KB_EVAL2(RB, EF)   \
+  if (gen)                       \
+    RBMDX_KB_EVAL(RB, EF, true); \
   else                           \
-    RBMDX_KB_PAIR(RB, EF, false)
+    RBMDX_KB_EVAL(RB, EF, false)
   if (rbl && eflag) {
-    RBMDX_KB_PAIR2(true, true);
+    RBMDX_KB_EVAL2(true, true);
   } else if (rbl) {
-    RBMDX_KB_PAIR2(true, false);
+    RBMDX_KB_EVAL2(true, false);
   } else if (eflag) {
-    RBMDX_KB_PAIR2(false, true);
+    RBMDX_KB_EVAL2(false, true);
   } else {
-    RBMDX_KB_PAIR2(false, false);
+    RBMDX_KB_EVAL2(false, false);
   }
-#undef RBMDX_KB_PAIR2
-#undef RBMDX_KB_PAIR
-  if (coulomb && d.P > 0) {
-    const int kg = std::min(rg.r1 - rg.r0, 4 * num_cu);
-    if (eflag)
-      hipLaunchKernelGGL((kb_kspace<true>), dim3(kg), dim3(256), 0, s, d, pc, rg);
-    else
-      hipLaunchKernelGGL((kb_kspace<false>), dim3(kg), dim3(256), 0, s, d, pc, rg);
-  }
-  hipLaunchKernelGGL(kb_finish, dim3(cdiv(na, 256)), dim3(256), 0, s, d, rg, rbl);
+#undef RBMDX_KB_EVAL2
+#undef RBMDX_KB_EVAL
+  hipLaunchKernelGGL(kb_finish, dim3(cdiv(na, 256)), dim3(256), 0, s, d, rg, rbl,
+                     coulomb ? 1 : 0, nk > 0 ? 1 : 0);
   return hipGetLastError();
 }
 

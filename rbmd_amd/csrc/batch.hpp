@@ -14,7 +14,6 @@ namespace rbmdx {
 
 constexpr int kBatchStageCap = 1536;  // atoms staged per brick (LDS)
 constexpr int kBatchMaxSlots = 64;    // neighbourhood cells per brick (bw <= 2)
-constexpr int kBatchQSlots = 512;     // cells of the charged pass's neighbourhood
 constexpr int kBatchMaxK = 512;       // k-vectors per replica
 constexpr int kBatchMaxTypes = 8;     // atom types (LDS LJ table)
 constexpr int kBatchAcc = 11;         // per-replica pair sums: F (3), E_lj, E_c, W (6)
@@ -27,6 +26,7 @@ struct RepInfo {
   int c0;           // first global cell id; cells are x-fastest per replica
   int nc[3];        // cells per dimension (side >= the LJ pair radius)
   int ext_c[3];     // charged-pair stencil half-width in cells
+  int bw;           // brick width in cells (the batch's, or 1 where that overfills the stage)
   int nb[3];        // bricks per dimension (bw^3 cells each, ragged at the top)
   Box<float> box;
   float freq;       // RBL shell-selection frequency of this replica
@@ -37,7 +37,8 @@ struct RepInfo {
   double ktau;      // RBSOG: virial coefficient of a sampled k, -(S_npt / P) qqr2e / (4 V)
 };
 
-// One work item of the pair stage: a brick of one replica.
+// One work item of the pair stage: a brick of one replica (LJ), or the first
+// compact charged atom of a run (Coulomb).
 struct BatchWork {
   int rep, brick;
 };
@@ -49,7 +50,9 @@ struct BatchDev {
   const int* type = nullptr;      // [N] caller order
   const int* gid = nullptr;       // [N] caller order, ids within the replica
   const float* charge = nullptr;  // [N] caller order
-  const BatchWork* work = nullptr;  // [nwork], replica-major
+  const BatchWork* work = nullptr;  // [nwork] bricks, replica-major
+  const BatchWork* qwork = nullptr;  // charged runs, replica-major
+  const int* qpos = nullptr;      // [N] caller atom -> charged atoms before it, -1: neutral
   const float* lj = nullptr;      // [4 ntypes^2] (-24 eps, sigma^2, eps, sigma)
   // per evaluation
   const float* px = nullptr;
@@ -72,19 +75,21 @@ struct BatchDev {
   const int4* spn = nullptr;      // [N] (n12, n13, n14, 0)
   const int* spid = nullptr;      // [N * ms]
   // scratch
-  int* cnt = nullptr;             // [ncell] atoms per cell (zero between calls)
-  int* cntq = nullptr;            // [ncell] charged atoms per cell (likewise)
+  unsigned long long* cnt = nullptr;  // [ncell] atoms (low half) and charged atoms (high
+                                      // half) per cell, zero between calls
   int* start = nullptr;           // [ncell + 1] first sorted atom of a cell
   int* qstart = nullptr;          // [ncell + 1] first compact charged atom
   int* cell_of = nullptr;         // [N] caller atom -> global cell
   int* slot = nullptr;            // [N] caller atom -> arrival rank in its cell
-  int* tmp = nullptr;             // [N] cell-bucketed caller atoms
-  float4* xs = nullptr;           // [N] sorted (x, y, z wrapped into the box, q)
-  int2* tg = nullptr;             // [N] sorted (type, id)
-  unsigned long long* hj = nullptr;  // [N] sorted RBL hash of the id
+  int* tmp = nullptr;             // [N] cell-bucketed sort keys of the caller atoms
+  float4* xs = nullptr;           // [N] sorted (x, y, z wrapped into the box, LJ row offset)
+  int* gid_s = nullptr;           // [N] sorted ids
   int* perm = nullptr;            // [N] sorted -> caller
-  int* qidx = nullptr;            // [NQ] compact charged -> sorted
-  float4* fs = nullptr;           // [N] sorted pair + k-space force
+  float4* xqc = nullptr;          // [NQ] compact charged order: (x, y, z, q)
+  int4* qi = nullptr;             // [NQ] its (id, qpos, cell, caller atom)
+  float4* fs = nullptr;           // [N] LJ force, caller order
+  float4* fq = nullptr;           // [NQ] Coulomb pair force, by qpos
+  float4* fk = nullptr;           // [NQ] k-space force, by qpos
   double* racc = nullptr;         // [R * kBatchAcc]
   double* kacc = nullptr;         // [R * kBatchKAcc]
   long long* epoch = nullptr;     // [1] RBL sampling epoch of the evaluation
@@ -93,9 +98,9 @@ struct BatchDev {
 // Launch shapes chosen by the autotuner.
 struct BatchTune {
   int bw = 2;            // brick width in cells (1 or 2)
-  int pair_block = 128;  // threads per pair workgroup
-  int grid_per_cu = 2;   // persistent pair workgroups per CU
-  int qlanes = 8;        // lanes per charged atom in the Coulomb pass
+  int pair_block = 256;  // threads per pair workgroup
+  int grid_per_cu = 8;   // persistent LJ workgroups per CU
+  int qlanes = 16;       // lanes per charged atom in the Coulomb pass
 };
 
 // Replica range [r0, r1): atoms, cells and work items are the contiguous
@@ -104,8 +109,8 @@ struct BatchRange {
   int r0, r1;
   int a0, a1;  // atoms
   int c0, c1;  // cells
-  int w0, w1;  // work items
-  int q0;      // first compact charged atom
+  int w0, w1;  // bricks of the work list
+  int x0, x1;  // charged runs
 };
 
 hipError_t batch_set_epoch(long long* epoch, long long step, hipStream_t s);
