@@ -10,8 +10,7 @@
 //   k_scan_fin    on a rebuild the scan of the cell counts; beside it, the
 //                 S(k) reduction per k tile (rho_k, per-k energy terms and
 //                 force coefficients)
-//   k_scatter_rbe on a rebuild the scatter into cell order; beside it, the
-//                 RBE / RBSOG force per charged atom
+//   k_scatter     on a rebuild the scatter into cell order
 //   k_cellsort,   on a rebuild only (early exit otherwise): deterministic
 //   k_lists,      in-cell order and the gather in it; brick-local all-atom
 //   k_lists_dense candidate lists from LDS-staged neighbourhoods and the
@@ -23,9 +22,10 @@
 //                 add LJ + Coulomb over their charged-pair lists
 //   k_pair_b      mostly charged systems: the charged pairs, one wave per
 //                 atom (k_pair is not launched when list A is empty)
-//   k_reduce      one block: the per-block partials in a fixed order (mean
-//                 pair force, energies, virial, k-space sums; list
-//                 statistics)
+//   k_reduce      a block per component: the per-block partials in a fixed
+//                 order (mean pair force, energies, virial, k-space sums; list
+//                 statistics).  Beside them, the RBE / RBSOG force per charged
+//                 atom
 //   k_assemble    F = F_pair - <F_pair> + F_kspace in caller order (and the
 //                 leapfrog update when asked)
 // Cross-block reductions happen at kernel boundaries only: no same-address
@@ -1804,93 +1804,61 @@ struct KSum {
   double L[3] = {1.0, 1.0, 1.0};
 };
 
-// Per-thread sums in a fixed order, then one block sum of NP pair values
-// (force sum; with energies E_lj, E_coul and the virial) and, with k-space,
-// the seven k-space values.
-template <int NP, bool KS>
-__device__ __forceinline__ void reduce_sums(const double* __restrict__ pair_part,
-                                            int npair, const double* __restrict__ part2,
-                                            int npair2, const KSum& ks, double* thermo,
-                                            double* mean, int mean_fix, double n_global,
-                                            double* smem) {
-  constexpr int NV = NP + (KS ? 7 : 0);
-  double v[NV];
-#pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] = 0.0;
-  const int ntot = npair + npair2;
-  for (int blk = threadIdx.x; blk < ntot; blk += blockDim.x)
-#pragma unroll
-    for (int q = 0; q < NP; ++q)
-      v[q] += blk < npair ? pair_part[(size_t)q * npair + blk]
-                          : part2[(size_t)q * npair2 + (blk - npair)];
-  if (KS) {
-    const double two_pi = 6.283185307179586476925;
-    for (int k = threadIdx.x; k < ks.K; k += blockDim.x) {
-#pragma unroll
-      for (int q = 0; q < 7; ++q) v[NP + q] += ks.part[(size_t)k * 8 + q];
-      if (ks.tensor) {
-        const int sk = ks.src[k];
-        const double kx = two_pi * ks.m[3 * sk] / ks.L[0];
-        const double ky = two_pi * ks.m[3 * sk + 1] / ks.L[1];
-        const double kz = two_pi * ks.m[3 * sk + 2] / ks.L[2];
-        const double2 r = ks.rho[sk];
-        const double2 tv = ks.kvir[k];
-        double tt = tv.x * (r.x * r.x + r.y * r.y);
-        if (tv.y != 0.0) {
-          const double k2 = kx * kx + ky * ky + kz * kz;
-          tt /= k2 * k2;
-        }
-        v[NP + 1] += tt * kx * kx;
-        v[NP + 2] += tt * ky * ky;
-        v[NP + 3] += tt * kz * kz;
-        v[NP + 4] += tt * kx * ky;
-        v[NP + 5] += tt * kx * kz;
-        v[NP + 6] += tt * ky * kz;
-      }
-    }
-  }
-  block_sum<NV>(v, smem);
-  if (threadIdx.x == 0) {
-    if (ntot > 0) {
-      for (int q = 0; q < 11; ++q) thermo[q] = q < NP ? v[q] : 0.0;
-      for (int q = 0; q < 3; ++q) mean[q] = mean_fix ? v[q] / n_global : 0.0;
-    }
-    if (KS)
-      for (int q = 0; q < 7; ++q) thermo[16 + q] = v[NP + q];
-  }
+// Component `q` of the pair sums (one block of 256 threads): the per-block
+// FP64 partials in a fixed order into thermo[q] (0-2 force sum, 3 E_lj,
+// 4 E_coul, 5-10 virial), and of the force sum the mean pair force when
+// mean_fix.  Without energies components 3 and up are zeroed by block 0.
+__device__ __forceinline__ void reduce_pair(const double* __restrict__ pair_part, int npair,
+                                            const double* __restrict__ part2, int npair2,
+                                            int eflag, int q, double* thermo, double* mean,
+                                            int mean_fix, double n_global, double* smem) {
+  double v[1] = {0.0};
+#pragma unroll 4
+  for (int k = threadIdx.x; k < npair; k += blockDim.x) v[0] += pair_part[(size_t)q * npair + k];
+#pragma unroll 4
+  for (int k = threadIdx.x; k < npair2; k += blockDim.x) v[0] += part2[(size_t)q * npair2 + k];
+  block_sum<1>(v, smem);
+  if (threadIdx.x != 0) return;
+  thermo[q] = v[0];
+  if (q < 3) mean[q] = mean_fix ? v[0] / n_global : 0.0;
+  if (q == 0 && !eflag)
+    for (int e = 3; e < 11; ++e) thermo[e] = 0.0;
 }
 
-// One block after the pair kernels: FP64 sums of the per-block partials in
-// a fixed order (thermo[0..10]: force sum, E_lj, E_coul, virial; the mean
-// pair force when mean_fix; eflag 0 sums the force only and zeroes the rest),
-// the k-space energy and virial (thermo[16..22]) and, after a rebuild, the
-// list statistics of the per-block partials of k_lists.
-__global__ __launch_bounds__(1024) void k_reduce(
-    const double* __restrict__ pair_part, int npair,
-    const double* __restrict__ part2, int npair2, int eflag,
-    double* thermo, double* mean, int mean_fix, double n_global,
-    const int4* lista_part, int nlista, const int2* listb_part, int nlistb,
-    Ctrl* ctrl, unsigned thr, KSum ksum) {
-  __shared__ double smem[16 * 18];
-  if (npair + npair2 > 0 || ksum.K > 0) {
-    if (ksum.K > 0) {
-      if (eflag)
-        reduce_sums<11, true>(pair_part, npair, part2, npair2, ksum, thermo, mean, mean_fix,
-                              n_global, smem);
-      else
-        reduce_sums<3, true>(pair_part, npair, part2, npair2, ksum, thermo, mean, mean_fix,
-                             n_global, smem);
-    } else {
-      if (eflag)
-        reduce_sums<11, false>(pair_part, npair, part2, npair2, ksum, thermo, mean,
-                               mean_fix, n_global, smem);
-      else
-        reduce_sums<3, false>(pair_part, npair, part2, npair2, ksum, thermo, mean, mean_fix,
-                              n_global, smem);
+// Component `q` of the k-space sums into thermo[16 + q] (energy, virial
+// xx yy zz xy xz yz): the per-k terms and, for RBSOG, the tensor part.
+__device__ __forceinline__ void reduce_kspace(const KSum& ks, int q, double* thermo,
+                                              double* smem) {
+  const double two_pi = 6.283185307179586476925;
+  double v[1] = {0.0};
+  for (int k = threadIdx.x; k < ks.K; k += blockDim.x) {
+    v[0] += ks.part[(size_t)k * 8 + q];
+    if (ks.tensor && q > 0) {
+      const int sk = ks.src[k];
+      const double kx = two_pi * ks.m[3 * sk] / ks.L[0];
+      const double ky = two_pi * ks.m[3 * sk + 1] / ks.L[1];
+      const double kz = two_pi * ks.m[3 * sk + 2] / ks.L[2];
+      const double2 r = ks.rho[sk];
+      const double2 tv = ks.kvir[k];
+      double tt = tv.x * (r.x * r.x + r.y * r.y);
+      if (tv.y != 0.0) {
+        const double k2 = kx * kx + ky * ky + kz * kz;
+        tt /= k2 * k2;
+      }
+      const double ka = q == 1 || q == 4 || q == 5 ? kx : (q == 2 || q == 6 ? ky : kz);
+      const double kb = q == 1 ? kx : (q == 2 || q == 4 ? ky : kz);
+      v[0] += tt * ka * kb;
     }
   }
-  if (!rebuild_now(ctrl, thr)) return;
-  __syncthreads();
+  block_sum<1>(v, smem);
+  if (threadIdx.x == 0) thermo[16 + q] = v[0];
+}
+
+// List statistics of a rebuild (one block): the per-block partials of the
+// list builds into the control block.
+__device__ __forceinline__ void reduce_lists(const int4* lista_part, int nlista,
+                                             const int2* listb_part, int nlistb, Ctrl* ctrl,
+                                             double* smem) {
   double s[6] = {0, 0, 0, 0, 0, 0};  // max_a, sum_a, stage, unstaged, max_b, sum_b
   for (int k = threadIdx.x; k < nlista; k += blockDim.x) {
     const int4 v = lista_part[k];
@@ -2190,19 +2158,22 @@ __device__ __forceinline__ void skfin2_block(const Dev<R>& d, const Box<R>& b,
     for (int q = 0; q < 7; ++q) d.kfin_part[(size_t)k * 8 + q] = kv[q];
 }
 
-// RBE / Ewald force on 64 charged atoms (block `bid`, one lane per atom, the
-// fixed order of xqs and fk).  The per-k coefficients are staged in LDS
-// kRbeStage k's at a time; wave w takes k's w, w + nw, ... of each stage
-// with broadcast reads, and the waves' sums are added in wave order.
+// RBE / Ewald force on 2^ash charged atoms (block `bid`, the fixed order of
+// xqs and fk), block / 2^ash threads per atom.  The per-k coefficients are
+// staged in LDS kRbeStage k's at a time; thread group r of an atom takes k's
+// r, r + groups, ... of each stage with broadcast reads, and the groups' sums
+// are added in group order.  Bound by VALU and transcendental issue once the
+// machine is full, by latency below that: 64 atoms per block leave 216 blocks
+// for 13,824 charged atoms (2,196 k's: 30 us), so fewer atoms per block (more
+// threads per atom) are taken until there are kRbeBlocks of them.
 template <typename R>
 __device__ __forceinline__ void rbe2_block(const Dev<R>& d, const Box<R>& b, int K,
-                                           int bid) {
+                                           int ash, int bid) {
   __shared__ float4 s_k0[kRbeStage], s_k1[kRbeStage];
-  __shared__ float s_f[kRbeWaves][3][64];
-  const int nw = (int)blockDim.x >> 6;
-  const int t = (int)threadIdx.x, lane = t & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int c = bid * 64 + lane;
+  __shared__ float s_f[3][kBlock];
+  const int t = (int)threadIdx.x, al = t & ((1 << ash) - 1);
+  const int r = t >> ash, ng = (int)blockDim.x >> ash;
+  const int c = (bid << ash) + al;
   float sx = 0.f, sy = 0.f, sz = 0.f, q = 0.f;
   if (c < d.nc) {
     const R4T<R> pp = d.xqs[c];
@@ -2219,7 +2190,7 @@ __device__ __forceinline__ void rbe2_block(const Dev<R>& d, const Box<R>& b, int
     }
     __syncthreads();
 #pragma unroll 4
-    for (int k = wv; k < ns; k += nw) {
+    for (int k = r; k < ns; k += ng) {
       const float4 a = s_k0[k];
       const float4 e = s_k1[k];
       const float ph = fma_r(a.x, sx, fma_r(a.y, sy, a.z * sz));
@@ -2231,25 +2202,26 @@ __device__ __forceinline__ void rbe2_block(const Dev<R>& d, const Box<R>& b, int
       fz = fma_r(gg, e.z, fz);
     }
   }
-  s_f[wv][0][lane] = fx;
-  s_f[wv][1][lane] = fy;
-  s_f[wv][2][lane] = fz;
+  s_f[0][t] = fx;
+  s_f[1][t] = fy;
+  s_f[2][t] = fz;
   __syncthreads();
-  if (wv == 0 && c < d.nc) {
+  if (r == 0 && c < d.nc) {
     float ax = 0.f, ay = 0.f, az = 0.f;
-    for (int w = 0; w < nw; ++w) {
-      ax += s_f[w][0][lane];
-      ay += s_f[w][1][lane];
-      az += s_f[w][2][lane];
+    for (int w = 0; w < ng; ++w) {
+      ax += s_f[0][(w << ash) + al];
+      ay += s_f[1][(w << ash) + al];
+      az += s_f[2][(w << ash) + al];
     }
     d.fk[d.qcall[c]] = make4<R>((R)(q * ax), (R)(q * ay), (R)(q * az), R(0));
   }
 }
 
-// k-space work that rides on the rebuild kernels' launches (their blocks
-// exit at once unless the evaluation rebuilds), so that one evaluation is one
-// stream of kernels: the S(k) partials after the skin kernel has written the
-// fixed-order charged copy, their reduction next, the RBE force after that.
+// k-space work that rides on launches that leave the machine idle, so that
+// one evaluation is one stream of kernels: the S(k) partials beside the
+// binning (after the skin kernel has written the fixed-order charged copy) and
+// their reduction beside the cell scan, whose own blocks exit at once unless
+// the evaluation rebuilds, and the RBE force beside the final reduction.
 // The k-space kernels index the charged atoms in that fixed order, which a
 // rebuild does not change.
 struct KsArgs {
@@ -2260,7 +2232,8 @@ struct KsArgs {
   const int* src = nullptr;     // RBSOG virial-chain sources (device)
   int vmode = 0;                // virial form (0 RBE / EWALD, 1 RBSOG)
   int nchunks = 0, ntiles = 0;  // S(k) blocks: kSkAtoms-atom chunks x kSkK-k tiles
-  int nrbe = 0;                 // RBE force blocks (64 charged atoms each)
+  int nrbe = 0;                 // RBE force blocks (2^rbe_ash charged atoms each)
+  int rbe_ash = 6;
   Params p;
 };
 
@@ -2293,15 +2266,56 @@ __global__ __launch_bounds__(1024) void k_scan_fin(Dev<R> d, Box<R> b, int ncell
                     buf);
 }
 
-// The sorted-order scatter (blocks [0, nsc)) and the RBE force (the blocks
-// after).
+// What k_reduce adds up after the pair kernels.
+struct RedArgs {
+  const double* pair_part = nullptr;  // [11 * npair] component-major
+  int npair = 0;
+  const double* part2 = nullptr;      // [11 * npair2]
+  int npair2 = 0;
+  int eflag = 0, mean_fix = 0;
+  double n_global = 1.0;
+  double* thermo = nullptr;
+  double* mean = nullptr;
+  const int4* lista_part = nullptr;
+  int nlista = 0;
+  const int2* listb_part = nullptr;
+  int nlistb = 0;
+  Ctrl* ctrl = nullptr;
+  unsigned thr = 0;
+  KSum ks;
+  // blocks: one per pair component (0, 3 or 11), one per k-space component (0
+  // or 7), one for the list statistics; the RBE force blocks follow
+  int ncp() const { return npair + npair2 > 0 ? (eflag ? 11 : 3) : 0; }
+  int nck() const { return ks.K > 0 ? 7 : 0; }
+};
+
+// The sums after the pair kernels, a block per component so that each has one
+// short chain of loads (one block for all took 6.7 us, 17 us with energies),
+// and beside them the RBE force blocks (5 us as a launch of its own), which
+// only the assembly needs.
 template <typename R>
-__global__ __launch_bounds__(256) void k_scatter_rbe(Dev<R> d, Box<R> b, unsigned thr,
-                                                     int nsc, KsArgs ks) {
-  if ((int)blockIdx.x < nsc)
-    scatter_block<R>(d, thr, blockIdx.x, nsc);
-  else
-    rbe2_block<R>(d, b, ks.K, (int)blockIdx.x - nsc);
+__global__ __launch_bounds__(256) void k_reduce(Dev<R> d, Box<R> b, RedArgs a, int ncp,
+                                                int nck, int K, int ash) {
+  const int blk = (int)blockIdx.x;
+  if (blk > ncp + nck) {
+    rbe2_block<R>(d, b, K, ash, blk - ncp - nck - 1);
+    return;
+  }
+  __shared__ double smem[6 * 4];
+  if (blk < ncp) {
+    reduce_pair(a.pair_part, a.npair, a.part2, a.npair2, a.eflag, blk, a.thermo, a.mean,
+                a.mean_fix, a.n_global, smem);
+  } else if (blk < ncp + nck) {
+    reduce_kspace(a.ks, blk - ncp, a.thermo, smem);
+  } else if (rebuild_now(a.ctrl, a.thr)) {
+    reduce_lists(a.lista_part, a.nlista, a.listb_part, a.nlistb, a.ctrl, smem);
+  }
+}
+
+// The sorted-order scatter of a rebuild.
+template <typename R>
+__global__ __launch_bounds__(256) void k_scatter(Dev<R> d, unsigned thr) {
+  scatter_block<R>(d, thr, blockIdx.x, gridDim.x);
 }
 
 // v + 0.5 F / m dt ftm2v evaluated left to right, as RBMD's UpdateVelocity
@@ -2482,8 +2496,7 @@ hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
   hipLaunchKernelGGL((k_scan_fin<R>), dim3(kon ? 1 + ks.ntiles : 1), dim3(1024), 0, s,
                      d, a.box,
                      g.ncell, thr, ks);
-  hipLaunchKernelGGL((k_scatter_rbe<R>), dim3(gb + (kon ? ks.nrbe : 0)), dim3(kBlock), 0,
-                     s, d, a.box, thr, gb, ks);
+  hipLaunchKernelGGL((k_scatter<R>), dim3(gb), dim3(kBlock), 0, s, d, thr);
   hipLaunchKernelGGL((k_cellsort<R>), dim3(blocks_for(g.ncell * 64, kBlock)),
                      dim3(kBlock), 0, s, d, a.box, g.ncell, thr, a.pc.ms);
   const bool dense = a.p.split && d.nc > 0 && g.qblocks;
@@ -2505,10 +2518,14 @@ hipError_t launch_build(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   hipError_t e = build_part<R>(d, a, 1, s);
   if (e != hipSuccess) return e;
   // list statistics only (no pair partials)
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, s, d.pair_part, 0,
-                     (const double*)nullptr, 0, 0, d.thermo, d.mean, 0, 1.0, d.lista_part,
-                     a.grid.nbrick, d.listb_part, list_b_grid(a.p, d.nc, a.grid), d.ctrl,
-                     a.rebuild_thr, KSum());
+  RedArgs ra;
+  ra.lista_part = d.lista_part;
+  ra.nlista = a.grid.nbrick;
+  ra.listb_part = d.listb_part;
+  ra.nlistb = list_b_grid(a.p, d.nc, a.grid);
+  ra.ctrl = d.ctrl;
+  ra.thr = a.rebuild_thr;
+  hipLaunchKernelGGL((k_reduce<R>), dim3(1), dim3(256), 0, s, d, a.box, ra, 0, 0, 0, 6);
   return hipGetLastError();
 }
 
@@ -2539,7 +2556,8 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
     ks.vmode = sog ? 1 : 0;
     ks.nchunks = (d.nc + kSkAtoms - 1) / kSkAtoms;
     ks.ntiles = (K + kSkK - 1) / kSkK;
-    ks.nrbe = blocks_for(d.nc, 64);
+    while (ks.rbe_ash > 3 && blocks_for(d.nc, 1 << ks.rbe_ash) < kRbeBlocks) --ks.rbe_ash;
+    ks.nrbe = blocks_for(d.nc, 1 << ks.rbe_ash);
     ks.p = p;
   }
   if (a.ev[3]) hipEventRecord(a.ev[3], s);
@@ -2645,11 +2663,25 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
     ksum.rho = d.rho;
     for (int q = 0; q < 3; ++q) ksum.L[q] = (double)a.box.L[q];
   }
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, s, d.pair_part,
-                     has_a ? g.nbrick * g.psub : 0, (const double*)d.pairb_part, g.qblocks,
-                     p.eflag ? 1 : 0, d.thermo, d.mean, p.mean_fix, p.n_global,
-                     d.lista_part, g.nbrick, d.listb_part,
-                     list_b_grid(p, d.nc, g), d.ctrl, a.rebuild_thr, ksum);
+  RedArgs ra;
+  ra.pair_part = d.pair_part;
+  ra.npair = has_a ? g.nbrick * g.psub : 0;
+  ra.part2 = d.pairb_part;
+  ra.npair2 = g.qblocks;
+  ra.eflag = p.eflag ? 1 : 0;
+  ra.mean_fix = p.mean_fix;
+  ra.n_global = p.n_global;
+  ra.thermo = d.thermo;
+  ra.mean = d.mean;
+  ra.lista_part = d.lista_part;
+  ra.nlista = g.nbrick;
+  ra.listb_part = d.listb_part;
+  ra.nlistb = list_b_grid(p, d.nc, g);
+  ra.ctrl = d.ctrl;
+  ra.thr = a.rebuild_thr;
+  ra.ks = ksum;
+  hipLaunchKernelGGL((k_reduce<R>), dim3(ra.ncp() + ra.nck() + 1 + ks.nrbe), dim3(256), 0, s,
+                     d, a.box, ra, ra.ncp(), ra.nck(), K, ks.rbe_ash);
   hipLaunchKernelGGL((k_assemble<R>), dim3(blocks_for(d.n)), dim3(kBlock), 0,
                      s, d, p.mean_fix, has_a ? 1 : 0, ks_on ? 1 : 0, p.split ? 1 : 0, (R)a.dt,
                      (R)a.dt_ftm, a.md_kick, (R)a.ftm2v);
