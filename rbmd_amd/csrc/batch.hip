@@ -184,8 +184,7 @@ __device__ __forceinline__ SpecRow batch_spec_row(const BatchDev& d, int ms, int
 
 // LDS of kb_eval's workgroups: one buffer for the three roles.
 //   LJ: the stage (position and LJ-row offset), 64 entries of padding that
-//       the unrolled tests may read past a row, the sentinel, then the
-//       per-lane lists of accepted stage positions [kLjList][block] and, with
+//       the unrolled tests may read past a row, then the per-lane lists of accepted stage positions [kLjList][block] and, with
 //       GEN, the staged global ids;
 //   Coulomb: per-lane lists of accepted charged atoms [kQList][block];
 //   k-space: the atom tile, per-k coefficients and rho, and partial sums.
@@ -194,13 +193,34 @@ constexpr int kLjList = 44;
 constexpr int kStagePad = 64;
 constexpr int kQList = 8;
 constexpr int kKsTile = 256;
-constexpr size_t kStageBytes = (size_t)(kBatchStageCap + kStagePad + 1) * sizeof(float4);
+constexpr size_t kStageBytes = (size_t)(kBatchStageCap + kStagePad) * sizeof(float4);
 constexpr size_t kListBytes = (size_t)kLjList * kEvalBlock * sizeof(unsigned short);
 constexpr size_t kGidBytes = (size_t)kBatchStageCap * sizeof(int);
 constexpr size_t kKsBytes = kKsTile * sizeof(float4) + 2 * (size_t)kBatchMaxK * sizeof(float4) +
                             (size_t)kBatchMaxK * sizeof(double2) +
                             2 * (size_t)kEvalBlock * sizeof(double);
 static_assert(kKsBytes <= kStageBytes + kListBytes, "k-space LDS");
+
+// r^2 with room for the rounding of a test that shifts another operand across
+// the box edge than the evaluation does: coordinates are within |lo| + L of 0,
+// so the two d differ by at most 1.8e-7 (|lo| + L) per dimension and d^2 at
+// the cutoff by 3.7e-7 r times the sum of these.
+__device__ __forceinline__ float test_r2(const Box<float>& b, float r2) {
+  const float s = fabsf(b.lo[0]) + b.L[0] + fabsf(b.lo[1]) + b.L[1] + fabsf(b.lo[2]) + b.L[2];
+  return r2 + 1e-6f * sqrtf(r2) * s;
+}
+
+// Where an owner's rows wrap (MODE 2 of lj_lane): per dimension the first
+// neighbourhood cell, and the cell count of a dimension of three or four cells
+// (0: its neighbourhood is staged shifted).
+struct WrapLane {
+  int rs[3], nc[3];
+  // image shift of the owner against neighbourhood cell k
+  __device__ __forceinline__ float shift(int q, int k, const Box<float>& b) const {
+    const int u = rs[q] + k;
+    return nc[q] == 0 ? 0.f : (u < 0 ? -b.L[q] : (u >= nc[q] ? b.L[q] : 0.f));
+  }
+};
 
 // LJ pairs of one owner lane over the part [w0, w1) of the neighbourhood that
 // the stage holds.  Two phases, so that the pair terms run on lanes that hold
@@ -211,26 +231,38 @@ static_assert(kKsBytes <= kStageBytes + kListBytes, "k-space LDS");
 // lanes of an owner each take a contiguous part of every row.
 // Bound by VALU issue.  256 electrolytes (777,841 atoms): 3352 us with every
 // candidate's terms evaluated in one pass at the default shape.
-template <bool RBL, bool EFLAG, bool GEN, bool MI>
+//
+// MODE 0: every dimension is staged in shifted images.  MODE 2: some dimension
+// has three or four cells.  It is staged unshifted and its pairs take the
+// minimum image as one subtraction of L from r_j - r_i, so that a pair at a
+// cutoff falls on the side the single-box path puts it; the tests shift the
+// owner instead (per row, and in x per side of the wrapped cell: two
+// instructions a test) against test_r2, and the evaluation decides.  MODE 1: some dimension has fewer than three cells, and
+// the tests take the minimum image as well.
+template <bool RBL, bool EFLAG, bool GEN, int MODE>
 __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<float>& b,
                                         const float* s_lj, const float4* sx,
                                         const int* sgid, const int* soff,
                                         unsigned short* list, int T, const int lo3[3],
                                         const int hi3[3], int rn0, int rn1, int w0, int w1,
-                                        bool live, const float4& xi, int li, int sub,
-                                        int lsh, bool shell, unsigned long long hi,
+                                        bool live, const float4& xi, int li,
+                                        const WrapLane& wl, int sub, int lsh, bool shell, unsigned long long hi,
                                         const SpecRow& sr, float& fx, float& fy, float& fz,
                                         Acc<float>& a) {
   const float r2 = (EFLAG || GEN) ? fminf(pc.rclj2, pc.rc2) : pc.a_hi;
   const char* lj_row =
       reinterpret_cast<const char*>(s_lj) + (__float_as_int(xi.w) * pc.ntypes);
-  constexpr int kSent = kBatchStageCap + kStagePad;
+  const float r2t = MODE == 2 ? test_r2(b, r2) : r2;
   auto d2_of = [&](const float4& xj, float& dx, float& dy, float& dz) {
-    return MI ? pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz)
-              : pair_d2<float, false>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
+    return MODE ? pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz)
+                : pair_d2<float, false>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
   };
   int cnt = 0;
-  auto eval = [&](int l) {
+  // entry k of the list; past its end a stand-in (the stage's first atom)
+  // whose terms are dropped
+  auto eval = [&](int k) {
+    const bool on = k < cnt;
+    const int l = on ? list[k * T] : 0;
     const float4 xj = sx[l];
     float dx, dy, dz;
     const float d2 = d2_of(xj, dx, dy, dz);
@@ -240,14 +272,13 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
     const float s6 = s2 * s2 * s2;
     float flj = lj.x * (2.f * s6 - 1.f) * s6 * inv;
     if (!EFLAG && !GEN) {
-      // the list's test was d^2 < a_hi; the sentinel and coincident atoms go
-      const float f = ((d2 < r2) & (d2 > pc.a_lo)) ? flj : 0.f;
+      const float f = (on & (d2 < r2) & (d2 > pc.a_lo)) ? flj : 0.f;
       fx = fma_r(f, dx, fx);
       fy = fma_r(f, dy, fy);
       fz = fma_r(f, dz, fz);
       return;
     }
-    const bool in = d2 < r2;
+    const bool in = on & (d2 < r2);
     float ws = 1.f;
     if (GEN && in && sr.n14 > 0) ws = special_w<float>(sr, sgid[l], pc);
     flj *= ws;
@@ -271,10 +302,8 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
   };
   auto drain = [&]() {
     for (int k = 0; __any(k < cnt); k += 2) {
-      const int l0 = k < cnt ? list[k * T] : kSent;
-      const int l1 = k + 1 < cnt ? list[(k + 1) * T] : kSent;
-      eval(l0);
-      eval(l1);
+      eval(k);
+      eval(k + 1);
     }
     cnt = 0;
   };
@@ -286,6 +315,19 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
       const int len = max(l1 - l0, 0), part = (len + (1 << lsh) - 1) >> lsh;
       const int b0 = l0 + sub * part;
       const int n = live ? min(part, len - sub * part) : 0;
+      // MODE 2: the owner's position as the tests of this row see it, on the
+      // first xn candidates of the lane's part (x0) and on the rest (x1)
+      float x0 = xi.x, x1 = xi.x, yr = xi.y, zr = xi.z;
+      int xn = 0;
+      if (MODE == 2) {
+        yr -= wl.shift(1, ky, b);
+        zr -= wl.shift(2, kz, b);
+        x0 -= wl.shift(0, lo3[0], b);
+        x1 -= wl.shift(0, hi3[0], b);
+        // the wrapped cell is the row's first (x0) or its last (x1)
+        const int sp = x0 != xi.x ? lo3[0] + 1 : hi3[0];
+        xn = soff[srow + sp] - w0 - b0;
+      }
       for (int k0 = 0; __any(k0 < n); k0 += 32) {
         unsigned m = 0;
 #pragma unroll
@@ -298,8 +340,12 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
           const float4* xp = sx + (k0 + 8 * g < n ? b0 + k0 + 8 * g : 0);
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
-            float dx, dy, dz;
-            const float s = d2_of(xp[u], dx, dy, dz) - r2;
+            float dx, dy, dz, s;
+            if (MODE == 2)
+              s = pair_d2<float, false>(b, u + 8 * g + k0 < xn ? x0 : x1, yr, zr, xp[u].x,
+                                        xp[u].y, xp[u].z, dx, dy, dz) - r2t;
+            else
+              s = d2_of(xp[u], dx, dy, dz) - r2t;
             m = __builtin_amdgcn_alignbit(m, __float_as_uint(s), 31);
           }
         }
@@ -352,8 +398,6 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
     if (s < h.nslots) soff[s] = inc - cnt;
     if (s == 63) soff[h.nslots] = inc;
   }
-  if (threadIdx.x == 0)
-    sx[kBatchStageCap + kStagePad] = make_float4(1e18f, 1e18f, 1e18f, 0.f);
   __syncthreads();
   const int total = soff[h.nslots];
   // the brick's own cells u = 0..own_n-1 (x-fastest within the brick) and
@@ -381,6 +425,14 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
   // a neighbourhood beyond the stage goes in windows of kBatchStageCap atoms
   // (staged again for every pass over the owners)
   const bool one = total <= kBatchStageCap;
+  WrapLane wl;
+  bool unsh = false;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    wl.rs[q] = h.rs[q];
+    wl.nc[q] = p.nc[q] < 5 ? p.nc[q] : 0;
+    unsh = unsh || p.nc[q] < 5;
+  }
   for (int t0 = 0; t0 < (nown << lsh); t0 += blockDim.x) {
     const int tt = t0 + (int)threadIdx.x;
     const bool live = tt < (nown << lsh);
@@ -420,7 +472,7 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
 #pragma unroll
           for (int q = 0; q < 3; ++q) {
             const int c = (e >> (2 * q)) & 3;
-            sh[q] = c == 0 ? -b.L[q] : (c == 2 ? b.L[q] : 0.f);
+            sh[q] = p.nc[q] < 5 ? 0.f : (c == 0 ? -b.L[q] : (c == 2 ? b.L[q] : 0.f));
           }
           const int le = min(soff[s + 1], w1);
           for (int l = max(o, w0) + lane; l < le; l += 16) {
@@ -435,13 +487,17 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
         __syncthreads();
       }
       if (h.mi)
-        lj_lane<RBL, EFLAG, GEN, true>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3,
-                                       hi3, h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, sub,
-                                       lsh, shell, hi, sr, fx, fy, fz, a);
+        lj_lane<RBL, EFLAG, GEN, 1>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3, hi3,
+                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, sub,
+                                     lsh, shell, hi, sr, fx, fy, fz, a);
+      else if (unsh)
+        lj_lane<RBL, EFLAG, GEN, 2>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3, hi3,
+                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, sub,
+                                     lsh, shell, hi, sr, fx, fy, fz, a);
       else
-        lj_lane<RBL, EFLAG, GEN, false>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3,
-                                        hi3, h.rn[0], h.rn[1], w0, w1, live, xi, li - w0,
-                                        sub, lsh, shell, hi, sr, fx, fy, fz, a);
+        lj_lane<RBL, EFLAG, GEN, 0>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3, hi3,
+                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, sub,
+                                     lsh, shell, hi, sr, fx, fy, fz, a);
     }
     fs[0] += fx;
     fs[1] += fy;
@@ -496,14 +552,30 @@ __device__ __forceinline__ void coul_run(const BatchDev& d, const PairConst<floa
   const int rw = qlanes / cw, rl = gl / cw, ql = gl % cw;
   float fx = 0.f, fy = 0.f, fz = 0.f;
   int cnt = 0;
+  // The nearest image of r_j - r_i: across the edge of a dimension that the
+  // two-cell brick widened by ext_c on both sides does not cover, r_j is
+  // shifted by L before the subtraction, else r_j - r_i after it.  The last
+  // bit decides the class of a pair at a cutoff; the tests, which always
+  // shift r_j - r_i, go against test_r2.
+  const int own[3] = {cx, cy, cz};
+  bool shifted[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    shifted[q] = min(2, p.nc[q] - (own[q] & ~1)) + 2 * p.ext_c[q] < p.nc[q];
+  auto image = [&](int q, float x, float y) {
+    const float t = y - x, k = rint(t * b.invL[q]);
+    return fma_r(-k, b.L[q], shifted[q] ? y : t) - (shifted[q] ? x : 0.f);
+  };
+  const float rc2t = test_r2(b, pc.rc2);
   auto drain = [&]() {
     for (int k = 0; __any(k < cnt); ++k) {
       if (k < cnt) {
         const int j = list[k * T];
         const float4 xj = d.xqc[j];
-        float dx, dy, dz;
-        const float d2 =
-            pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
+        const float dx = image(0, xi.x, xj.x), dy = image(1, xi.y, xj.y),
+                    dz = image(2, xi.z, xj.z);
+        const float d2 = fma_r(dz, dz, fma_r(dy, dy, mul_rn(dx, dx)));
+        if (!(d2 < pc.rc2)) continue;  // the list's test has slack
         float w = 1.f, ws = 1.f;
         if (RBL || GEN) {
           const int gj = d.qi[j].x;
@@ -548,7 +620,7 @@ __device__ __forceinline__ void coul_run(const BatchDev& d, const PairConst<floa
           float dx, dy, dz;
           const float d2 = pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj[u].x, xj[u].y, xj[u].z,
                                                dx, dy, dz);
-          if (j + u * cw < j1 && j + u * cw != c && d2 < pc.rc2) {
+          if (j + u * cw < j1 && j + u * cw != c && d2 < rc2t) {
             list[cnt * T] = j + u * cw;
             ++cnt;
           }

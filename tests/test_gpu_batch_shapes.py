@@ -62,3 +62,83 @@ def test_batch_shapes_match_the_oracle(device, kind, lj_cut, shape):
         np.testing.assert_allclose(E[r, 2], ek, rtol=1e-5, atol=1e-9)
         w = np.asarray(vir) + np.asarray(vk)
         np.testing.assert_allclose(E[r, 3:], w, rtol=1e-5, atol=1e-5 * np.abs(w).max())
+
+
+def _pair_box(L, pos, q):
+    s = systems.electrolyte(2, frac_ion=0.0, seed=1)
+    s.box_len = np.array([L, L, L], dtype=np.float64)
+    s.box_lo = np.zeros(3)
+    s.pos = pos.astype(np.float64)
+    s.types = np.array([0, 1] if q else [2, 2], dtype=np.int32)
+    s.charges = np.array([1.0, -1.0] if q else [0.0, 0.0])
+    return s
+
+
+@pytest.mark.parametrize("q", [0, 1])
+def test_pairs_at_the_cutoff_across_an_edge(device, q):
+    """Boxes of three and four cells per dimension holding one pair across an
+    edge, within rounding of the cutoff: it carries a force exactly when the
+    FP32 square of its minimum image (one subtraction of L from r_j - r_i) is
+    below the cutoff's."""
+    import torch
+
+    f32 = np.float32
+    rc = 3.5 if q else 2.5
+    rng = np.random.default_rng(5 + q)
+    reps, want = [], []
+    for r in range(192):
+        L = float(f32(rng.uniform(7.6, 12.4)))
+        u = rng.normal(size=3)
+        u[r % 3] = 3.0 * np.sign(u[r % 3])
+        u /= np.linalg.norm(u)
+        x0 = rng.uniform(0.3, 0.7, 3) * L
+        x0[r % 3] = L - 0.3 if u[r % 3] > 0 else 0.3
+        x1 = x0 + u * (rc + rng.uniform(-6e-7, 6e-7))
+        x0, x1 = x0.astype(f32), (x1 - L * np.floor(x1 / L)).astype(f32)
+        d = x1 - x0
+        d = np.where(np.abs(d) > f32(0.5) * f32(L), d - np.copysign(f32(L), d), d)
+        t = f32(d[0] * d[0])
+        for k in (1, 2):  # fused: one rounding
+            t = f32(np.float64(d[k]) * np.float64(d[k]) + np.float64(t))
+        want.append(bool(t < f32(rc) * f32(rc)))
+        reps.append(_pair_box(L, np.stack([x0, x1]), q))
+    assert 40 < sum(want) < 152
+    cfg = systems.ljsalt_config(P=8)
+    cfg["hyper_parameters"]["neighbor"].update(type="Verlet-List")
+    b = BatchContext(cfg, device=0)
+    b.set_systems(reps)
+    p = torch.tensor(np.concatenate([s.pos for s in reps]).astype(f32), device=device)
+    px, py, pz = (p[:, d].contiguous() for d in range(3))
+    m = torch.zeros(3 * 8 * len(reps), dtype=torch.int32, device=device)
+    m[0::3] = 1
+    f = [torch.zeros(b.n, dtype=torch.float32, device=device) for _ in range(3)]
+    b.force(1, px, py, pz, *f, m_samples=m, energy=True, sync=True)
+    E = b.energies()
+    # the pair's own energy term: the k-space force of a charged pair is never 0
+    got = E[:, 1 if q else 0] != 0.0
+    assert got.tolist() == want
+
+
+def test_box_edge_of_a_power_of_two(device):
+    """Fewer than three cells per dimension (minimum image per pair), edges a
+    power of two, full lists, as many atoms as leave lanes idle."""
+    import torch
+
+    cfg = systems.ljsalt_config(P=8, lj_cut_off=3.5)
+    cfg["hyper_parameters"]["neighbor"].update(type="Verlet-List")
+    s = systems.electrolyte(9, frac_ion=0.0, seed=3)
+    g = np.stack(np.meshgrid([0, 1, 2], [0, 1, 2], [0], indexing="ij"), -1).reshape(-1, 3)
+    s.box_lo, s.box_len = np.zeros(3), np.array([8.0, 8.0, 8.0])
+    s.pos = 0.4 + 1.3 * g + 0.05 * np.random.default_rng(4).normal(size=(9, 3))
+    b = BatchContext(cfg, device=0)
+    b.set_systems([s])
+    p = torch.tensor(s.pos.astype(np.float32), device=device)
+    px, py, pz = (p[:, d].contiguous() for d in range(3))
+    f = [torch.zeros(b.n, dtype=torch.float32, device=device) for _ in range(3)]
+    kv = np.tile(np.array([[1, 0, 0]], dtype=np.int32), (8, 1))
+    m = torch.tensor(kv.reshape(-1), device=device)
+    Fo, en, _, _, _ = reference_force(s, s.pos.astype(np.float32), cfg, 1, kv)
+    for energy in (False, True):
+        b.force(1, px, py, pz, *f, m_samples=m, energy=energy, sync=True)
+        assert rel_rms(np.stack([t.double().cpu().numpy() for t in f], 1), Fo) < 2e-5
+    np.testing.assert_allclose(b.energies()[0, 0], en[0], rtol=1e-5)
