@@ -482,7 +482,12 @@ class Engine : public EngineBase {
     v.nq_blocks = (params_.split && d_.nc > 0 && d_.nc < n_) ? grid_.nbrick : 0;
     v.pacc = alloc<double>(3 * kVjpMaxTypes);
     // caller indices, charged atoms type-major then neutral atoms type-major,
-    // cut into chunks of at most kSkChunk atoms of one type and part
+    // cut into chunks of one type and part: at most kSkChunk atoms, charged
+    // ones fewer (down to 64) until the structure sums have kVjpSkBlocks blocks
+    int chunk_c = kSkChunk;
+    while (chunk_c > 64 &&
+           (int64_t)(d_.nc / chunk_c) * ((d_.kcap + kSkK - 1) / kSkK) < kVjpSkBlocks)
+      chunk_c /= 2;
     auto neutral = [&](int i) { return (R)q_[i] == R(0) ? 1 : 0; };
     std::vector<int> ord(n_), beg, gbeg, gtyp;
     std::iota(ord.begin(), ord.end(), 0);
@@ -503,7 +508,7 @@ class Engine : public EngineBase {
       }
       int e = s;
       while (e < n_ && neutral(ord[e]) == neutral(i0) && type_[ord[e]] == type_[i0] &&
-             e - s < kSkChunk)
+             e - s < (neutral(i0) ? kSkChunk : chunk_c))
         ++e;
       beg.push_back(s);
       s = e;

@@ -16,6 +16,7 @@ constexpr int kMaxTypes = 32;    // LJ type table held in LDS
 constexpr int kMaxSpecial = 64;  // CVFF special partners per atom
 constexpr int kSkTile = 8;       // k-vectors per S(k) block
 constexpr int kSkChunk = 1024;   // charged atoms per S(k) block
+constexpr int kVjpSkBlocks = 1024;  // adjoint structure-sum blocks wanted before a chunk grows
 constexpr int kRbeBlocks = 1024; // RBE-force blocks wanted before a block takes more atoms
 constexpr int kRbeStage = 256;   // k coefficients per LDS stage of the RBE force
 constexpr int kSkAtoms = 256;    // charged atoms per S(k) block (4 waves of 64)

@@ -2802,13 +2802,14 @@ __device__ __forceinline__ void vjp_flush(float* tab, int nt, int a, const R* s_
   if (c.ds != 0.f) atomicAdd(&tab[2 * nt + a], c.ds);
 }
 
-// Cotangent to sorted and charged order, with block sums for its mean.
+// Cotangent to sorted and charged order, with block sums for its mean (one of
+// v.gather_blocks blocks).
 template <typename R>
-__global__ __launch_bounds__(256) void k_vjp_gather(Dev<R> d, VjpDev<R> v) {
+__device__ __forceinline__ void vjp_gather_block(const Dev<R>& d, const VjpDev<R>& v) {
   if (blockIdx.x == 0 && threadIdx.x < 3 * kVjpMaxTypes) v.pacc[threadIdx.x] = 0.0;
   double s[3] = {0, 0, 0};
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < d.n;
-       i += gridDim.x * blockDim.x) {
+       i += v.gather_blocks * blockDim.x) {
     const R gx = v.gx[i], gy = v.gy[i], gz = v.gz[i];
     s[0] += (double)gx;
     s[1] += (double)gy;
@@ -2823,13 +2824,12 @@ __global__ __launch_bounds__(256) void k_vjp_gather(Dev<R> d, VjpDev<R> v) {
     for (int q = 0; q < 3; ++q) v.gpart[3 * blockIdx.x + q] = s[q];
 }
 
-__global__ __launch_bounds__(256) void k_vjp_mean(const double* gpart, int nb,
-                                                  double n, int mean_fix,
-                                                  double* gmean) {
+// The mean cotangent from the gather blocks' sums (one block of 256 threads).
+__device__ __forceinline__ void vjp_mean_block(const double* gpart, int nb, double n,
+                                               int mean_fix, double* gmean, double* smem) {
   double s[3] = {0, 0, 0};
   for (int b = threadIdx.x; b < nb; b += blockDim.x)
     for (int q = 0; q < 3; ++q) s[q] += gpart[3 * b + q];
-  __shared__ double smem[16 * 3];
   block_sum<3>(s, smem);
   if (threadIdx.x == 0)
     for (int q = 0; q < 3; ++q) gmean[q] = mean_fix ? s[q] / n : 0.0;
@@ -3294,22 +3294,28 @@ __global__ __launch_bounds__(256) void k_vjp_qnc(Dev<R> d, VjpDev<R> v, Box<R> b
     if (tab[q] != 0.f) atomicAdd(&v.pacc[q], (double)tab[q]);
 }
 
-// Adjoint structure sums: one k-vector per thread, atoms staged through LDS.
-constexpr int kVjpSkBlock = 128;  // k-vectors per block
-constexpr int kVjpSkTile = 256;   // atoms per LDS tile
-
-// Per chunk (type-major runs of at most kSkChunk atoms of one type, the
-// charged atoms' chunks first) and k: (T, U, rho, beta) with
+// Adjoint structure sums of one chunk of atoms (type-major runs of one type,
+// the charged atoms' chunks first) and kSkK k's: (T, U, rho, beta) with
 // T = sum e^{i theta}, U = sum (G . k) e^{i theta}, rho = sum q e^{i theta},
 // beta = sum q (G . k) e^{i theta}; a neutral chunk has rho = beta = 0.
-// Float sums over a tile, FP64 across tiles.
+// One lane per k; the four waves take every fourth atom of a tile staged in
+// LDS (broadcast reads), FP32 over a tile (at most 64 terms), FP64 across
+// tiles and waves.  Bound by VALU and transcendental issue once the machine is
+// full; the host cuts the charged atoms into chunks so small that it is
+// (32,000 atoms, 3,200 charged, 200 k's: 63 us with 1,024 atoms a chunk and
+// 128 k's a block, 8 blocks in all).
+constexpr int kVjpSkTile = 256;   // atoms per LDS tile
+
 template <typename R>
-__global__ __launch_bounds__(kVjpSkBlock) void k_vjp_sk(Dev<R> d, VjpDev<R> v, Box<R> b,
-                                                        const int* __restrict__ m, int K) {
+__device__ __forceinline__ void vjp_sk_block(const Dev<R>& d, const VjpDev<R>& v,
+                                             const Box<R>& b, const int* __restrict__ m, int K,
+                                             int ch, int tile) {
   __shared__ float4 sa[kVjpSkTile];  // (s_x, s_y, s_z, q)
   __shared__ float4 sg[kVjpSkTile];  // (G_x, G_y, G_z, 0)
-  const int ch = blockIdx.x;
-  const int k = blockIdx.y * kVjpSkBlock + threadIdx.x;
+  __shared__ double s_w[3][8][kSkK];
+  const int lane = (int)threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int k = tile * kSkK + lane;
   const int kk = k < K ? k : K - 1;
   const double two_pi = 6.283185307179586476925;
   const float mx = (float)m[3 * kk], my = (float)m[3 * kk + 1], mz = (float)m[3 * kk + 2];
@@ -3331,47 +3337,60 @@ __global__ __launch_bounds__(kVjpSkBlock) void k_vjp_sk(Dev<R> d, VjpDev<R> v, B
     }
     __syncthreads();
     float f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (charged) {
-      for (int j = 0; j < nt; ++j) {
+    auto sum = [&](auto with_q) {
+#pragma unroll 2
+      for (int j = wv; j < nt; j += 4) {
         const float4 a = sa[j], g = sg[j];
         float sn, cs;
         sincos_rev(fma_r(mx, a.x, fma_r(my, a.y, mz * a.z)), sn, cs);
         const float gk = fma_r(g.x, kx, fma_r(g.y, ky, g.z * kz));
-        const float qg = a.w * gk;
         f[0] += cs;
         f[1] += sn;
         f[2] = fma_r(gk, cs, f[2]);
         f[3] = fma_r(gk, sn, f[3]);
+        if (!decltype(with_q)::value) continue;
+        const float qg = a.w * gk;
         f[4] = fma_r(a.w, cs, f[4]);
         f[5] = fma_r(a.w, sn, f[5]);
         f[6] = fma_r(qg, cs, f[6]);
         f[7] = fma_r(qg, sn, f[7]);
       }
-    } else {
-      for (int j = 0; j < nt; ++j) {
-        const float4 a = sa[j], g = sg[j];
-        float sn, cs;
-        sincos_rev(fma_r(mx, a.x, fma_r(my, a.y, mz * a.z)), sn, cs);
-        const float gk = fma_r(g.x, kx, fma_r(g.y, ky, g.z * kz));
-        f[0] += cs;
-        f[1] += sn;
-        f[2] = fma_r(gk, cs, f[2]);
-        f[3] = fma_r(gk, sn, f[3]);
-      }
-    }
+    };
+    if (charged)
+      sum(std::true_type());
+    else
+      sum(std::false_type());
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[q] += (double)f[q];
   }
-  if (k < K) {
+  if (wv > 0)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s_w[wv - 1][q][lane] = acc[q];
+  __syncthreads();
+  if (wv == 0 && k < K) {
     double* o = v.vsk + ((size_t)ch * K + k) * 8;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) o[q] = acc[q];
+    for (int q = 0; q < 8; ++q)
+      o[q] = acc[q] + s_w[0][q][lane] + s_w[1][q][lane] + s_w[2][q][lane];
   }
+}
+
+// The gather and the structure sums, which read the caller's arrays alone.
+template <typename R>
+__global__ __launch_bounds__(256) void k_vjp_gather_sk(Dev<R> d, VjpDev<R> v, Box<R> b,
+                                                       const int* __restrict__ m, int K,
+                                                       int nch) {
+  const int q = (int)blockIdx.x - v.gather_blocks;
+  if (q < 0)
+    vjp_gather_block<R>(d, v);
+  else
+    vjp_sk_block<R>(d, v, b, m, K, q % nch, q / nch);
 }
 
 // One block per k: FP64 sums of the chunk partials per group (the chunks of
 // one type, charged or neutral), then the k-space charge gradient's terms of
-// this k per type and the k's coefficients of the position pass.
+// this k per type and the k's coefficients of the position pass.  Block K
+// forms the mean cotangent.
 template <typename R>
 __global__ __launch_bounds__(256) void k_vjp_sk_red(Dev<R> d, VjpDev<R> v, Box<R> b,
                                                     const int* m, int K, Params p,
@@ -3379,6 +3398,10 @@ __global__ __launch_bounds__(256) void k_vjp_sk_red(Dev<R> d, VjpDev<R> v, Box<R
   __shared__ double gsum[2 * kVjpMaxTypes][8];
   __shared__ double smem[16 * 8];
   const int k = blockIdx.x;
+  if (k == K) {
+    vjp_mean_block(v.gpart, v.gather_blocks, (double)d.n, p.mean_fix, v.gmean, smem);
+    return;
+  }
   for (int g = 0; g < ngrp; ++g) {
     double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int ch = v.grp_beg[g] + threadIdx.x; ch < v.grp_beg[g + 1]; ch += blockDim.x) {
@@ -3468,35 +3491,11 @@ __global__ __launch_bounds__(256) void k_vjp_kforce(Dev<R> d, VjpDev<R> v,
   if (live) v.drk[c] = make4<R>((R)(q * rx), (R)(q * ry), (R)(q * rz), R(0));
 }
 
-// dL/dr in caller order; keeps the evaluation counter in step with the
-// forward path (the step ring is indexed by it).
-template <typename R>
-__global__ __launch_bounds__(256) void k_vjp_assemble(Dev<R> d, VjpDev<R> v, int has_k) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) {
-    d.ctrl->maxdisp_bits = 0u;
-    d.ctrl->step_count += 1;
-    if (d.ctrl_host) d.ctrl_host->step_count = d.ctrl->step_count;
-  }
-  if (i >= d.n) return;
-  R4T<R> r = v.drs[d.inv_perm[i]];
-  const int c = d.c_of[i];
-  if (has_k && c >= 0) {
-    const R4T<R> k = v.drk[c];
-    r.x += k.x;
-    r.y += k.y;
-    r.z += k.z;
-  }
-  v.dx[i] = r.x;
-  v.dy[i] = r.y;
-  v.dz[i] = r.z;
-}
-
 // Parameter gradients: the pair passes' FP64 per-type sums (each workgroup
 // adds its LDS table with FP64 atomics) plus the k-space charge terms per k,
 // summed in a fixed order.  dparam = [dL/dQ | dL/deps | dL/dsigma].
 template <typename R>
-__global__ __launch_bounds__(256) void k_vjp_params(VjpDev<R> v, int nt, int K) {
+__device__ __forceinline__ void vjp_params_block(const VjpDev<R>& v, int nt, int K) {
   __shared__ double smem[16 * kVjpMaxTypes];
   double s[kVjpMaxTypes];
 #pragma unroll
@@ -3509,6 +3508,35 @@ __global__ __launch_bounds__(256) void k_vjp_params(VjpDev<R> v, int nt, int K) 
 #pragma unroll
     for (int q = 0; q < 3 * kVjpMaxTypes; ++q)
       if (q < 3 * nt) v.dparam[q] = v.pacc[q] + (q < nt ? s[q % kVjpMaxTypes] : 0.0);
+}
+
+// dL/dr in caller order (block 0: the parameter gradients); keeps the
+// evaluation counter in step with the forward path (the step ring is indexed
+// by it).
+template <typename R>
+__global__ __launch_bounds__(256) void k_vjp_assemble(Dev<R> d, VjpDev<R> v, int nt, int K) {
+  if (blockIdx.x == 0) {
+    vjp_params_block<R>(v, nt, K);
+    return;
+  }
+  const int i = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
+  if (i == 0) {
+    d.ctrl->maxdisp_bits = 0u;
+    d.ctrl->step_count += 1;
+    if (d.ctrl_host) d.ctrl_host->step_count = d.ctrl->step_count;
+  }
+  if (i >= d.n) return;
+  R4T<R> r = v.drs[d.inv_perm[i]];
+  const int c = d.c_of[i];
+  if (K > 0 && c >= 0) {
+    const R4T<R> k = v.drk[c];
+    r.x += k.x;
+    r.y += k.y;
+    r.z += k.z;
+  }
+  v.dx[i] = r.x;
+  v.dy[i] = r.y;
+  v.dz[i] = r.z;
 }
 
 // The rebuild part of an evaluation alone: skin check and gather, and the
@@ -3527,9 +3555,15 @@ hipError_t launch_vjp(const Dev<R>& d, const VjpDev<R>& v, const StepArgs<R>& a,
   const Params& p = a.p;
   const Grid& g = a.grid;
   const int nt = a.pc.ntypes;
-  hipLaunchKernelGGL((k_vjp_gather<R>), dim3(v.gather_blocks), dim3(kBlock), 0, s, d, v);
-  hipLaunchKernelGGL(k_vjp_mean, dim3(1), dim3(256), 0, s, v.gpart, v.gather_blocks,
-                     (double)d.n, p.mean_fix, v.gmean);
+  const int K = p.kspace && d.nc > 0 ? p.num_k : 0;
+  // with the neutral atoms' charges held at zero, only the charged chunks
+  const int nch = v.neutral_q ? v.nch : v.nch_c;
+  const int ngrp = v.neutral_q ? v.ngrp : v.ngrp_c;
+  hipLaunchKernelGGL((k_vjp_gather_sk<R>),
+                     dim3(v.gather_blocks + nch * ((K + kSkK - 1) / kSkK)), dim3(kBlock), 0, s,
+                     d, v, a.box, (const int*)d.m_dev, K, nch);
+  hipLaunchKernelGGL((k_vjp_sk_red<R>), dim3(K + 1), dim3(256), 0, s, d, v, a.box,
+                     (const int*)d.m_dev, K, p, ngrp);
   const size_t lds = 4 * sizeof(R) * (size_t)nt * nt;
 #define RBMDX_PAIR_VJP(RBL, SP)                                                 \
   hipLaunchKernelGGL((k_pair_vjp<R, RBL, SP>), dim3(g.nbrick), dim3(g.block), lds, s, \
@@ -3561,22 +3595,11 @@ hipError_t launch_vjp(const Dev<R>& d, const VjpDev<R>& v, const StepArgs<R>& a,
     }
 #undef RBMDX_QNC
   }
-  const int K = p.kspace ? p.num_k : 0;
-  const bool has_k = K > 0 && d.nc > 0;
-  // with the neutral atoms' charges held at zero, only the charged chunks
-  const int nch = v.neutral_q ? v.nch : v.nch_c;
-  const int ngrp = v.neutral_q ? v.ngrp : v.ngrp_c;
-  if (has_k) {
-    hipLaunchKernelGGL((k_vjp_sk<R>), dim3(nch, (K + kVjpSkBlock - 1) / kVjpSkBlock),
-                       dim3(kVjpSkBlock), 0, s, d, v, a.box, (const int*)d.m_dev, K);
-    hipLaunchKernelGGL((k_vjp_sk_red<R>), dim3(K), dim3(256), 0, s, d, v, a.box,
-                       (const int*)d.m_dev, K, p, ngrp);
+  if (K > 0)
     hipLaunchKernelGGL((k_vjp_kforce<R>), dim3(blocks_for(d.nc)), dim3(kBlock), 0, s, d,
                        v, a.box, K);
-  }
-  hipLaunchKernelGGL((k_vjp_assemble<R>), dim3(blocks_for(d.n)), dim3(kBlock), 0, s, d,
-                     v, has_k ? 1 : 0);
-  hipLaunchKernelGGL((k_vjp_params<R>), dim3(1), dim3(256), 0, s, v, nt, has_k ? K : 0);
+  hipLaunchKernelGGL((k_vjp_assemble<R>), dim3(1 + blocks_for(d.n)), dim3(kBlock), 0, s, d,
+                     v, nt, K);
   return hipGetLastError();
 }
 
