@@ -1132,14 +1132,48 @@ class Engine : public EngineBase {
       const double apc = (double)n_ / grid_.ncell;
       const int stage_cap = (24 * 1024) / (int)sizeof(R4);  // the kernels' LDS stage
       grid_.bw = (64.0 * apc * 1.15 <= stage_cap) ? 2 : 1;
+      // a small system takes single cells: more CUs have a brick
+      // (4,000 atoms: 27 or 216 bricks, 59 or 53 us per step).  Not with a
+      // dimension of four cells, which two-cell bricks stage whole (minimum
+      // image) and single cells in shifted images: the pairs at a cutoff would
+      // round otherwise.
+      {
+        int64_t nb2 = 1;
+        bool four = false;
+        for (int d = 0; d < 3; ++d) {
+          nb2 *= (grid_.nc[d] + 1) / 2;
+          four = four || grid_.nc[d] == 4;
+        }
+        if (nb2 < num_cu_ / 2 && !four) grid_.bw = 1;
+      }
       int nb = 1;
       for (int d = 0; d < 3; ++d) {
         grid_.nb[d] = (grid_.nc[d] + grid_.bw - 1) / grid_.bw;
         nb *= grid_.nb[d];
       }
       grid_.nbrick = nb;
-      const int per = (int)std::ceil(1.25 * apc * grid_.bw * grid_.bw * grid_.bw);
-      grid_.block = std::min(512, std::max(64, (per + 63) / 64 * 64));
+      // lanes per atom over list A: small systems split each atom's list over
+      // up to 8 lanes, which fills waves that the few atoms leave empty; beyond
+      // about one wave per SIMD the split costs more (partial groups, the list
+      // build's counting pass) than it hides.  LJ fluids, whose blocks have no
+      // list-B wave beside them, gain up to four waves per SIMD.
+      // Per step: 4,000 LJ atoms in FP64 66 -> 50 us, a 4,001-atom electrolyte
+      // 62 -> 55, 27,000 atoms 61 -> 60, 45,000 66 (67 with two lanes), 200,000 92
+      // (105 with two); 50,000 LJ atoms with energies 104 -> 78, in FP64 115 -> 97.
+      const int64_t lanes = split_ ? 65536 : 262144;
+      grid_.lsh = 0;
+      while (grid_.lsh < 3 && ((int64_t)n_ << (grid_.lsh + 1)) <= lanes) ++grid_.lsh;
+      const double per = 1.25 * apc * grid_.bw * grid_.bw * grid_.bw;
+      auto threads = [&](double lanes, int most) {
+        return std::min(most, std::max(64, ((int)std::ceil(lanes) + 63) / 64 * 64));
+      };
+      grid_.block = threads(per * (1 << grid_.lsh), 512);
+      // The adjoint's blocks hold 50 KB of LDS and 118 VGPRs a thread: three
+      // blocks of four waves fill a CU, and five or six waves per block leave it
+      // half empty (2,000,000 atoms, forward and adjoint: 1 lane per atom in 192
+      // threads 1636 us, 2 in 320 1856, 4 in 256 1542).
+      grid_.vsh = 2;
+      grid_.vblock = threads(per * (1 << grid_.vsh), 256);
       // mostly charged systems put nearly all pairs in list B: kernels of
       // their own take them, one wave per charged atom, with one resident
       // round of 5 waves per SIMD (contiguous runs of atoms per wave)

@@ -673,7 +673,11 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
                                              int split, int lcap, int cap,
                                              int& mx, int& sum) {
   const int i0 = d.key_start[2 * h.cell0], i1 = d.key_start[2 * h.cell1];
-  for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
+  // 2^lsh adjacent lanes per atom, each a contiguous range of the stencil
+  // rows: they count their entries first, and their offsets in the row follow
+  const int lsh = g.lsh, sub = (int)threadIdx.x & ((1 << lsh) - 1);
+  for (int ii = threadIdx.x; ii < (i1 - i0) << lsh; ii += blockDim.x) {
+    const int i = i0 + (ii >> lsh);
     int c[3];
     unpack_coord(g.coord_of_cell[d.cell_s[i]], c);
     const Stencil st = atom_stencil(g, h, c);
@@ -699,8 +703,11 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
     // time; the charged atoms of each cell are skipped for a charged i.
     const bool rows = STAGED && st.mode[0] != 1;
     const int runlen = rows ? st.n[0] : 1;
-    for (int kz = 0; kz < st.n[2]; ++kz)
-      for (int ky = 0; ky < st.n[1]; ++ky) {
+    const int nrow = st.n[2] * st.n[1];
+    for (int pass = lsh > 0 ? 0 : 1; pass < 2; ++pass) {
+      const bool count_pass = pass == 0;
+      for (int row_ = (nrow * sub) >> lsh; row_ < (nrow * (sub + 1)) >> lsh; ++row_) {
+        const int kz = row_ / st.n[1], ky = row_ - kz * st.n[1];
         const int srow = (st.at(2, kz) * h.cnt[1] + st.at(1, ky)) * h.cnt[0];
         for (int kx = 0; kx < st.n[0]; kx += runlen) {
           const int s0 = srow + st.at(0, kx);
@@ -734,6 +741,10 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
               if (nk < 64) ok &= (1ull << nk) - 1ull;
               const int so = self - cb;
               if (so >= 0 && so < nk) ok &= ~(1ull << so);
+              if (count_pass) {
+                count += __popcll(ok);
+                continue;
+              }
               while (ok) {
                 const int u = __builtin_ctzll(ok);
                 ok &= ok - 1;
@@ -748,11 +759,30 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
               R dx, dy, dz;
               const R d2 = pair_d2<R>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z,
                                       dx, dy, dz);
-              if (d2 < r2 && l != self) accept(l);
+              if (d2 < r2 && l != self) {
+                if (count_pass)
+                  ++count;
+                else
+                  accept(l);
+              }
             }
           }
         }
       }
+      if (count_pass) {
+        // this lane's first entry: the entries of the lanes before it
+        int inc = count;
+        for (int o = 1; o < (1 << lsh); o <<= 1) {
+          const int u = __shfl_up(inc, o, 64);
+          if (sub >= o) inc += u;
+        }
+        count = inc - count;
+        wo = (size_t)(count >> 3) * n8 + (count & 7);
+      }
+    }
+    // the atom's entries: the last lane's end
+    if (lsh > 0) count = __shfl(count, (int)(threadIdx.x & 63) | ((1 << lsh) - 1), 64);
+    if (sub != 0) continue;
     if ((count & 7) && count <= lcap) {
       // the rest of the last group: the pair kernel's sentinel entry
       const uint16_t sent = (uint16_t)((StageCap<R>::value - 1) << sh);
@@ -1295,8 +1325,8 @@ template <typename R, bool RBL, bool EFLAG, bool SHELL, bool STAGED, bool MI,
 __device__ __forceinline__ void list_a_atom(
     const Dev<R>& d, const Box<R>& b, const PairConst<R>& pc, const R* s_lj,
     const SlotTables<kMaxSlots>& t, int nslots, const R4T<R>* stage, int i,
-    int cnt, const R4T<R>& xi, int ti, unsigned long long hi, Acc<R>& a,
-    const SpecRow& sr, const int* sgid) {
+    int cnt, int sub, int lsh, const R4T<R>& xi, int ti, unsigned long long hi,
+    Acc<R>& a, const SpecRow& sr, const int* sgid) {
   using R2 = typename R2Of<R>::type;
   using R4 = R4T<R>;
   constexpr int sh = StageShift<R>::value;
@@ -1309,10 +1339,11 @@ __device__ __forceinline__ void list_a_atom(
     return t.first[s] + (l - t.off[s]);
   };
   // the next 16-byte group is loaded while the current one is evaluated
-  uint4 q_next = cnt > 0 ? lp[0] : make_uint4(0u, 0u, 0u, 0u);
-  for (int k0 = 0; k0 < cnt; k0 += 8) {
+  const int step = 8 << lsh;  // groups sub, sub + 2^lsh, ...
+  uint4 q_next = 8 * sub < cnt ? lp[(size_t)sub * d.n] : make_uint4(0u, 0u, 0u, 0u);
+  for (int k0 = 8 * sub; k0 < cnt; k0 += step) {
     const uint4 q8 = q_next;
-    if (k0 + 8 < cnt) q_next = lp[(size_t)((k0 >> 3) + 1) * d.n];
+    if (k0 + step < cnt) q_next = lp[(size_t)((k0 + step) >> 3) * d.n];
     const int kn = cnt - k0;
     const unsigned wv[4] = {q8.x, q8.y, q8.z, q8.w};
 #pragma unroll
@@ -1469,8 +1500,10 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
     const int i0 = d.key_start[2 * h.cell0], i1 = d.key_start[2 * h.cell1];
     // phase 1: LJ over list A, the atoms in the order of the last rebuild
     // (longest list first)
-    for (int k = (int)threadIdx.x; k < i1 - i0 && (int)threadIdx.x < TA; k += TA) {
-      const int i = d.order_a[i0 + k];
+    // 2^lsh adjacent lanes per atom, each every 2^lsh-th group of its list
+    const int lsh = g.lsh, sub_l = (int)threadIdx.x & ((1 << lsh) - 1);
+    for (int k = (int)threadIdx.x; k < (i1 - i0) << lsh && (int)threadIdx.x < TA; k += TA) {
+      const int i = d.order_a[i0 + (k >> lsh)];
       Acc<R> a;
       const R4T<R> xi = d.xs[i];
       const int ti = (int)xi.w;
@@ -1480,14 +1513,14 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
       if (cnt <= d.cap_a) {
         if (staged && !h.mi)
           list_a_atom<R, RBL, EFLAG, SHELL, true, false, SPECIAL>(
-              d, b, pc, s_lj, t, h.nslots, stage, i, cnt, xi, ti, hi, a, sr, sgid);
+              d, b, pc, s_lj, t, h.nslots, stage, i, cnt, sub_l, lsh, xi, ti, hi, a, sr, sgid);
         else if (staged)
           list_a_atom<R, RBL, EFLAG, SHELL, true, true, SPECIAL>(
-              d, b, pc, s_lj, t, h.nslots, stage, i, cnt, xi, ti, hi, a, sr, sgid);
+              d, b, pc, s_lj, t, h.nslots, stage, i, cnt, sub_l, lsh, xi, ti, hi, a, sr, sgid);
         else
           list_a_atom<R, RBL, EFLAG, SHELL, false, true, SPECIAL>(
-              d, b, pc, s_lj, t, h.nslots, stage, i, cnt, xi, ti, hi, a, sr, sgid);
-      } else {
+              d, b, pc, s_lj, t, h.nslots, stage, i, cnt, sub_l, lsh, xi, ti, hi, a, sr, sgid);
+      } else if (sub_l == 0) {
         // list overflow since the last rebuild: scan the 27 cells directly
         int c[3];
         unpack_coord(g.coord_of_cell[d.cell_s[i]], c);
@@ -1509,7 +1542,6 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
               }
             }
       }
-      d.fa[d.perm[i]] = make4<R>(a.fx, a.fy, a.fz, R(0));
       acc.fx += a.fx;
       acc.fy += a.fy;
       acc.fz += a.fz;
@@ -1517,6 +1549,12 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
         acc.e_lj += a.e_lj;
         for (int k = 0; k < 6; ++k) acc.v[k] += a.v[k];
       }
+      for (int o = 1; o < (1 << lsh); o <<= 1) {
+        a.fx += __shfl_xor(a.fx, o, 64);
+        a.fy += __shfl_xor(a.fy, o, 64);
+        a.fz += __shfl_xor(a.fz, o, 64);
+      }
+      if (sub_l == 0) d.fa[d.perm[i]] = make4<R>(a.fx, a.fy, a.fz, R(0));
     }
   }
   // phase 2: charged atoms of the brick over list B, QL lanes per atom (8 in
@@ -2938,9 +2976,11 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
   }
   constexpr int sh = StageShift<R>::value;
   const int i0 = d.key_start[2 * h.cell0], i1 = d.key_start[2 * h.cell1];
-  // the brick's atoms in the pair kernel's order (longest list first)
-  for (int k = (int)threadIdx.x; k < i1 - i0; k += blockDim.x) {
-    const int i = d.order_a[i0 + k];
+  // the brick's atoms in the pair kernel's order (longest list first),
+  // 2^lsh adjacent lanes per atom, each every 2^lsh-th group of its list
+  const int lsh = g.vsh, sub = (int)threadIdx.x & ((1 << lsh) - 1);
+  for (int k = (int)threadIdx.x; k < (i1 - i0) << lsh; k += blockDim.x) {
+    const int i = d.order_a[i0 + (k >> lsh)];
     const R4T<R> xi = d.xs[i];
     const int ti = (int)xi.w;
     const R4T<R> g4 = v.gs[i];
@@ -2977,7 +3017,7 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
       auto run = [&](auto mi) {
         constexpr bool MI = decltype(mi)::value;
         const uint4* lp = reinterpret_cast<const uint4*>(d.list_a) + i;
-        for (int k0 = 0; k0 < cnt; k0 += 8) {
+        for (int k0 = 8 * sub; k0 < cnt; k0 += 8 << lsh) {
           const uint4 q8 = lp[(size_t)(k0 >> 3) * d.n];
           const unsigned wv[4] = {q8.x, q8.y, q8.z, q8.w};
 #pragma unroll
@@ -3002,7 +3042,7 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
         run(std::false_type());
     } else if (staged && cnt <= d.cap_a) {
       const uint4* lp = reinterpret_cast<const uint4*>(d.list_a) + i;
-      for (int k0 = 0; k0 < cnt; k0 += 8) {
+      for (int k0 = 8 * sub; k0 < cnt; k0 += 8 << lsh) {
         const uint4 q8 = lp[(size_t)(k0 >> 3) * d.n];
         const unsigned wv[4] = {q8.x, q8.y, q8.z, q8.w};
         const int kn = min(8, cnt - k0);
@@ -3019,7 +3059,7 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
           one(dx, dy, dz, u, tj, gj, gidj);
         }
       }
-    } else {
+    } else if (sub == 0) {
       // unstaged brick or list overflow: scan the 27 cells directly
       int c[3];
       unpack_coord(g.coord_of_cell[d.cell_s[i]], c);
@@ -3044,6 +3084,13 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
             }
           }
     }
+    for (int o = 1; o < (1 << lsh); o <<= 1) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) r[q] += __shfl_xor(r[q], o, 64);
+      acc.de += __shfl_xor(acc.de, o, 64);
+      acc.ds += __shfl_xor(acc.ds, o, 64);
+    }
+    if (sub != 0) continue;
     v.drs[i] = make4<R>(r[0], r[1], r[2], R(0));
     vjp_flush<R>(tab, nt, ti, s_lj, acc);
   }
@@ -3566,7 +3613,7 @@ hipError_t launch_vjp(const Dev<R>& d, const VjpDev<R>& v, const StepArgs<R>& a,
                      (const int*)d.m_dev, K, p, ngrp);
   const size_t lds = 4 * sizeof(R) * (size_t)nt * nt;
 #define RBMDX_PAIR_VJP(RBL, SP)                                                 \
-  hipLaunchKernelGGL((k_pair_vjp<R, RBL, SP>), dim3(g.nbrick), dim3(g.block), lds, s, \
+  hipLaunchKernelGGL((k_pair_vjp<R, RBL, SP>), dim3(g.nbrick), dim3(g.vblock), lds, s, \
                      d, v, a.box, g, a.pc, a.lj_tab, p.split)
   if (p.special) {
     if (p.rbl)
