@@ -292,23 +292,20 @@ class Engine : public EngineBase {
     p.num_steps = m.num_steps;
     p.e_self = e_self_;
     if (!md_state_) {
-      // [0], [1]: the alternating running states; [2]: the next step's opened state
-      md_state_ = alloc<MdState>(3);
+      md_state_ = alloc<MdState>(3);  // MdCopy
       md_part_ = alloc<double>(std::max<int64_t>(kMdParts, md_assemble_parts()));
     }
     const MdArrays<R> a = md_arrays(c);
     md_ = p;
     md_ready_ = false;
     HIPCHK(hipMemsetAsync(md_state_, 0, 3 * sizeof(MdState), s));
-    md_cur_ = 0;
     HIPCHK(md_launch_wrap(a, s));
     const uint32_t ff = md_force_flags(flags);
     force(0, c.px, c.py, c.pz, c.fx, c.fy, c.fz, nullptr, 0, ff, s);
     HIPCHK(md_launch_second(a, md_, 0, s));
     HIPCHK(md_launch_thermostat(md_, md_part_, md_init_parts(n_), d_.thermo,
-                                md_state_ + md_cur_, md_state_ + (md_cur_ ^ 1),
-                                md_state_ + 2, 0, 1, (ff & RBMDX_FLAG_ENERGY) ? 1 : 0, s));
-    md_cur_ ^= 1;
+                                md_state_ + kMdStep, md_state_ + kMdClosed,
+                                md_state_ + kMdOpen, 1, (ff & RBMDX_FLAG_ENERGY) ? 1 : 0, s));
     md_step_ = 0;
     md_ready_ = true;
   }
@@ -323,39 +320,50 @@ class Engine : public EngineBase {
     HIPCHK(hipSetDevice(device_));
     const MdArrays<R> a = md_arrays(c);
     const uint32_t ff = md_force_flags(flags);
-    const int with_pe = (ff & RBMDX_FLAG_ENERGY) ? 1 : 0;
-    MdState* open = md_state_ + 2;
-    if (nsteps > 0) HIPCHK(md_launch_open(md_, md_state_ + md_cur_, open, md_step_ + 1, s));
-    const int parts = (int)md_assemble_parts();
-    for (int32_t k = 0; k < nsteps; ++k) {
-      const int64_t step = md_step_ + 1;
-      HIPCHK(md_launch_first(a, md_, open, md_state_ + (md_cur_ ^ 1), s));
-      md_cur_ ^= 1;
-      // the force with the closing half-kick and kinetic-energy partials
-      // folded into its assembly kernel
-      d_.vx = (R*)c.vx;
-      d_.vy = (R*)c.vy;
-      d_.vz = (R*)c.vz;
-      d_.md_mass = md_mass_;
-      d_.md_part = md_part_;
-      md_kick_ = true;
-      try {
-        force(step, c.px, c.py, c.pz, c.fx, c.fy, c.fz, nullptr, 0, ff, s);
-      } catch (...) {
-        d_.vx = d_.vy = d_.vz = nullptr;
-        md_kick_ = false;
-        throw;
-      }
-      d_.vx = d_.vy = d_.vz = nullptr;
+    if (nsteps == 0) return;  // nothing pending
+    HIPCHK(md_launch_open(md_, md_state_ + kMdClosed, md_state_ + kMdOpen, md_step_ + 1, s));
+    // a step is one evaluation: its first kernel opens the step, the assembly
+    // closes it, the thermostat follows (launch_step)
+    d_.vx = (R*)c.vx;
+    d_.vy = (R*)c.vy;
+    d_.vz = (R*)c.vz;
+    d_.xw = (R*)c.px;
+    d_.yw = (R*)c.py;
+    d_.zw = (R*)c.pz;
+    d_.ix = c.ix;
+    d_.iy = c.iy;
+    d_.iz = c.iz;
+    d_.md_mass = md_mass_;
+    d_.md_part = md_part_;
+    d_.md_open = md_state_ + kMdOpen;
+    md_kick_ = true;
+    auto unbind = [&] {
+      d_.vx = d_.vy = d_.vz = d_.xw = d_.yw = d_.zw = nullptr;
+      d_.ix = d_.iy = d_.iz = nullptr;
       md_kick_ = false;
-      HIPCHK(md_launch_thermostat(md_, md_part_, parts, d_.thermo, md_state_ + md_cur_,
-                                  md_state_ + (md_cur_ ^ 1), open, step, 0, with_pe, s));
-      md_cur_ ^= 1;
-      md_step_ = step;
+    };
+    try {
+      for (int32_t k = 0; k < nsteps; ++k) {
+        force(md_step_ + 1, c.px, c.py, c.pz, c.fx, c.fy, c.fz, nullptr, 0, ff, s);
+        ++md_step_;
+      }
+    } catch (...) {
+      unbind();
+      throw;
     }
+    unbind();
     // leave the caller's velocities with the last thermostat factor applied
-    HIPCHK(md_launch_apply(a, md_state_ + md_cur_, md_state_ + (md_cur_ ^ 1), s));
-    md_cur_ ^= 1;
+    HIPCHK(md_launch_apply(a, md_state_ + kMdStep, md_state_ + kMdClosed, s));
+  }
+
+  // One evaluation, and for an MD step the thermostat behind it.
+  hipError_t launch_step(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
+    hipError_t e = launch_force<R>(d, a, s);
+    if (e == hipSuccess && a.md_kick)
+      e = md_launch_thermostat(md_, md_part_, (int)md_assemble_parts(), d.thermo,
+                               md_state_ + kMdOpen, md_state_ + kMdStep, md_state_ + kMdOpen, 0,
+                               a.p.eflag, s);
+    return e;
   }
 
   void md_state(rbmdx_md_state_t* out) override {
@@ -363,7 +371,7 @@ class Engine : public EngineBase {
     HIPCHK(hipSetDevice(device_));
     if (last_stream_set_) HIPCHK(hipStreamSynchronize(last_stream_));
     MdState st;
-    HIPCHK(hipMemcpy(&st, md_state_ + md_cur_, sizeof(MdState), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(&st, md_state_ + kMdClosed, sizeof(MdState), hipMemcpyDeviceToHost));
     std::memset(out, 0, sizeof(*out));
     out->step = md_step_;
     out->mode = md_.mode;
@@ -740,7 +748,7 @@ class Engine : public EngineBase {
         auto& ev = timing_events_[timing_used_++];
         for (int q = 0; q < 6; ++q) a.ev[q] = ev[q];
       }
-      HIPCHK(launch_force<R>(d_, a, s));
+      HIPCHK(launch_step(d_, a, s));
     }
     HIPCHK(hipEventRecord(slot_events_[slot], s));
     slot_used_[slot] = true;
@@ -762,10 +770,11 @@ class Engine : public EngineBase {
   // Everything a captured evaluation bakes into its kernel arguments besides
   // the device buffers (whose reallocation bumps gen_).
   struct GraphKey {
-    const void* ptr[12];
+    const void* ptr[15];
     int eflag, num_k, m_from_ring, md_kick;
     double dt;
     uint64_t gen;
+    MdParams md;
   };
   static constexpr int kGraphCopies = 2;  // executable copies launched in turn
   static constexpr int kGraphCache = 4;   // captured evaluation shapes kept
@@ -778,15 +787,16 @@ class Engine : public EngineBase {
   GraphKey graph_key(const StepArgs<R>& a) const {
     GraphKey g;
     std::memset(&g, 0, sizeof g);
-    const void* p[12] = {d_.px, d_.py, d_.pz, d_.fx, d_.fy, d_.fz,
-                         d_.vx, d_.vy, d_.vz, d_.xw, d_.yw, d_.zw};
-    for (int q = 0; q < 12; ++q) g.ptr[q] = p[q];
+    const void* p[15] = {d_.px, d_.py, d_.pz, d_.fx, d_.fy, d_.fz, d_.vx, d_.vy,
+                         d_.vz, d_.xw, d_.yw, d_.zw, d_.ix, d_.iy, d_.iz};
+    for (int q = 0; q < 15; ++q) g.ptr[q] = p[q];
     g.eflag = a.p.eflag;
     g.num_k = a.p.num_k;
     g.m_from_ring = a.m_from_ring;
     g.md_kick = a.md_kick;
     g.dt = a.dt;
     g.gen = gen_;
+    if (a.md_kick) std::memcpy(&g.md, &md_, sizeof md_);  // the thermostat's constants
     return g;
   }
 
@@ -806,7 +816,7 @@ class Engine : public EngineBase {
     }
     if (!cap_stream_) HIPCHK(hipStreamCreateWithFlags(&cap_stream_, hipStreamNonBlocking));
     HIPCHK(hipStreamBeginCapture(cap_stream_, hipStreamCaptureModeRelaxed));
-    const hipError_t e1 = launch_force<R>(d_, a, cap_stream_);
+    const hipError_t e1 = launch_step(d_, a, cap_stream_);
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(cap_stream_, &g);
     if (e1 != hipSuccess || e2 != hipSuccess || !g) {
@@ -1002,7 +1012,6 @@ class Engine : public EngineBase {
   MdState* md_state_ = nullptr;
   double* md_part_ = nullptr;
   MdParams md_;
-  int md_cur_ = 0;
   int64_t md_step_ = 0;
   bool md_ready_ = false;
   bool md_kick_ = false;  // the current evaluation is an MD step's force

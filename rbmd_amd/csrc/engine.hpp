@@ -30,6 +30,8 @@ constexpr int kQWaves = 4;  // waves per block of the dense charged-pair kernel
 // counts and box-edge shifts [kMaxSlots each].
 constexpr int kBrickTabInts = 4 * kMaxSlots + 1;
 
+struct MdState;  // md.hpp
+
 // Device control block: rebuild decision, overflow bookkeeping.
 struct Ctrl {
   unsigned int maxdisp_bits;  // max |dr|^2 since the last rebuild (float bits)
@@ -157,6 +159,10 @@ struct Dev {
   R* inv_mass = nullptr;   // [ntypes]
   const double* md_mass = nullptr;  // [ntypes] FP64 masses (MD closing half-kick)
   double* md_part = nullptr;        // [assemble workgroups] sum m v^2 (MD step)
+  const MdState* md_open = nullptr; // the opened state of the MD step
+  int* ix = nullptr;       // [n] image flags of an MD step (may be null)
+  int* iy = nullptr;
+  int* iz = nullptr;
   int* type = nullptr;     // [n]
   int* gid = nullptr;      // [n]
   R* charge = nullptr;     // [n]
@@ -274,8 +280,10 @@ struct StepArgs {
   double e_self = 0.0;        // k-space self + background energy
   double dt = 0.0;            // fused leapfrog: x += dt v
   double dt_ftm = 0.0;        //                 v += dt ftm2v F / m
-  int md_kick = 0;            // MD step: closing half-kick + kinetic energy
-  double ftm2v = 1.0;         //          (dt above is the time step)
+  int md_kick = 0;            // MD step: opening half-kick, drift and wrap ahead of
+                              //          the evaluation, closing half-kick + kinetic
+                              //          energy after it (dt above is the time step)
+  double ftm2v = 1.0;
   hipEvent_t ev[6] = {};      // optional section timing events
 };
 

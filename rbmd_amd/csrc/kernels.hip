@@ -38,6 +38,7 @@
 
 #include "device.hpp"
 #include "engine.hpp"
+#include "md.hpp"
 
 namespace rbmdx {
 namespace {
@@ -339,9 +340,40 @@ __device__ __forceinline__ void unpack_coord(int packed, int c[3]) {
 // the gather.  force (an explicit rebuild of the list builder alone) skips
 // the sorted gather.
 // ---------------------------------------------------------------------------
+// v + 0.5 F / m dt ftm2v evaluated left to right, as RBMD's UpdateVelocity
+// (update_velocity_op.hip.cu:19-21), without contraction into FMA.
 template <typename R>
+__device__ __forceinline__ R md_half_kick(R v, R f, R m, R dt, R ftm2v) {
+#pragma clang fp contract(off)
+  return v + (R)0.5 * f / m * dt * ftm2v;
+}
+
+// The opening of a velocity-Verlet step on one atom: the thermostat's pending
+// factor, the half-kick with the last force, the drift, and the periodic wrap
+// (one image shift, flags counted), without contraction into FMA.
+template <typename R>
+__device__ __forceinline__ void md_open_coord(R& x, R& v, R f, R sc, R m, R dt, R ftm2v,
+                                              R lo, R hi, R L, int* img, int i) {
+#pragma clang fp contract(off)
+  if (sc != (R)1) v *= sc;
+  v = md_half_kick(v, f, m, dt, ftm2v);
+  x = x + v * dt;
+  if (x >= hi) {
+    x -= L;
+    if (img) img[i] += 1;
+  }
+  if (x < lo) {
+    x += L;
+    if (img) img[i] -= 1;
+  }
+}
+
+// MD: the evaluation of a molecular-dynamics step.  The step's opening (kick,
+// drift, wrap) rides on this pass over the atoms (4.3 us as a kernel of its
+// own at 200,000 atoms).
+template <typename R, bool MD>
 __global__ __launch_bounds__(256) void k_skin(Dev<R> d, Box<R> b, int force, int ctl,
-                                              int kcopy, int with_src) {
+                                              int kcopy, int with_src, R dt, R ftm2v) {
   __shared__ float s_max[4];
   const int nab = (int)gridDim.x - ctl;  // blocks over the atoms
   if ((int)blockIdx.x == nab) {
@@ -373,10 +405,25 @@ __global__ __launch_bounds__(256) void k_skin(Dev<R> d, Box<R> b, int force, int
     return;
   }
   float mx = 0.f;
+  const R sc = MD ? (R)d.md_open->scale : R(1);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < d.n; i += nab * blockDim.x) {
-    const R x = wrap<R>(d.px[i], b.lo[0], b.hi[0], b.L[0], b.invL[0]);
-    const R y = wrap<R>(d.py[i], b.lo[1], b.hi[1], b.L[1], b.invL[1]);
-    const R z = wrap<R>(d.pz[i], b.lo[2], b.hi[2], b.L[2], b.invL[2]);
+    R cx0 = d.px[i], cy0 = d.py[i], cz0 = d.pz[i];
+    if (MD) {
+      const R m = (R)d.md_mass[d.type[i]];
+      R vx = d.vx[i], vy = d.vy[i], vz = d.vz[i];
+      md_open_coord(cx0, vx, d.fx[i], sc, m, dt, ftm2v, b.lo[0], b.hi[0], b.L[0], d.ix, i);
+      md_open_coord(cy0, vy, d.fy[i], sc, m, dt, ftm2v, b.lo[1], b.hi[1], b.L[1], d.iy, i);
+      md_open_coord(cz0, vz, d.fz[i], sc, m, dt, ftm2v, b.lo[2], b.hi[2], b.L[2], d.iz, i);
+      d.vx[i] = vx;
+      d.vy[i] = vy;
+      d.vz[i] = vz;
+      d.xw[i] = cx0;
+      d.yw[i] = cy0;
+      d.zw[i] = cz0;
+    }
+    const R x = wrap<R>(cx0, b.lo[0], b.hi[0], b.L[0], b.invL[0]);
+    const R y = wrap<R>(cy0, b.lo[1], b.hi[1], b.L[1], b.invL[1]);
+    const R z = wrap<R>(cz0, b.lo[2], b.hi[2], b.L[2], b.invL[2]);
     // the charged atoms in their fixed order for the k-space kernels
     // (independent of the sorted order, so also on a forced rebuild)
     if (d.qpos) {
@@ -2356,14 +2403,6 @@ __global__ __launch_bounds__(256) void k_scatter(Dev<R> d, unsigned thr) {
   scatter_block<R>(d, thr, blockIdx.x, gridDim.x);
 }
 
-// v + 0.5 F / m dt ftm2v evaluated left to right, as RBMD's UpdateVelocity
-// (update_velocity_op.hip.cu:19-21), without contraction into FMA.
-template <typename R>
-__device__ __forceinline__ R md_half_kick(R v, R f, R m, R dt, R ftm2v) {
-#pragma clang fp contract(off)
-  return v + (R)0.5 * f / m * dt * ftm2v;
-}
-
 // Total force in caller order (one thread per caller atom); resets the skin
 // accumulator for the next call and mirrors the counters to the host.  With
 // velocities bound it also applies the leapfrog update
@@ -2552,7 +2591,8 @@ hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
 
 template <typename R>
 hipError_t launch_build(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_skin<R>), dim3(1), dim3(kBlock), 0, s, d, a.box, 1, 0, 0, 0);
+  hipLaunchKernelGGL((k_skin<R, false>), dim3(1), dim3(kBlock), 0, s, d, a.box, 1, 0, 0, 0,
+                     R(0), R(0));
   hipError_t e = build_part<R>(d, a, 1, s);
   if (e != hipSuccess) return e;
   // list statistics only (no pair partials)
@@ -2580,8 +2620,12 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   // does the sampled k-sample, which k_skin copies to HBM)
   const int kcopy = (ks_on && a.m_from_ring) ? K : 0;
   const int ctl = d.hdr_ring ? 1 : 0;
-  hipLaunchKernelGGL((k_skin<R>), dim3(sb + ctl), dim3(kBlock), 0, s, d, a.box, 0, ctl,
-                     kcopy, p.kspace == 3 ? 1 : 0);
+  if (a.md_kick)
+    hipLaunchKernelGGL((k_skin<R, true>), dim3(sb + ctl), dim3(kBlock), 0, s, d, a.box, 0, ctl,
+                       kcopy, p.kspace == 3 ? 1 : 0, (R)a.dt, (R)a.ftm2v);
+  else
+    hipLaunchKernelGGL((k_skin<R, false>), dim3(sb + ctl), dim3(kBlock), 0, s, d, a.box, 0, ctl,
+                       kcopy, p.kspace == 3 ? 1 : 0, R(0), R(0));
   // k-space blocks beside the rebuild kernels' blocks (one stream, no fork)
   KsArgs ks;
   if (ks_on) {
@@ -3592,7 +3636,8 @@ template <typename R>
 hipError_t launch_skin_build(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   const int sb = blocks_for(d.n, kBlock, kSkinBlocksMax);
   const int ctl = d.hdr_ring ? 1 : 0;
-  hipLaunchKernelGGL((k_skin<R>), dim3(sb + ctl), dim3(kBlock), 0, s, d, a.box, 0, ctl, 0, 0);
+  hipLaunchKernelGGL((k_skin<R, false>), dim3(sb + ctl), dim3(kBlock), 0, s, d, a.box, 0, ctl, 0,
+                     0, R(0), R(0));
   return build_part<R>(d, a, sb + ctl, s);
 }
 

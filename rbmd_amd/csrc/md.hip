@@ -9,13 +9,13 @@
 //   F = force(x),  v += dt/2 F/m,
 //   [NVT] temperature, chain half-step (scales v)
 //   [NVE + RBL] temperature, energy-stable rescale of v.
-// Here that is two launches around the force: k_md_first (one scale -- the
-// pending end-of-step factor times the chain's opening factor of step n --
-// then kick, drift and wrap) and k_md_thermostat (one workgroup: temperature
-// from the kinetic-energy partials that the force's assembly kernel wrote
-// with the closing half-kick, the end-of-step chain half or the
+// Here the force's first kernel opens the step (one scale -- the pending
+// end-of-step factor times the chain's opening factor of step n -- then kick,
+// drift and wrap), its assembly kernel closes it (half-kick, kinetic-energy
+// partials), and k_md_thermostat follows in the same captured graph (one
+// workgroup: temperature from the partials, the end-of-step chain half or the
 // energy-stable factor, left pending, and the opening half of step n + 1
-// computed ahead for the next k_md_first).  k_md_open opens the first step
+// computed ahead).  k_md_open opens the first step
 // of a run; k_md_apply applies the pending factor at its end; k_md_second
 // (kick = 0) gives the partials of the starting velocities.  All thermostat
 // scalars stay in device memory, so a run of many steps needs no host round
@@ -138,43 +138,6 @@ __global__ void k_md_open(MdParams p, const MdState* __restrict__ in,
   *out = st;
 }
 
-// Scale by the opened state's factor, half-kick, drift, wrap.  Workgroup 0
-// stores the opened state (scale applied) as the step's running state.
-template <typename R>
-__global__ __launch_bounds__(kMdBlock) void k_md_first(
-    MdArrays<R> a, MdParams p, const MdState* __restrict__ open,
-    MdState* __restrict__ out) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    MdState st = *open;
-    st.scale = 1.0;
-    *out = st;
-  }
-  const R f = (R)open->scale, dt = (R)p.dt, c = (R)p.ftm2v;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n;
-       i += gridDim.x * blockDim.x) {
-    const R m = (R)a.mass[a.type[i]];
-    R vx = a.vx[i], vy = a.vy[i], vz = a.vz[i];
-    if (f != (R)1) {
-      vx *= f;
-      vy *= f;
-      vz *= f;
-    }
-    vx = half_kick(vx, a.fx[i], m, dt, c);
-    vy = half_kick(vy, a.fy[i], m, dt, c);
-    vz = half_kick(vz, a.fz[i], m, dt, c);
-    a.vx[i] = vx;
-    a.vy[i] = vy;
-    a.vz[i] = vz;
-    R x = a.px[i] + vx * dt, y = a.py[i] + vy * dt, z = a.pz[i] + vz * dt;
-    wrap_flag(x, a.ix, i, (R)a.lo[0], (R)a.hi[0], (R)a.L[0]);
-    wrap_flag(y, a.iy, i, (R)a.lo[1], (R)a.hi[1], (R)a.L[1]);
-    wrap_flag(z, a.iz, i, (R)a.lo[2], (R)a.hi[2], (R)a.L[2]);
-    a.px[i] = x;
-    a.py[i] = y;
-    a.pz[i] = z;
-  }
-}
-
 template <typename R>
 __global__ __launch_bounds__(kMdBlock) void k_md_second(MdArrays<R> a, MdParams p,
                                                         int kick) {
@@ -204,16 +167,19 @@ __global__ __launch_bounds__(kMdBlock) void k_md_second(MdArrays<R> a, MdParams 
 
 __global__ __launch_bounds__(1024) void k_md_thermostat(
     MdParams p, const double* __restrict__ part, int nparts,
-    const double* __restrict__ thermo, const MdState* __restrict__ in,
-    MdState* __restrict__ out, MdState* __restrict__ open, int64_t step, int setup,
-    int with_pe) {
+    const double* __restrict__ thermo, const MdState* in, MdState* out, MdState* open,
+    int setup, int with_pe) {
   __shared__ double smem[16];
   double acc = 0.0;
   for (int q = threadIdx.x; q < nparts; q += blockDim.x) acc += part[q];
   double v[1] = {acc};
   block_sum<1>(v, smem);
   if (threadIdx.x != 0) return;
+  // (in may be open: the opened state of this step, whose scale the step's
+  // first kernel has applied)
   MdState st = *in;
+  st.scale = 1.0;
+  const int64_t step = setup ? 0 : st.step + 1;
   // temperature as SampleCurrentTemperatureState computes it
   // (nose_hoover_controller.cpp:256-287; energy_stable_scheme_controller.cpp:98-101)
   st.temp_sum = v[0] * p.mvv2e;
@@ -307,14 +273,6 @@ hipError_t md_launch_open(const MdParams& p, const MdState* in, MdState* out,
 }
 
 template <typename R>
-hipError_t md_launch_first(const MdArrays<R>& a, const MdParams& p,
-                           const MdState* open, MdState* out, hipStream_t s) {
-  hipLaunchKernelGGL((k_md_first<R>), dim3(md_blocks(a.n)), dim3(kMdBlock), 0, s,
-                     a, p, open, out);
-  return hipGetLastError();
-}
-
-template <typename R>
 hipError_t md_launch_second(const MdArrays<R>& a, const MdParams& p, int kick,
                             hipStream_t s) {
   hipLaunchKernelGGL((k_md_second<R>), dim3(md_blocks(a.n)), dim3(kMdBlock), 0, s,
@@ -326,10 +284,10 @@ int md_init_parts(int64_t n) { return md_blocks(n); }
 
 hipError_t md_launch_thermostat(const MdParams& p, const double* part, int nparts,
                                 const double* thermo, const MdState* in,
-                                MdState* out, MdState* open, int64_t step, int setup,
-                                int with_pe, hipStream_t s) {
+                                MdState* out, MdState* open, int setup, int with_pe,
+                                hipStream_t s) {
   hipLaunchKernelGGL(k_md_thermostat, dim3(1), dim3(1024), 0, s, p, part, nparts,
-                     thermo, in, out, open, step, setup, with_pe);
+                     thermo, in, out, open, setup, with_pe);
   return hipGetLastError();
 }
 
@@ -343,8 +301,6 @@ hipError_t md_launch_apply(const MdArrays<R>& a, const MdState* in, MdState* out
 
 #define RBMDX_MD_INST(R)                                                        \
   template hipError_t md_launch_wrap<R>(const MdArrays<R>&, hipStream_t);      \
-  template hipError_t md_launch_first<R>(const MdArrays<R>&, const MdParams&,  \
-                                         const MdState*, MdState*, hipStream_t); \
   template hipError_t md_launch_second<R>(const MdArrays<R>&, const MdParams&, \
                                           int, hipStream_t);                   \
   template hipError_t md_launch_apply<R>(const MdArrays<R>&, const MdState*,   \
