@@ -466,10 +466,23 @@ __global__ __launch_bounds__(256) void k_skin(Dev<R> d, Box<R> b, int force, int
 // in-cell order is made deterministic by k_cellsort.
 // Block `bid` of `nblk` binning blocks.
 template <typename R>
-__device__ __forceinline__ void bin_block(const Dev<R>& d, const Box<R>& b,
-                                          const Grid& g, int split, unsigned thr,
-                                          int nskin, int bid, int nblk) {
-  // rebuild decision, part 2: every block folds the skin-check maxima
+__device__ __forceinline__ int cell_key(const Dev<R>& d, const Box<R>& b, const Grid& g,
+                                        int split, int i) {
+  const R x = wrap<R>(d.px[i], b.lo[0], b.hi[0], b.L[0], b.invL[0]);
+  const R y = wrap<R>(d.py[i], b.lo[1], b.hi[1], b.L[1], b.invL[1]);
+  const R z = wrap<R>(d.pz[i], b.lo[2], b.hi[2], b.L[2], b.invL[2]);
+  const int cx = cell_coord((float)(x - b.lo[0]), g.scale[0], g.nc[0]);
+  const int cy = cell_coord((float)(y - b.lo[1]), g.scale[1], g.nc[1]);
+  const int cz = cell_coord((float)(z - b.lo[2]), g.scale[2], g.nc[2]);
+  const int cell = g.cell_of_coord[(cz * g.nc[1] + cy) * g.nc[0] + cx];
+  return 2 * cell + ((!split || d.charge[i] == R(0)) ? 1 : 0);
+}
+
+// The rebuild decision, part 2: a block of 256 threads folds the skin-check
+// maxima (every binning block for itself; `first` publishes the result).
+template <typename R>
+__device__ __forceinline__ bool rebuild_decision(const Dev<R>& d, unsigned thr, int nskin,
+                                                 bool first) {
   __shared__ float s_max[4];
   float m = 0.f;
   for (int k = threadIdx.x; k < nskin; k += blockDim.x)
@@ -478,22 +491,69 @@ __device__ __forceinline__ void bin_block(const Dev<R>& d, const Box<R>& b,
   if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-  if (bid == 0 && threadIdx.x == 0)
-    d.ctrl->maxdisp_bits = __float_as_uint(m);
-  if (!(__float_as_uint(m) > thr)) return;
+  if (first && threadIdx.x == 0) d.ctrl->maxdisp_bits = __float_as_uint(m);
+  return __float_as_uint(m) > thr;
+}
+
+template <typename R>
+__device__ __forceinline__ void bin_block(const Dev<R>& d, const Box<R>& b,
+                                          const Grid& g, int split, unsigned thr,
+                                          int nskin, int bid, int nblk) {
+  if (!rebuild_decision(d, thr, nskin, bid == 0)) return;
   for (int i = bid * blockDim.x + threadIdx.x; i < d.n; i += nblk * blockDim.x) {
-    const R x = wrap<R>(d.px[i], b.lo[0], b.hi[0], b.L[0], b.invL[0]);
-    const R y = wrap<R>(d.py[i], b.lo[1], b.hi[1], b.L[1], b.invL[1]);
-    const R z = wrap<R>(d.pz[i], b.lo[2], b.hi[2], b.L[2], b.invL[2]);
-    const int cx = cell_coord((float)(x - b.lo[0]), g.scale[0], g.nc[0]);
-    const int cy = cell_coord((float)(y - b.lo[1]), g.scale[1], g.nc[1]);
-    const int cz = cell_coord((float)(z - b.lo[2]), g.scale[2], g.nc[2]);
-    const int cell = g.cell_of_coord[(cz * g.nc[1] + cy) * g.nc[0] + cx];
-    const int neutral = (!split || d.charge[i] == R(0)) ? 1 : 0;
-    const int key = 2 * cell + neutral;
+    const int key = cell_key(d, b, g, split, i);
     d.key[i] = key;
     d.slot[i] = atomicAdd(&d.key_count[key], 1);
   }
+}
+
+// Binning, cell scans and sorted-order scatter of a small system (at most
+// kSmallAtoms atoms and kSmallKeys keys) in one block of 256 threads, the
+// counters in LDS.  Two launches fewer per evaluation, most of which do not
+// rebuild: 4,000 LJ atoms 47.2 -> 45.8 us per step,
+// 13,824 ions 86.5 -> 84.5.
+template <typename R>
+__device__ __forceinline__ void small_rebuild(const Dev<R>& d, const Box<R>& b, const Grid& g,
+                                              int split, unsigned thr, int nskin) {
+  __shared__ int cnt[kSmallKeys];
+  __shared__ int smem[33];
+  if (!rebuild_decision(d, thr, nskin, true)) return;
+  const int t = threadIdx.x, nt = blockDim.x, ncell = g.ncell;
+  for (int k = t; k < 2 * ncell; k += nt) cnt[k] = 0;
+  __syncthreads();
+#pragma unroll 4
+  for (int i = t; i < d.n; i += nt) {
+    const int key = cell_key(d, b, g, split, i);
+    d.key[i] = key;
+    d.slot[i] = atomicAdd(&cnt[key], 1);
+  }
+  __syncthreads();
+  const int per = (ncell + nt - 1) / nt;  // consecutive cells per thread
+  const int c0 = min(ncell, t * per), c1 = min(ncell, c0 + per);
+  int sa = 0, sq = 0;
+  for (int c = c0; c < c1; ++c) {
+    sa += cnt[2 * c] + cnt[2 * c + 1];
+    sq += cnt[2 * c];
+  }
+  int tot_a, tot_q;
+  int ra = block_excl_scan(sa, tot_a, smem);
+  int rq = block_excl_scan(sq, tot_q, smem);
+  for (int c = c0; c < c1; ++c) {
+    const int nq = cnt[2 * c], nn = cnt[2 * c + 1];
+    d.key_start[2 * c] = cnt[2 * c] = ra;
+    d.key_start[2 * c + 1] = cnt[2 * c + 1] = ra + nq;
+    d.cstart[c] = rq;
+    ra += nq + nn;
+    rq += nq;
+  }
+  if (t == 0) {
+    d.key_start[2 * ncell] = tot_a;
+    d.cstart[ncell] = tot_q;
+    d.ctrl->rebuild_count += 1;
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int i = t; i < d.n; i += nt) d.perm[cnt[d.key[i]] + d.slot[i]] = i;
 }
 
 // Exclusive scans in one block of 1024 threads: key_start over all 2 ncell
@@ -570,9 +630,8 @@ __device__ __forceinline__ void scatter_block(const Dev<R>& d, unsigned thr, int
 // special-bond rows (ms per atom).  A cell of at most 64 atoms is gathered in
 // one pass with the caller indices taken from the sort's registers.
 template <typename R>
-__global__ __launch_bounds__(256) void k_cellsort(Dev<R> d, Box<R> b,
-                                                  int ncell, unsigned thr,
-                                                  int ms) {
+__device__ __forceinline__ void cellsort_block(const Dev<R>& d, const Box<R>& b, int ncell,
+                                               unsigned thr, int ms) {
   if (!rebuild_now(d.ctrl, thr)) return;
   int* perm = d.perm;
   const int* key_start = d.key_start;
@@ -2167,8 +2226,8 @@ __device__ __forceinline__ void sk2_block(const Dev<R>& d, const Box<R>& b,
 }
 
 // FP64 reduction of the S(k) chunk partials of the kSkK k's of k tile
-// `tile` (16 threads per k, each a contiguous run of chunks, then the 16 in
-// order; the kernel boundary after the S(k) blocks makes every partial
+// `tile` (block / kSkK threads per k, each a contiguous run of chunks, then
+// these in order; the kernel boundary after the S(k) blocks makes every partial
 // visible) into rho_k and the per-k force coefficients
 //   A_k = w_k (-4 pi qqr2e) / (V k^2),  kf0 = (m, A Re rho), kf1 = (k, A Im rho),
 // and each k's terms of the k-space energy and virial (without the self
@@ -2183,7 +2242,7 @@ __device__ __forceinline__ void skfin2_block(const Dev<R>& d, const Box<R>& b,
                                              const int* __restrict__ m, int K, int nchunks,
                                              const Params& p, int vmode, int tile,
                                              char* buf) {
-  constexpr int kSub = 16;  // threads per k (blockDim = kSkK * kSub)
+  const int kSub = (int)blockDim.x / kSkK;  // threads per k
   // buf: LDS of kSub * 2 * kSkK doubles
   auto s_s = reinterpret_cast<double (*)[2][kSkK]>(buf);
   const int t = (int)threadIdx.x;
@@ -2321,6 +2380,38 @@ struct KsArgs {
   int rbe_ash = 6;
   Params p;
 };
+
+// The cell sort; in a small system the blocks after its ncb ones reduce the
+// S(k) partials, one k tile each.
+template <typename R>
+__global__ __launch_bounds__(256) void k_cellsort(Dev<R> d, Box<R> b, int ncell, unsigned thr,
+                                                  int ms) {
+  cellsort_block<R>(d, b, ncell, thr, ms);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_cellsort_fin(Dev<R> d, Box<R> b, int ncell,
+                                                      unsigned thr, int ms, int ncb,
+                                                      KsArgs ks) {
+  __shared__ __align__(16) char buf[(size_t)(kBlock / kSkK) * 2 * kSkK * sizeof(double)];
+  if ((int)blockIdx.x < ncb)
+    cellsort_block<R>(d, b, ncell, thr, ms);
+  else
+    skfin2_block<R>(d, b, ks.m_fin, ks.K, ks.nchunks, ks.p, ks.vmode, (int)blockIdx.x - ncb,
+                    buf);
+}
+
+// A small system's rebuild up to the cell sort (block 0) and the S(k)
+// partials (the blocks after).
+template <typename R>
+__global__ __launch_bounds__(256) void k_small_sk(Dev<R> d, Box<R> b, Grid g, int split,
+                                                  unsigned thr, int nskin, KsArgs ks) {
+  if (blockIdx.x == 0) {
+    small_rebuild<R>(d, b, g, split, thr, nskin);
+    return;
+  }
+  const int q = (int)blockIdx.x - 1;
+  sk2_block<R>(d, b, ks.m_arg, ks.from_ring, ks.K, q % ks.nchunks, q / ks.nchunks);
+}
 
 // Binning (blocks [0, nbin)) and the S(k) partials (the blocks after).
 template <typename R>
@@ -2568,14 +2659,22 @@ hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
   const int cap_a = a.count_only ? 0 : d.cap_a;
   const int cap_b = a.count_only ? 0 : d.cap_b;
   const bool kon = ks.K > 0;
-  hipLaunchKernelGGL((k_bin_sk<R>), dim3(gb + (kon ? ks.nchunks * ks.ntiles : 0)),
-                     dim3(kBlock), 0, s, d, a.box, g, a.p.split, thr, nskin, gb, ks);
-  hipLaunchKernelGGL((k_scan_fin<R>), dim3(kon ? 1 + ks.ntiles : 1), dim3(1024), 0, s,
-                     d, a.box,
-                     g.ncell, thr, ks);
-  hipLaunchKernelGGL((k_scatter<R>), dim3(gb), dim3(kBlock), 0, s, d, thr);
-  hipLaunchKernelGGL((k_cellsort<R>), dim3(blocks_for(g.ncell * 64, kBlock)),
-                     dim3(kBlock), 0, s, d, a.box, g.ncell, thr, a.pc.ms);
+  const int nsk = kon ? ks.nchunks * ks.ntiles : 0, nfin = kon ? ks.ntiles : 0;
+  const int ncb = blocks_for(g.ncell * 64, kBlock);
+  if (d.n <= kSmallAtoms && 2 * g.ncell <= kSmallKeys) {
+    hipLaunchKernelGGL((k_small_sk<R>), dim3(1 + nsk), dim3(kBlock), 0, s, d, a.box, g,
+                       a.p.split, thr, nskin, ks);
+    hipLaunchKernelGGL((k_cellsort_fin<R>), dim3(ncb + nfin), dim3(kBlock), 0, s, d, a.box,
+                       g.ncell, thr, a.pc.ms, ncb, ks);
+  } else {
+    hipLaunchKernelGGL((k_bin_sk<R>), dim3(gb + nsk), dim3(kBlock), 0, s, d, a.box, g,
+                       a.p.split, thr, nskin, gb, ks);
+    hipLaunchKernelGGL((k_scan_fin<R>), dim3(1 + nfin), dim3(1024), 0, s, d, a.box, g.ncell,
+                       thr, ks);
+    hipLaunchKernelGGL((k_scatter<R>), dim3(gb), dim3(kBlock), 0, s, d, thr);
+    hipLaunchKernelGGL((k_cellsort<R>), dim3(ncb), dim3(kBlock), 0, s, d, a.box, g.ncell, thr,
+                       a.pc.ms);
+  }
   const bool dense = a.p.split && d.nc > 0 && g.qblocks;
   hipLaunchKernelGGL((k_lists<R>), dim3(g.nbrick + (dense ? 0 : list_b_grid(a.p, d.nc, g))),
                      dim3(g.block), 0, s, d, a.box, g, a.pc.r2_list_a,
