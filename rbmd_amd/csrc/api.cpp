@@ -1370,6 +1370,7 @@ class Engine : public EngineBase {
         HIPCHK(hipMemcpy(d_.qcall, qc.data(), sizeof(int) * nc, hipMemcpyHostToDevice));
     }
     d_.cnt_a = alloc<int>(n_);
+    HIPCHK(hipMemset(d_.cnt_a, 0, sizeof(int) * n_));  // (list A may never be built)
     d_.order_a = alloc<int>(n_);
     d_.cnt_b = alloc<int>(nc);
     d_.inv_mass = alloc<R>(ntypes_);

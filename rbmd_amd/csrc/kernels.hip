@@ -2650,6 +2650,13 @@ int list_b_grid(const Params& p, int nc, const Grid& g) {
   return (p.split && nc > 0) ? list_b_count(g, nc) : 0;
 }
 
+// Whether list A can hold pairs.  With every atom charged (water, molten
+// salts) every pair is list B's: neither the list-A build (24 us per rebuild of
+// 72,981 atoms) nor the brick pair kernel is launched; the rows' counts stay 0.
+bool list_a_used(const Params& p, int n, int nc, const Grid& g) {
+  return !(p.split && nc == n && g.qblocks > 0);
+}
+
 template <typename R>
 hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
                       hipStream_t s, const KsArgs& ks = KsArgs()) {
@@ -2676,9 +2683,10 @@ hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
                        a.pc.ms);
   }
   const bool dense = a.p.split && d.nc > 0 && g.qblocks;
-  hipLaunchKernelGGL((k_lists<R>), dim3(g.nbrick + (dense ? 0 : list_b_grid(a.p, d.nc, g))),
-                     dim3(g.block), 0, s, d, a.box, g, a.pc.r2_list_a,
-                     a.pc.r2_list_b, a.p.split, cap_a, cap_b, thr);
+  if (list_a_used(a.p, d.n, d.nc, g))
+    hipLaunchKernelGGL((k_lists<R>), dim3(g.nbrick + (dense ? 0 : list_b_grid(a.p, d.nc, g))),
+                       dim3(g.block), 0, s, d, a.box, g, a.pc.r2_list_a,
+                       a.pc.r2_list_b, a.p.split, cap_a, cap_b, thr);
   if (dense)
     hipLaunchKernelGGL((k_lists_dense<R>), dim3(g.ncell * g.dsplit), dim3(kDenseBlock), 0, s,
                        d, a.box, g,
@@ -2697,7 +2705,7 @@ hipError_t launch_build(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   // list statistics only (no pair partials)
   RedArgs ra;
   ra.lista_part = d.lista_part;
-  ra.nlista = a.grid.nbrick;
+  ra.nlista = list_a_used(a.p, d.n, d.nc, a.grid) ? a.grid.nbrick : 0;
   ra.listb_part = d.listb_part;
   ra.nlistb = list_b_grid(a.p, d.nc, a.grid);
   ra.ctrl = d.ctrl;
@@ -2765,9 +2773,7 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
                      a.lj_tab, p.split)
   // list A holds RBL shell pairs only when the LJ cutoff exceeds r_core
   const bool shell_a = a.pc.rclj2 > a.pc.rs2;
-  // every atom charged (water, molten salts): list A is empty and every pair
-  // is k_pair_b's, so the brick kernel is not launched at all
-  const bool has_a = !(p.split && d.nc == d.n && g.qblocks > 0);
+  const bool has_a = list_a_used(p, d.n, d.nc, g);
   if (!has_a) {
     // nothing: k_assemble reads no list-A force
   } else if (p.special) {
@@ -2855,7 +2861,7 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   ra.thermo = d.thermo;
   ra.mean = d.mean;
   ra.lista_part = d.lista_part;
-  ra.nlista = g.nbrick;
+  ra.nlista = has_a ? g.nbrick : 0;
   ra.listb_part = d.listb_part;
   ra.nlistb = list_b_grid(p, d.nc, g);
   ra.ctrl = d.ctrl;
