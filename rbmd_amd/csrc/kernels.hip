@@ -653,9 +653,8 @@ __device__ __forceinline__ void scatter_block(const Dev<R>& d, unsigned thr, int
     d.perm[d.key_start[d.key[i]] + d.slot[i]] = i;
 }
 
-// One wave per cell: both key segments are sorted by caller index (bitonic
-// across the wave up to 64 atoms, a rank sort up to 512, serial by lane 0
-// beyond), then the cell's atoms are gathered into the sorted tiles:
+// One wave per cell: both key segments are sorted by caller index (by rank up
+// to 512 atoms, from the lanes' registers, serial by lane 0 beyond), then the cell's atoms are gathered into the sorted tiles:
 // positions (and the charged copy), reference positions for the skin check,
 // sorted ids, RBL hashes and cells, the charged map, inv_perm, and the CVFF
 // special-bond rows (ms per atom).  A cell of at most 64 atoms is gathered in
@@ -667,7 +666,8 @@ __device__ __forceinline__ void cellsort_block(const Dev<R>& d, const Box<R>& b,
   int* perm = d.perm;
   const int* key_start = d.key_start;
   const int lane = threadIdx.x & 63;
-  const int cell = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int cell =
+      __builtin_amdgcn_readfirstlane((int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   if (cell >= ncell) return;
   // the key starts (charged segment, neutral segment, end) and, for segments
   // of at most 64 atoms, the sorted caller indices in lane order
@@ -682,13 +682,12 @@ __device__ __forceinline__ void cellsort_block(const Dev<R>& d, const Box<R>& b,
     if (len <= 64) {
       int v = lane < len ? perm[a + lane] : 0x7fffffff;
       if (len > 1) {
-        for (int k = 2; k <= 64; k <<= 1)
-          for (int j = k >> 1; j > 0; j >>= 1) {
-            const int p = __shfl_xor(v, j, 64);
-            const bool up = (lane & k) == 0;
-            const bool lower = (lane & j) == 0;
-            v = (lower == up) ? min(v, p) : max(v, p);
-          }
+        // rank among the segment's values (lanes past it stay in place), then
+        // each value to the lane of its rank
+        int r = lane < len ? 0 : lane;
+        for (int l = 0; l < len; ++l)
+          r += __builtin_amdgcn_readlane(v, l) < v && lane < len ? 1 : 0;
+        v = __builtin_amdgcn_ds_permute(4 * r, v);
         if (lane < len) perm[a + lane] = v;
       }
       sv[seg] = v;
@@ -795,6 +794,11 @@ __device__ __forceinline__ bool charged_w(R w) {
   return w != (R)(int)w;
 }
 
+// The word that holds a value's sign bit.
+__device__ __forceinline__ unsigned sign_word(float x) { return __float_as_uint(x); }
+__device__ __forceinline__ unsigned sign_word(double x) { return (unsigned)__double2hiint(x); }
+constexpr int kStagePad = 8;  // stage entries the unrolled tests may read past a row
+
 // All-atom candidate list of one brick: every j != i within r2 among the 27
 // cells around i, except charged-charged pairs when the work is split (those
 // go to list B).  Entries are 16-bit positions in the brick's staged
@@ -836,8 +840,8 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
       wo += (count & 7) ? 1 : n8 - 7;
     };
     // Staged neighbourhoods scan a stencil row (its x cells are consecutive
-    // slots, hence one contiguous stage range) as one run, 4 candidates at a
-    // time; the charged atoms of each cell are skipped for a charged i.
+    // slots, hence one contiguous stage range) as one run; the charged atoms of
+    // each cell are skipped for a charged i.
     const bool rows = STAGED && st.mode[0] != 1;
     const int runlen = rows ? st.n[0] : 1;
     const int nrow = st.n[2] * st.n[1];
@@ -850,41 +854,42 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
           const int s0 = srow + st.at(0, kx);
           const int l0 = t.off[s0], l1 = t.off[s0 + runlen];
           if (STAGED) {
-            // chunks of up to 64 candidates: first the accept mask (no
-            // branches; candidate cb + 4k + u sets bit 4k + u), then the
-            // accepted entries in candidate order
-            for (int cb = l0; cb < l1; cb += 64) {
-              const int ce = min(l1, cb + 64), nk = ce - cb;
-              unsigned long long ok = 0;
+            // chunks of up to 32 candidates: first the accept mask, without
+            // branches (the sign of d^2 - r^2 shifted in, candidate u at bit
+            // 31 - u), then the accepted entries in candidate order.  The
+            // loads may run past the row (the stage has padding).
+            for (int cb = l0; __any(cb < l1); cb += 32) {
+              const int nk = min(max(l1 - cb, 0), 32);
+              unsigned ok = 0;
 #pragma unroll
-              for (int k = 0; k < 16; ++k) {
-                const int l = cb + 4 * k;
-                if (l >= ce) continue;
-                R4T<R> xj[4];
+              for (int k = 0; k < 4; ++k) {
+                if (!__any(8 * k < nk)) {
+                  ok <<= 8;
+                  continue;
+                }
+                // a lane whose row is over reads the stage's start
+                const R4T<R>* xp = stage + (8 * k < nk ? cb + 8 * k : 0);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) xj[u] = stage[min(l + u, ce - 1)];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < 8; ++u) {
                   R dx, dy, dz;
-                  const R d2 = pair_d2<R, MI>(b, xi.x, xi.y, xi.z, xj[u].x, xj[u].y,
-                                              xj[u].z, dx, dy, dz);
+                  const R d2 = pair_d2<R, MI>(b, xi.x, xi.y, xi.z, xp[u].x, xp[u].y,
+                                              xp[u].z, dx, dy, dz);
                   // charged-charged pairs belong to list B: the stage's .w
                   // (1e30 for a charged j) pushes them past the cutoff
-                  ok |= (unsigned long long)(fma_r(qf, xj[u].w, d2) < r2) << (4 * k + u);
+                  ok = __builtin_amdgcn_alignbit(ok, sign_word(fma_r(qf, xp[u].w, d2) - r2), 31);
                 }
               }
-              // the bits past the chunk's end (their loads repeat its last
-              // candidate) and i itself are not entries
-              if (nk < 64) ok &= (1ull << nk) - 1ull;
+              // neither the bits past the chunk's end nor i itself are entries
+              ok &= (unsigned)(0xffffffff00000000ull >> nk);
               const int so = self - cb;
-              if (so >= 0 && so < nk) ok &= ~(1ull << so);
+              if ((unsigned)so < 32u) ok &= ~(0x80000000u >> so);
               if (count_pass) {
-                count += __popcll(ok);
+                count += __popc(ok);
                 continue;
               }
               while (ok) {
-                const int u = __builtin_ctzll(ok);
-                ok &= ok - 1;
+                const int u = __clz((int)ok);
+                ok &= ~(0x80000000u >> u);
                 accept(cb + u);
               }
             }
@@ -937,7 +942,7 @@ template <typename R>
 __device__ __forceinline__ void list_a_brick(const Dev<R>& d, const Box<R>& b,
                                              const Grid& g, int brick, R r2,
                                              int split, int cap) {
-  __shared__ R4T<R> stage[StageCap<R>::value];
+  __shared__ R4T<R> stage[StageCap<R>::value + kStagePad];
   __shared__ SlotTables<kMaxSlots> t;
   const int e1[3] = {1, 1, 1};
   const Neigh h = brick_neigh(g, brick, e1);
@@ -994,31 +999,23 @@ __device__ __forceinline__ void list_a_brick(const Dev<R>& d, const Box<R>& b,
   if (na <= kOrderMax) {
     __threadfence_block();  // this block's counts are read back below
     __syncthreads();
-    // keys (longer list first, then position) in a bitonic sort over the next
-    // power of two, padded with the largest key
-    int np = 1;
-    while (np < na) np <<= 1;
+    // each key's rank (longer list first, then position) among all keys, four
+    // at a time; a bitonic sort takes 28-45 passes with a barrier each
+    const int np = (na + 3) & ~3;
     for (int k = threadIdx.x; k < np; k += blockDim.x)
       s_key[k] = k < na ? ((unsigned)(0xffff - min(d.cnt_a[i0 + k], 0xffff)) << 16) |
                               (unsigned)k
                         : 0xffffffffu;
     __syncthreads();
-    for (int kk = 2; kk <= np; kk <<= 1)
-      for (int j = kk >> 1; j > 0; j >>= 1) {
-        for (int t = threadIdx.x; t < np; t += blockDim.x) {
-          const int u = t ^ j;
-          if (u > t) {
-            const unsigned x = s_key[t], y = s_key[u];
-            if ((x > y) == ((t & kk) == 0)) {
-              s_key[t] = y;
-              s_key[u] = x;
-            }
-          }
-        }
-        __syncthreads();
+    for (int k = threadIdx.x; k < na; k += blockDim.x) {
+      const unsigned key = s_key[k];
+      int r = 0;
+      for (int q = 0; q < np; q += 4) {
+        const uint4 o = *reinterpret_cast<const uint4*>(s_key + q);
+        r += (o.x < key) + (o.y < key) + (o.z < key) + (o.w < key);
       }
-    for (int k = threadIdx.x; k < na; k += blockDim.x)
-      d.order_a[i0 + k] = i0 + (int)(s_key[k] & 0xffffu);
+      d.order_a[i0 + r] = i0 + k;
+    }
   } else {
     for (int k = threadIdx.x; k < na; k += blockDim.x) d.order_a[i0 + k] = i0 + k;
   }
