@@ -1185,13 +1185,19 @@ class Engine : public EngineBase {
       grid_.vblock = threads(per * (1 << grid_.vsh), 256);
       // mostly charged systems put nearly all pairs in list B: kernels of
       // their own take them, one wave per charged atom, with one resident
-      // round of 5 waves per SIMD (contiguous runs of atoms per wave)
+      // round (contiguous runs of atoms per wave): the FP32 force pass runs 6
+      // waves per SIMD, with energies 4 (9,000 water atoms: 144 us per evaluation
+      // with 1,024 blocks, 148 with 1,280, a quarter of them in a second round)
       grid_.psub = 1;
-      grid_.qblocks = 0;
+      grid_.qblocks = grid_.qblocks_e = 0;
       grid_.dsplit = 1;
       if (split_ && 2 * (long)nc > (long)n_) {
-        grid_.qblocks = std::max(1, std::min((nc + kQWaves - 1) / kQWaves,
-                                             num_cu_ * 4 * 5 / kQWaves));
+        auto round = [&](int waves) {
+          return std::max(1, std::min((nc + kQWaves - 1) / kQWaves,
+                                      num_cu_ * 4 * waves / kQWaves));
+        };
+        grid_.qblocks = round(sizeof(R) == 4 ? 6 : 5);
+        grid_.qblocks_e = round(sizeof(R) == 4 ? 4 : 5);
         // the list build's groups of 64 charged atoms per cell, with margin
         // for cells above the mean
         const double qpc = (double)nc / grid_.ncell;

@@ -98,6 +98,7 @@ struct Grid {
   // blocks of the dense charged-pair kernel (one wave per charged atom) that
   // takes list B in mostly charged systems; 0: list B inside the pair kernel
   int qblocks = 0;
+  int qblocks_e = 0;  // the same with energies
   // blocks per cell of the dense charged-pair list build (64 charged atoms
   // of the cell per block and pass)
   int dsplit = 1;
@@ -105,6 +106,9 @@ struct Grid {
   const int* coord_of_cell = nullptr;  // [ncell] cell id -> packed x|y<<10|z<<20
   const int* brick_cell0 = nullptr;    // [nbrick+1] first cell id of a brick
 };
+
+// Blocks of the dense charged-pair kernel of an evaluation.
+inline int q_grid(const Grid& g, int eflag) { return eflag ? g.qblocks_e : g.qblocks; }
 
 // Blocks of the charged-pair list build: dsplit per cell in mostly charged
 // systems, else kChargedLanes lanes per charged atom.
@@ -298,7 +302,7 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s);
 // per-evaluation partial results (reduction partials, S(k) chunk partials,
 // per-k coefficients) that a context otherwise allocates.  Every call on one
 // device shares the device's copy.
-constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
+constexpr size_t kNoAllocScratchBytes = ((size_t)16 << 20) + ((size_t)128 << 10);
 // Resolves the array's address on `device`, which must be the current
 // device; the first call per device does the lookup, later calls keep it.
 hipError_t noalloc_scratch_init(int device);

@@ -1786,7 +1786,10 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
 // a fixed tree over the wave; block partials of the thermo sums in `part`
 // (k_reduce's second segment).  Each wave takes a contiguous run of atoms,
 // and the runs of one XCD are contiguous, so an XCD's L2 holds one region's
-// neighbours.
+// neighbours.  Bound by the latency of the gathers (TD busy 89 %, VALU 77 %):
+// 72,981 water atoms take 295, 238, 222 and 208 us with 2.5, 4, 5 and 6 waves per
+// SIMD, and 236 with 8, where registers spill; so the force pass is held to 80
+// registers (6 waves) and the grid to one resident round.
 // ---------------------------------------------------------------------------
 constexpr int kQBatch = 3;  // list steps of 64 entries per load batch
 constexpr int kRing = 256;  // ring entries per wave (>= 63 + 64 * kQBatch)
@@ -1794,7 +1797,7 @@ static_assert(kRing >= 63 + 64 * kQBatch && (kRing & (kRing - 1)) == 0, "ring si
 
 template <typename R, bool RBL, bool EFLAG, bool SPECIAL>
 __global__ __launch_bounds__(64 * kQWaves)
-__attribute__((amdgpu_waves_per_eu(4))) void k_pair_b(Dev<R> d, Box<R> b, Grid g,
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !EFLAG ? 6 : 4))) void k_pair_b(Dev<R> d, Box<R> b, Grid g,
                                                       PairConst<R> pc_arg,
                                                       const R* lj_tab, double* part) {
   PairConst<R> pc = pc_arg;
@@ -2827,7 +2830,7 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
 #undef RBMDX_PAIR
   if (g.qblocks > 0) {
 #define RBMDX_PAIRB(RBLv, EFv, SPv)                                             \
-  hipLaunchKernelGGL((k_pair_b<R, RBLv, EFv, SPv>), dim3(g.qblocks),           \
+  hipLaunchKernelGGL((k_pair_b<R, RBLv, EFv, SPv>), dim3(q_grid(g, p.eflag)),  \
                      dim3(64 * kQWaves), lj_bytes, s, d, a.box, g, a.pc, a.lj_tab, \
                      d.pairb_part)
     if (p.special) {
@@ -2871,7 +2874,7 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   ra.pair_part = d.pair_part;
   ra.npair = has_a ? g.nbrick * g.psub : 0;
   ra.part2 = d.pairb_part;
-  ra.npair2 = g.qblocks;
+  ra.npair2 = q_grid(g, p.eflag);
   ra.eflag = p.eflag ? 1 : 0;
   ra.mean_fix = p.mean_fix;
   ra.n_global = p.n_global;
