@@ -187,6 +187,13 @@ int rbmdx_set_system(rbmdx_ctx* ctx, int64_t n, const double* box_lo,
 /* Replace the charges (host array, n entries); keeps lists. */
 int rbmdx_set_charges(rbmdx_ctx* ctx, const double* charge);
 
+/* rbmdx_set_charges (every atom the charge of its type) and rbmdx_set_lj in
+ * one call ordered on `stream`, without waiting for the device: charge, eps
+ * and sigma hold one value per type.  The evaluations that follow run on the
+ * same stream. */
+int rbmdx_set_type_params(rbmdx_ctx* ctx, const double* charge, const double* eps,
+                          const double* sigma, void* stream);
+
 /* Replace the per-type LJ parameters (host arrays, ntypes entries); keeps
  * lists.  Synchronises the device. */
 int rbmdx_set_lj(rbmdx_ctx* ctx, const double* eps, const double* sigma);

@@ -125,6 +125,7 @@ SIGNATURES = {
     "rbmdx_set_charges": (ctypes.c_int, [_P, _DP]),
     "rbmdx_set_special": (ctypes.c_int, [_P, _I32, _IP, _IP]),
     "rbmdx_set_lj": (ctypes.c_int, [_P, _DP, _DP]),
+    "rbmdx_set_type_params": (ctypes.c_int, [_P, _DP, _DP, _DP, _P]),
     "rbmdx_force_vjp": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                                        ctypes.c_uint32, _P]),
     "rbmdx_force": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _P, _P, _P, _I32,
@@ -392,6 +393,13 @@ class ForceContext:
         e = np.ascontiguousarray(eps, dtype=np.float64)
         s = np.ascontiguousarray(sigma, dtype=np.float64)
         self._check(self.lib.rbmdx_set_lj(self._h, _dptr(e), _dptr(s)))
+
+    def set_type_params(self, charges, eps, sigma, stream):
+        """Charge, eps and sigma per type (set_charges of charges[type] and
+        set_lj) ordered on the stream of the evaluations, without a wait."""
+        q, e, s = (np.ascontiguousarray(a, dtype=np.float64) for a in (charges, eps, sigma))
+        self._check(self.lib.rbmdx_set_type_params(self._h, _dptr(q), _dptr(e), _dptr(s),
+                                                   ctypes.c_void_p(stream)))
 
     def force_vjp(self, step, px, py, pz, gx, gy, gz, dx, dy, dz, dparam, sync=False,
                   neutral_q=False, stream=None):

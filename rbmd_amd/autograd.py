@@ -18,36 +18,36 @@ pass must run before the next forward evaluation of the same context.
 import numpy as np
 import torch
 
-from . import ForceContext
+from . import ForceContext, _current_stream
 
 
 class _ForceFn(torch.autograd.Function):
     @staticmethod
     def forward(fctx, pos, Q, eps, sigma, model, step, m_samples, num_k):
-        model._apply(Q, eps, sigma)
-        pos = pos.contiguous()
-        px, py, pz = (pos[:, d].contiguous() for d in range(3))
-        f = [torch.empty_like(px) for _ in range(3)]
-        model.ctx.force(step, px, py, pz, *f, m_samples=m_samples, num_k=num_k)
-        fctx.save_for_backward(px, py, pz)
+        model._apply(Q, eps, sigma, pos.device)
+        # one transposing copy each way; the rows are the SoA arrays
+        x = pos.t().contiguous()
+        f = torch.empty_like(x)
+        model.ctx.force(step, *x.unbind()[:3], *f.unbind()[:3], m_samples=m_samples,
+                        num_k=num_k)
+        fctx.save_for_backward(x)
         fctx.model = model
         fctx.step = step
         fctx.pdev = (Q.device, eps.device, sigma.device)
         fctx.pdtype = (Q.dtype, eps.dtype, sigma.dtype)
-        return torch.stack(f, dim=1)
+        return f[:3].t().contiguous()
 
     @staticmethod
     def backward(fctx, gF):
-        px, py, pz = fctx.saved_tensors
+        x, = fctx.saved_tensors
         model = fctx.model
-        gF = gF.contiguous().to(px.dtype)
-        gx, gy, gz = (gF[:, d].contiguous() for d in range(3))
-        d = [torch.empty_like(px) for _ in range(3)]
+        g = gF.to(x.dtype).t().contiguous()
+        d = torch.empty_like(g)
         nt = model.ntypes
-        dparam = torch.empty(3 * nt, dtype=torch.float64, device=px.device)
-        model.ctx.force_vjp(fctx.step, px, py, pz, gx, gy, gz, *d, dparam,
+        dparam = torch.empty(3 * nt, dtype=torch.float64, device=x.device)
+        model.ctx.force_vjp(fctx.step, *x.unbind()[:3], *g.unbind(), *d.unbind(), dparam,
                             neutral_q=model.neutral_charge_grad)
-        dpos = torch.stack(d, dim=1).to(gF.dtype)
+        dpos = d.t().contiguous()
         grads = [dparam[k * nt:(k + 1) * nt].to(device=dev, dtype=dt)
                  for k, (dev, dt) in enumerate(zip(fctx.pdev, fctx.pdtype))]
         return (dpos, *grads, None, None, None, None)
@@ -71,20 +71,27 @@ class DifferentiableForce:
                             system.charges, system.eps, system.sigma)
         self._state = None
 
-    def _apply(self, Q, eps, sigma):
-        q = np.asarray(Q.detach().cpu(), dtype=np.float64)
-        e = np.asarray(eps.detach().cpu(), dtype=np.float64)
-        s = np.asarray(sigma.detach().cpu(), dtype=np.float64)
-        if self._state is not None:
-            q0, e0, s0 = self._state
-            same_q = np.array_equal(q, q0)
-            same_lj = np.array_equal(e, e0) and np.array_equal(s, s0)
+    def _apply(self, Q, eps, sigma, device):
+        par = [t.detach() for t in (Q, eps, sigma)]
+        if all(t.is_cuda and t.device == Q.device for t in par):
+            # one copy to the host (each waits for the device)
+            flat = torch.cat([t.reshape(-1).to(torch.float64) for t in par]).cpu().numpy()
+            n = [t.numel() for t in par]
+            q, e, s = (a.reshape(t.shape) for a, t in
+                       zip(np.split(flat, [n[0], n[0] + n[1]]), par))
         else:
-            same_q = same_lj = False
-        if not same_q:
-            self.ctx.set_charges(q[self.types])
-        if not same_lj:
-            self.ctx.set_lj(e, s)
+            q, e, s = (np.asarray(t.cpu(), dtype=np.float64) for t in par)
+        same_q = self._state is not None and np.array_equal(q, self._state[0])
+        same_lj = (self._state is not None and np.array_equal(e, self._state[1])
+                   and np.array_equal(s, self._state[2]))
+        if not (same_q and same_lj):
+            if q.shape == e.shape == s.shape == (self.ntypes,):
+                self.ctx.set_type_params(q, e, s, _current_stream(device))
+            else:
+                if not same_q:
+                    self.ctx.set_charges(q[self.types])
+                if not same_lj:
+                    self.ctx.set_lj(e, s)
         self._state = (q, e, s)
 
     def __call__(self, pos, Q, eps, sigma, step=0, m_samples=None, num_k=None):

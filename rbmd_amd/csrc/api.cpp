@@ -73,6 +73,8 @@ struct EngineBase {
                                const void* pz, int candidates, int32_t* gi,
                                int32_t* gj, int32_t* cls, int64_t cap) = 0;
   virtual void set_charges(const double* q) = 0;
+  virtual void set_type_params(const double* q, const double* eps, const double* sig,
+                               hipStream_t s) = 0;
   virtual void set_special(int32_t ms, const int32_t* nspecial,
                            const int32_t* special) = 0;
   virtual int kernel_times(const char** names, double* usec, int n) = 0;
@@ -160,6 +162,40 @@ class Engine : public EngineBase {
     upload_charges();
     charge_sums();
     hipDeviceSynchronize();
+  }
+
+  // The charge of every atom as its type's, with the types' LJ parameters
+  // (set_charges and set_lj of one training step): a kernel on the evaluations'
+  // stream, so that neither the host nor the device waits.  With split charges
+  // a type stays charged or neutral as its atoms are.
+  void set_type_params(const double* q, const double* eps, const double* sig,
+                       hipStream_t s) override {
+    if (!ready_) throw Error(RBMDX_E_STATE, "set_system first");
+    if (!q || !eps || !sig) throw Error(RBMDX_E_ARG, "null type parameters");
+    if (split_)
+      for (int t = 0; t < ntypes_; ++t)
+        if (type_atoms_[t] && type_part_[t] != ((R)q[t] != R(0) ? 1 : 2))
+          throw Error(RBMDX_E_ARG,
+                      "set_charges may not change which atoms are charged");
+    HIPCHK(hipSetDevice(device_));
+    // evaluations in flight on another stream read the current values
+    if (last_stream_set_ && last_stream_ != s) HIPCHK(hipDeviceSynchronize());
+    eps_.assign(eps, eps + ntypes_);
+    sig_.assign(sig, sig + ntypes_);
+    TypeParams tp;
+    sum_q_ = sum_q2_ = 0;
+    for (int t = 0; t < ntypes_; ++t) {
+      tp.q[t] = q[t];
+      tp.eps[t] = eps[t];
+      tp.sig[t] = sig[t];
+      sum_q_ += (double)type_atoms_[t] * q[t];
+      sum_q2_ += (double)type_atoms_[t] * (q[t] * q[t]);
+    }
+    // (with split charges the host copy serves only to tell them from neutral)
+    if (!split_)
+      for (int i = 0; i < n_; ++i) q_[i] = q[type_[i]];
+    HIPCHK(launch_type_params<R>(tp, ntypes_, d_.type, d_.charge, n_, lj_tab_, s));
+    self_energy();
   }
 
   // CVFF special-bond topology (DeviceData d_nspecial / d_special /
@@ -962,6 +998,7 @@ class Engine : public EngineBase {
   double lo_[3], L_[3];
   std::vector<int32_t> type_, id_;
   std::vector<double> q_, eps_, sig_;
+  std::vector<int> type_atoms_, type_part_;
   bool split_ = false;
   int kspace_ = 0;  // 0 none, 1 RBE, 2 EWALD
   double alpha_ = 0, rbe_S_ = 0, sum_q_ = 0, sum_q2_ = 0, e_self_ = 0;
@@ -1055,6 +1092,10 @@ class Engine : public EngineBase {
       sum_q_ += v;
       sum_q2_ += v * v;
     }
+    self_energy();
+  }
+
+  void self_energy() {
     params_.sum_q = sum_q_;
     params_.sum_q2 = sum_q2_;
     const double V = L_[0] * L_[1] * L_[2];
@@ -1085,6 +1126,13 @@ class Engine : public EngineBase {
       for (double v : q_) nc += (R)v != R(0);
     split_ = coulomb && nc > 0;
     if (!split_) nc = 0;
+    // per type: its atoms, and whether they are charged (bit 0) or neutral (1)
+    type_atoms_.assign(ntypes_, 0);
+    type_part_.assign(ntypes_, 0);
+    for (int i = 0; i < n_; ++i) {
+      ++type_atoms_[type_[i]];
+      type_part_[type_[i]] |= (R)q_[i] != R(0) ? 1 : 2;
+    }
     const double V = L_[0] * L_[1] * L_[2];
     charge_sums();
     // alpha: manual override wins, else DeriveAlphaFromAccuracy
@@ -1840,6 +1888,14 @@ int rbmdx_force_vjp(rbmdx_ctx* ctx, int64_t step, const void* px, const void* py
   return guarded(ctx, [&] {
     ctx->eng->force_vjp(step, px, py, pz, gx, gy, gz, dx, dy, dz, dparam, flags,
                         (hipStream_t)stream);
+  });
+}
+
+int rbmdx_set_type_params(rbmdx_ctx* ctx, const double* charge, const double* eps,
+                          const double* sigma, void* stream) {
+  if (!ctx) return RBMDX_E_ARG;
+  return guarded(ctx, [&] {
+    ctx->eng->set_type_params(charge, eps, sigma, (hipStream_t)stream);
   });
 }
 

@@ -293,6 +293,15 @@ struct StepArgs {
   hipEvent_t ev[6] = {};      // optional section timing events
 };
 
+// Charge, eps and sigma per type (kernel argument).
+struct TypeParams {
+  double q[kMaxTypes], eps[kMaxTypes], sig[kMaxTypes];
+};
+// charge[i] = q[type[i]] and the LJ table of the types.
+template <typename R>
+hipError_t launch_type_params(const TypeParams& tp, int ntypes, const int* type, R* charge, int n,
+                              R* lj_tab, hipStream_t s);
+
 // Launch one complete force evaluation (kernels.hip).
 template <typename R>
 hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s);

@@ -2897,6 +2897,36 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
 }
 
 template <typename R>
+__global__ __launch_bounds__(256) void k_type_params(TypeParams tp, int nt, const int* type,
+                                                     R* charge, int n, R* lj_tab) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    charge[i] = (R)tp.q[type[i]];
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k < nt * nt; k += blockDim.x) {
+      // the row as Engine::upload_lj forms it
+      const int a = k / nt, b = k % nt;
+      const double e = sqrt(tp.eps[a] * tp.eps[b]), sg = (tp.sig[a] + tp.sig[b]) / 2.0;
+      R* row = lj_tab + 4 * k;
+      row[0] = (R)-24 * (R)e;
+      row[1] = (R)(sg * sg);
+      row[2] = (R)e;
+      row[3] = (R)sg;
+    }
+}
+
+template <typename R>
+hipError_t launch_type_params(const TypeParams& tp, int ntypes, const int* type, R* charge, int n,
+                              R* lj_tab, hipStream_t s) {
+  hipLaunchKernelGGL((k_type_params<R>), dim3(blocks_for(n, kBlock, 1024)), dim3(kBlock), 0, s,
+                     tp, ntypes, type, charge, n, lj_tab);
+  return hipGetLastError();
+}
+template hipError_t launch_type_params<float>(const TypeParams&, int, const int*, float*, int,
+                                              float*, hipStream_t);
+template hipError_t launch_type_params<double>(const TypeParams&, int, const int*, double*, int,
+                                               double*, hipStream_t);
+
+template <typename R>
 hipError_t launch_export(const Dev<R>& d, const StepArgs<R>& a, int candidates,
                          int cap, hipStream_t s) {
   const Grid& g = a.grid;

@@ -1,0 +1,147 @@
+"""Sizes at which the launch rules change: lanes per atom over list A (8, 4, 2, 1),
+single-cell bricks, the one-block rebuild (at most 16,384 atoms), systems without
+list-A pairs, selection frequencies that are and are not powers of two, and the
+parameters of a training step set on the stream.
+
+Forces against the FP64 oracle at 2e-5 relative RMS (FP32 terms of about 1e-7
+relative, sums of about 100 of them), energies at 1e-5.
+"""
+import numpy as np
+import pytest
+
+from rbmd_amd import ForceContext, RbmdxError, rbe_sample_host, systems
+from tests.refs import reference_force, rel_rms
+
+pytestmark = pytest.mark.gpu
+
+
+def _ctx(s, cfg):
+    ctx = ForceContext(cfg, device=0)
+    ctx.set_system(s.box_lo, s.box_len, s.types, s.ids, s.charges, s.eps, s.sigma)
+    return ctx
+
+
+def _rows(a, device, dtype):
+    import torch
+
+    t = torch.tensor(np.ascontiguousarray(a.T), dtype=dtype, device=device)
+    return list(t.unbind())
+
+
+def _wrap32(pos, L):
+    p = (pos - L * np.floor(pos / L)).astype(np.float32)
+    return np.where(p >= L.astype(np.float32), np.float32(0), p)
+
+
+@pytest.mark.parametrize("n", [130, 1500, 4100, 8193, 16384, 16385, 33000])
+def test_forces_where_the_launch_rules_change(device, n):
+    import torch
+
+    s = systems.electrolyte(n, frac_ion=0.1, seed=21)
+    cfg = systems.ljsalt_config(P=60, cut_off=2.4 if n < 500 else 3.5,
+                                lj_cut_off=2.2, r_core=2.2, skin=0.2)
+    m = rbe_sample_host(0.09, s.box_len, 60, 5, 0)
+    mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
+    ctx = _ctx(s, cfg)
+    rng = np.random.default_rng(n)
+    f = [torch.zeros(n, device=device) for _ in range(3)]
+    # lists built, reused (a tenth of the skin), rebuilt
+    for step, amp in enumerate((0.0, 0.01, 0.15)):
+        p32 = _wrap32(s.pos + amp * rng.uniform(-1, 1, (n, 3)), s.box_len)
+        p = _rows(p32, device, torch.float32)
+        ctx.force(step, *p, *f, m_samples=mt, energy=step != 1, sync=True)
+        Fo, en, vir, ek, vk = reference_force(s, p32, cfg, step, m)
+        assert rel_rms(torch.stack(f, 1).double().cpu().numpy(), Fo) < 2e-5
+        if step != 1:
+            th = ctx.thermo()
+            assert th["e_vdwl"] == pytest.approx(en[0], rel=1e-5)
+            assert th["e_kspace"] == pytest.approx(ek, rel=1e-5)
+            w = np.asarray(vir) + np.asarray(vk)
+            np.testing.assert_allclose(th["virial"], w, rtol=1e-5, atol=1e-5 * np.abs(w).max())
+    assert ctx.thermo()["rebuilds"] >= 2
+
+
+@pytest.mark.parametrize("samples", [1000, 40, 30, 20])
+def test_all_charged_selection_frequencies(device, samples):
+    """Every atom charged (no list A): frequencies 1, 3, 4 and 5."""
+    import torch
+
+    n = 3000
+    s = systems.electrolyte(n, frac_ion=0.5, seed=8)
+    assert np.all(s.charges != 0)
+    cfg = systems.ljsalt_config(P=40, sample_num=samples)
+    m = rbe_sample_host(0.09, s.box_len, 40, 5, 0)
+    mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
+    ctx = _ctx(s, cfg)
+    f = [torch.zeros(n, device=device) for _ in range(3)]
+    p32 = _wrap32(s.pos, s.box_len)
+    p = _rows(p32, device, torch.float32)
+    for energy in (False, True):
+        ctx.force(3, *p, *f, m_samples=mt, energy=energy, sync=True)
+        Fo, en, _, _, _ = reference_force(s, p32, cfg, 3, m)
+        assert rel_rms(torch.stack(f, 1).double().cpu().numpy(), Fo) < 2e-5
+    th = ctx.thermo()
+    assert th["e_vdwl"] == pytest.approx(en[0], rel=1e-5)
+    assert th["pairs_a"] == 0 and th["rbl_frequency"] == {1000: 1, 40: 3, 30: 4, 20: 5}[samples]
+
+
+def test_md_runs_split_anywhere(device):
+    """NVE (no thermostat factor): one run of 9 steps equals runs of 0, 4, 1 and
+    4 bit for bit, with image flags and without."""
+    import torch
+
+    s = systems.electrolyte(700, frac_ion=0.0, seed=4)
+    cfg = systems.lj_config()
+    cfg["execution"] = {"ensemble": "NVE", "timestep": 0.004, "integration_type": "vv"}
+    out = []
+    for runs, flags in (((9,), True), ((0, 4, 1, 4), True), ((9,), False)):
+        ctx = _ctx(s, cfg)
+        ctx.set_masses(np.ones(len(s.eps)))
+        x, v = (_rows(a, device, torch.float64) for a in (s.pos, s.vel))
+        f = [torch.zeros_like(t) for t in x]
+        img = tuple(torch.zeros(s.n, dtype=torch.int32, device=device) for _ in range(3))
+        ctx.md_init(x, v, f, image=img if flags else None)
+        for k in runs:
+            ctx.md_run(k, x, v, f, image=img if flags else None)
+        assert ctx.md_state()["step"] == 9
+        out.append(torch.stack([*x, *v, *f]))
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+def test_type_parameters_on_the_stream(device):
+    """The parameters of a training step: forces bit for bit those of set_charges
+    and set_lj, the energies too (the charge sums per type), and a type may not
+    become charged or neutral."""
+    import torch
+
+    from rbmd_amd.autograd import DifferentiableForce
+
+    s = systems.electrolyte(2000, frac_ion=0.1, seed=6)
+    cfg = systems.ljsalt_config(P=40)
+    m = rbe_sample_host(0.09, s.box_len, 40, 5, 0)
+    mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
+    pos = torch.tensor(_wrap32(s.pos, s.box_len), device=device)
+    model = DifferentiableForce(cfg, s)
+    ref = _ctx(s, cfg)
+    f = [torch.zeros(s.n, device=device) for _ in range(3)]
+    rng = np.random.default_rng(3)
+    for k in range(3):
+        a = 1.0 + 0.1 * rng.normal()
+        Q, e, g = (np.array([a, -a, 0.0]), 1 + 0.1 * rng.normal(size=3),
+                   1 + 0.02 * rng.normal(size=3))
+        par = [torch.tensor(t, device=device) for t in (Q, e, g)]
+        if k == 2:
+            par = [t.cpu() for t in par]
+        F = model(pos, *par, step=k, m_samples=mt)
+        ref.set_charges(Q[s.types])
+        ref.set_lj(e, g)
+        ref.force(k, *pos.t().contiguous().unbind(), *f, m_samples=mt, energy=True, sync=True)
+        # (the reference adds energies: another kernel, the same force terms)
+        assert rel_rms(F.double().cpu().numpy(), torch.stack(f, 1).double().cpu().numpy()) < 1e-6
+        model.ctx.force(k, *pos.t().contiguous().unbind(), *f, m_samples=mt, energy=True,
+                        sync=True)
+        a, b = model.ctx.thermo(), ref.thermo()
+        for q in ("e_vdwl", "e_coul", "e_kspace"):
+            assert a[q] == pytest.approx(b[q], rel=1e-12)
+    with pytest.raises(RbmdxError, match="which atoms are charged"):
+        model(pos, par[0] + 0.5, par[1], par[2], step=0, m_samples=mt)
