@@ -1224,7 +1224,8 @@ class Engine : public EngineBase {
       auto threads = [&](double lanes, int most) {
         return std::min(most, std::max(64, ((int)std::ceil(lanes) + 63) / 64 * 64));
       };
-      grid_.block = threads(per * (1 << grid_.lsh), 512);
+      // (a shared list leaves the list-B wave its place in the block)
+      grid_.block = threads(per * (1 << grid_.lsh), split_ && grid_.lsh > 0 ? 448 : 512);
       // The adjoint's blocks hold 50 KB of LDS and 118 VGPRs a thread: three
       // blocks of four waves fill a CU, and five or six waves per block leave it
       // half empty (2,000,000 atoms, forward and adjoint: 1 lane per atom in 192

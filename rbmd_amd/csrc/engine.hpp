@@ -20,6 +20,7 @@ constexpr int kSmallKeys = 4096;    // and cell keys (LDS counters)
 constexpr int kSkChunk = 1024;   // charged atoms per S(k) block
 constexpr int kVjpSkBlocks = 1024;  // adjoint structure-sum blocks wanted before a chunk grows
 constexpr int kRbeBlocks = 1024; // RBE-force blocks wanted before a block takes more atoms
+constexpr int kMeanParts = 512;  // force partials that every assembly block adds up
 constexpr int kRbeStage = 256;   // k coefficients per LDS stage of the RBE force
 constexpr int kSkAtoms = 256;    // charged atoms per S(k) block (4 waves of 64)
 constexpr int kSkK = 64;         // k-vectors per S(k) block and per reduction block

@@ -2488,7 +2488,8 @@ struct RedArgs {
 // The sums after the pair kernels, a block per component so that each has one
 // short chain of loads (one block for all took 6.7 us, 17 us with energies),
 // and beside them the RBE force blocks (5 us as a launch of its own), which
-// only the assembly needs.
+// only the assembly needs.  Without k-space the sums ride in the assembly
+// instead (launch_force).
 template <typename R>
 __global__ __launch_bounds__(256) void k_reduce(Dev<R> d, Box<R> b, RedArgs a, int ncp,
                                                 int nck, int K, int ash) {
@@ -2523,10 +2524,46 @@ __global__ __launch_bounds__(256) void k_scatter(Dev<R> d, unsigned thr) {
 // With md_kick (the molecular-dynamics step) it applies the closing half-kick
 // v += 0.5 F / m dt ftm2v instead and writes the workgroup's FP64 sum of
 // m v^2 to d.md_part[blockIdx.x].
-template <typename R>
+// SUMS: k_reduce's sums ride here.  The blocks from nasm on take a component
+// each, block 0 the list statistics of a rebuild, and with mean_fix every block
+// adds up the force partials for itself (the same order, so the same mean),
+// which costs less than a launch up to kMeanParts of them.
+template <typename R, bool SUMS>
 __global__ __launch_bounds__(256) void k_assemble(Dev<R> d, int mean_fix, int has_a,
                                                   int has_k, int has_b, R dt,
-                                                  R dt_ftm, int md_kick, R ftm2v) {
+                                                  R dt_ftm, int md_kick, R ftm2v,
+                                                  RedArgs ra, int ncp, int nasm) {
+  __shared__ double smem[6 * 4];
+  __shared__ double s_mean[3];
+  if (SUMS) {
+    const int blk = (int)blockIdx.x - nasm;
+    if (blk >= 0) {
+      if (blk < ncp)
+        reduce_pair(ra.pair_part, ra.npair, ra.part2, ra.npair2, ra.eflag, blk, ra.thermo,
+                    ra.mean, mean_fix, ra.n_global, smem);
+      else
+        reduce_kspace(ra.ks, blk - ncp, ra.thermo, smem);
+      return;
+    }
+    if (blockIdx.x == 0) {
+      const bool rb = rebuild_now(ra.ctrl, ra.thr);
+      __syncthreads();  // every thread has read the decision that i == 0 resets
+      if (rb) reduce_lists(ra.lista_part, ra.nlista, ra.listb_part, ra.nlistb, ra.ctrl, smem);
+      __syncthreads();
+    }
+    if (mean_fix) {
+      double v[3] = {0.0, 0.0, 0.0};
+#pragma unroll 2
+      for (int k = threadIdx.x; k < ra.npair; k += blockDim.x)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v[q] += ra.pair_part[(size_t)q * ra.npair + k];
+      block_sum<3>(v, smem);
+      if (threadIdx.x == 0)
+        for (int q = 0; q < 3; ++q) s_mean[q] = v[q] / ra.n_global;
+      __syncthreads();
+    }
+  }
+  const double* mean = SUMS ? s_mean : d.mean;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     d.ctrl->maxdisp_bits = 0u;
@@ -2545,9 +2582,9 @@ __global__ __launch_bounds__(256) void k_assemble(Dev<R> d, int mean_fix, int ha
     // the neutral atoms): coalesced reads, no gathers through the maps
     R4T<R> f = has_a ? d.fa[i] : make4<R>(R(0), R(0), R(0), R(0));
     if (mean_fix) {
-      f.x -= (R)d.mean[0];
-      f.y -= (R)d.mean[1];
-      f.z -= (R)d.mean[2];
+      f.x -= (R)mean[0];
+      f.y -= (R)mean[1];
+      f.z -= (R)mean[2];
     }
     if (has_b) {
       const R4T<R> g = d.fb[i];
@@ -2587,8 +2624,8 @@ __global__ __launch_bounds__(256) void k_assemble(Dev<R> d, int mean_fix, int ha
     }
   }
   if (md_kick) {  // uniform: every thread of the workgroup reaches the sum
-    __shared__ double smem[16];
     double v[1] = {ke};
+    __syncthreads();  // (smem may still be read above)
     block_sum<1>(v, smem);
     if (threadIdx.x == 0) d.md_part[blockIdx.x] = v[0];
   }
@@ -2794,6 +2831,14 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   // list A holds RBL shell pairs only when the LJ cutoff exceeds r_core
   const bool shell_a = a.pc.rclj2 > a.pc.rs2;
   const bool has_a = list_a_used(p, d.n, d.nc, g);
+  // Without k-space the sums need no launch of their own: they ride in the
+  // assembly, while each of its blocks can add up the mean force for itself
+  // (4,000 LJ atoms with energies 43.6 -> 41.8 us per step).  The RBE force would
+  // have to move as well: beside the pair kernel it spills that kernel's
+  // registers (200,000 atoms 85.4 -> 85.6 us per step), on the list launch it is
+  // not hidden (88.9).
+  const int npair = has_a ? g.nbrick * g.psub : 0;
+  const bool sums = !ks_on && g.qblocks == 0 && (!p.mean_fix || npair <= kMeanParts);
   if (!has_a) {
     // nothing: k_assemble reads no list-A force
   } else if (p.special) {
@@ -2872,7 +2917,7 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   }
   RedArgs ra;
   ra.pair_part = d.pair_part;
-  ra.npair = has_a ? g.nbrick * g.psub : 0;
+  ra.npair = npair;
   ra.part2 = d.pairb_part;
   ra.npair2 = q_grid(g, p.eflag);
   ra.eflag = p.eflag ? 1 : 0;
@@ -2887,11 +2932,20 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   ra.ctrl = d.ctrl;
   ra.thr = a.rebuild_thr;
   ra.ks = ksum;
-  hipLaunchKernelGGL((k_reduce<R>), dim3(ra.ncp() + ra.nck() + 1 + ks.nrbe), dim3(256), 0, s,
-                     d, a.box, ra, ra.ncp(), ra.nck(), K, ks.rbe_ash);
-  hipLaunchKernelGGL((k_assemble<R>), dim3(blocks_for(d.n)), dim3(kBlock), 0,
-                     s, d, p.mean_fix, has_a ? 1 : 0, ks_on ? 1 : 0, p.split ? 1 : 0, (R)a.dt,
-                     (R)a.dt_ftm, a.md_kick, (R)a.ftm2v);
+  const int nasm = blocks_for(d.n), ncp = ra.ncp(), nck = ra.nck();
+#define RBMDX_ASSEMBLE(SUMSv)                                                             \
+  hipLaunchKernelGGL((k_assemble<R, SUMSv>), dim3(nasm + (SUMSv ? ncp + nck : 0)),       \
+                     dim3(kBlock), 0, s, d, p.mean_fix, has_a ? 1 : 0, ks_on ? 1 : 0,    \
+                     p.split ? 1 : 0, (R)a.dt, (R)a.dt_ftm, a.md_kick, (R)a.ftm2v, ra,   \
+                     ncp, nasm)
+  if (sums) {
+    RBMDX_ASSEMBLE(true);
+  } else {
+    hipLaunchKernelGGL((k_reduce<R>), dim3(ncp + nck + 1 + ks.nrbe), dim3(256), 0, s, d, a.box,
+                       ra, ncp, nck, K, ks.rbe_ash);
+    RBMDX_ASSEMBLE(false);
+  }
+#undef RBMDX_ASSEMBLE
   if (a.ev[5]) hipEventRecord(a.ev[5], s);
   return hipGetLastError();
 }
