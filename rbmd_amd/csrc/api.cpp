@@ -1250,7 +1250,15 @@ class Engine : public EngineBase {
         // the list build's groups of 64 charged atoms per cell, with margin
         // for cells above the mean
         const double qpc = (double)nc / grid_.ncell;
-        grid_.dsplit = std::max(1, std::min(16, (int)std::ceil(1.25 * qpc / 64.0)));
+        auto split = [&](int atoms, int most) {
+          return std::max(1, std::min(most, (int)std::ceil(1.25 * qpc / atoms)));
+        };
+        grid_.dls = 2;
+        grid_.dsplit = split(64, 16);
+        if ((int64_t)grid_.ncell * grid_.dsplit < 4 * num_cu_) {
+          grid_.dls = 4;
+          grid_.dsplit = split(16, 64);
+        }
       }
       // mostly neutral: one more wave per brick block takes the charged
       // pairs beside the list-A waves

@@ -103,6 +103,7 @@ struct Grid {
   // blocks per cell of the dense charged-pair list build (64 charged atoms
   // of the cell per block and pass)
   int dsplit = 1;
+  int dls = 2;     // log2 of its lanes per atom
   const int* cell_of_coord = nullptr;  // [ncell] (z*ny+y)*nx+x -> cell id
   const int* coord_of_cell = nullptr;  // [ncell] cell id -> packed x|y<<10|z<<20
   const int* brick_cell0 = nullptr;    // [nbrick+1] first cell id of a brick

@@ -1099,7 +1099,9 @@ __device__ __forceinline__ void list_b_block(const Dev<R>& d, const Box<R>& b,
 
 // Charged-pair candidate list of a mostly charged system.  A cell's charged
 // atoms are taken 64 at a time by blocks of 256 threads, four lanes per atom
-// (g.dsplit blocks per cell, the cell's groups of 64 atoms dealt over them).
+// (g.dsplit blocks per cell, the cell's groups of 64 atoms dealt over them); in
+// small systems, whose cells give too few such blocks, 16 at a time by sixteen
+// lanes per atom (LS = 4; what follows is told for LS = 2).
 // The charged atoms of the stencil cells are staged in LDS, 256 at a time,
 // double-buffered (the next chunk's loads are in flight while the current
 // one is scanned) and padded to whole groups of 64 with far-away sentinels.
@@ -1119,8 +1121,8 @@ __device__ __forceinline__ void list_b_block(const Dev<R>& d, const Box<R>& b,
 constexpr int kDenseCoop = 40;
 constexpr int kDenseBlock = 256;
 
-// Bits 4v (v < NV) of the acceptance mask of one lane: candidate st[4v].
-template <typename R, bool MI, bool SHIFT, int NV>
+// Bits 2^LS v (v < NV) of the acceptance mask of one lane: candidate st[2^LS v].
+template <typename R, bool MI, bool SHIFT, int LS, int NV>
 __device__ __forceinline__ unsigned long long dense_mask(const Box<R>& b,
                                                          const R4T<R>& xi,
                                                          const R4T<R>* st, R r2,
@@ -1128,7 +1130,7 @@ __device__ __forceinline__ unsigned long long dense_mask(const Box<R>& b,
   unsigned long long m = 0;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const R4T<R> xj = st[4 * v];
+    const R4T<R> xj = st[v << LS];
     R dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
     if (MI) {
       dx = min_image<R>(dx, b.L[0], b.half[0]);
@@ -1140,16 +1142,22 @@ __device__ __forceinline__ unsigned long long dense_mask(const Box<R>& b,
       dz -= sz;
     }
     const R d2 = fma_r(dz, dz, fma_r(dy, dy, mul_rn(dx, dx)));
-    m |= (d2 < r2 ? 1ull : 0ull) << (4 * v);
+    m |= (d2 < r2 ? 1ull : 0ull) << (v << LS);
   }
   return m;
 }
 
-// OR over the four lanes of each quad (DPP quad permutations [1,0,3,2] and
-// [2,3,0,1]).
-__device__ __forceinline__ unsigned quad_or(unsigned x) {
+// OR over the 2^LS lanes of an atom: a quad (DPP quad permutations [1,0,3,2] and
+// [2,3,0,1]) or a row of 16 (and rotations by 4 and 8).
+template <int LS>
+__device__ __forceinline__ unsigned lanes_or(unsigned x) {
+  static_assert(LS == 2 || LS == 4, "lanes per atom");
   x |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, false);
   x |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, false);
+  if (LS == 4) {
+    x |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xf, 0xf, false);
+    x |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false);
+  }
   return x;
 }
 
@@ -1185,7 +1193,7 @@ __device__ __forceinline__ DenseCell<R> dense_cell(const Grid& g, const Box<R>& 
   return dc;
 }
 
-template <typename R>
+template <typename R, int LS>
 __device__ __forceinline__ void list_b_dense(const Dev<R>& d, const Box<R>& b,
                                              const Grid& g, int cell, int part, int blk,
                                              R r2, int cap) {
@@ -1199,10 +1207,11 @@ __device__ __forceinline__ void list_b_dense(const Dev<R>& d, const Box<R>& b,
                       make_span(cc[2], g.ext_b[2], g.nc[2])};
   const int nst = sp[0].count * sp[1].count * sp[2].count;
   const R far = sizeof(R) == 4 ? R(1e30) : R(1e200);
-  const int t = (int)threadIdx.x, lane = t & 63, q = t & 3;
+  const int t = (int)threadIdx.x, lane = t & 63, q = t & ((1 << LS) - 1);
+  constexpr int kAtoms = kDenseBlock >> LS;  // atoms per pass
   int mx = 0, sum = 0;
-  for (int i0 = cs + 64 * part; i0 < ce; i0 += 64 * g.dsplit) {
-    const int c = i0 + (t >> 2);
+  for (int i0 = cs + kAtoms * part; i0 < ce; i0 += kAtoms * g.dsplit) {
+    const int c = i0 + (t >> LS);
     const bool act = c < ce;
     const R4T<R> xi = d.xqc[act ? c : cs];
     int* row = d.list_b + (size_t)(act ? c : cs) * cap;
@@ -1264,35 +1273,35 @@ __device__ __forceinline__ void list_b_dense(const Dev<R>& d, const Box<R>& b,
           const R4T<R>* sq = st_x[buf] + k0 + q;
           auto test = [&](auto nv) {
             constexpr int NV = decltype(nv)::value;
-            return cdc.mi ? dense_mask<R, true, false, NV>(b, xi, sq, r2, R(0), R(0), R(0))
-                   : shift ? dense_mask<R, false, true, NV>(b, xi, sq, r2, cdc.s[0],
+            return cdc.mi ? dense_mask<R, true, false, LS, NV>(b, xi, sq, r2, R(0), R(0), R(0))
+                   : shift ? dense_mask<R, false, true, LS, NV>(b, xi, sq, r2, cdc.s[0],
                                                             cdc.s[1], cdc.s[2])
-                           : dense_mask<R, false, false, NV>(b, xi, sq, r2, R(0), R(0),
+                           : dense_mask<R, false, false, LS, NV>(b, xi, sq, r2, R(0), R(0),
                                                              R(0));
           };
           // a last group of at most 32 atoms: the sentinels after them fail
           // every test, so only the first 32 are tested
-          m = nj - k0 <= 32 ? test(std::integral_constant<int, 8>())
-                            : test(std::integral_constant<int, 16>());
+          m = nj - k0 <= 32 ? test(std::integral_constant<int, (32 >> LS)>())
+                            : test(std::integral_constant<int, (64 >> LS)>());
           m <<= q;
         }
-        m = ((unsigned long long)quad_or((unsigned)(m >> 32)) << 32) |
-            quad_or((unsigned)m);
+        m = ((unsigned long long)lanes_or<LS>((unsigned)(m >> 32)) << 32) |
+            lanes_or<LS>((unsigned)m);
         const int self = c - (cjb + k0);
         if (self >= 0 && self < 64) m &= ~(1ull << self);
         const int na = __popcll(m);
         if (__ballot(na > kDenseCoop) != 0ull) {
           // many accepted: the wave writes each atom's entries of the group
           // with one coalesced store, lane k taking staged atom k0 + k
-          const int abase = __builtin_amdgcn_readfirstlane(i0 + ((t & ~63) >> 2));
-          for (int l = 0; l < 16; ++l) {
-            const unsigned lo = __builtin_amdgcn_readlane((unsigned)m, 4 * l);
-            const unsigned hi = __builtin_amdgcn_readlane((unsigned)(m >> 32), 4 * l);
+          const int abase = __builtin_amdgcn_readfirstlane(i0 + ((t & ~63) >> LS));
+          for (int l = 0; l < 64 >> LS; ++l) {
+            const unsigned lo = __builtin_amdgcn_readlane((unsigned)m, l << LS);
+            const unsigned hi = __builtin_amdgcn_readlane((unsigned)(m >> 32), l << LS);
             if ((lo | hi) == 0u) continue;
             const unsigned long long ml = ((unsigned long long)hi << 32) | lo;
             if ((ml >> lane) & 1ull) {
               const unsigned r =
-                  (unsigned)__builtin_amdgcn_readlane(pos, 4 * l) +
+                  (unsigned)__builtin_amdgcn_readlane(pos, l << LS) +
                   __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
               if (r < (unsigned)cap) {
                 const size_t o = (size_t)(abase + l) * cap;
@@ -1302,9 +1311,10 @@ __device__ __forceinline__ void list_b_dense(const Dev<R>& d, const Box<R>& b,
             }
           }
         } else {
-          // few: lane q of an atom appends its candidates 4v + q at their
+          // few: lane q of an atom appends its candidates 2^LS v + q at their
           // ranks in the mask, with their staged types
-          unsigned long long mq = m & (0x1111111111111111ull << q);
+          unsigned long long mq =
+              m & ((LS == 2 ? 0x1111111111111111ull : 0x0001000100010001ull) << q);
           while (mq) {
             const int u = __builtin_ctzll(mq);
             mq &= mq - 1;
@@ -1360,13 +1370,13 @@ __global__ __launch_bounds__(512) void k_lists(Dev<R> d, Box<R> b, Grid g,
     list_b_block<R>(d, b, g, blockIdx.x - g.nbrick, r2b, cap_b);
 }
 
-template <typename R>
+template <typename R, int LS>
 __global__ __launch_bounds__(kDenseBlock) void k_lists_dense(Dev<R> d, Box<R> b, Grid g,
                                                              R r2b, int cap_b, unsigned thr) {
   if (!rebuild_now(d.ctrl, thr)) return;
   // g.dsplit consecutive blocks per cell, each XCD a contiguous range of cells
   const int blk = xcd_brick(blockIdx.x, gridDim.x);
-  list_b_dense<R>(d, b, g, blk / g.dsplit, blk % g.dsplit, blk, r2b, cap_b);
+  list_b_dense<R, LS>(d, b, g, blk / g.dsplit, blk % g.dsplit, blk, r2b, cap_b);
 }
 
 template <typename R>
@@ -2745,9 +2755,12 @@ hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
                        dim3(g.block), 0, s, d, a.box, g, a.pc.r2_list_a,
                        a.pc.r2_list_b, a.p.split, cap_a, cap_b, thr);
   if (dense)
-    hipLaunchKernelGGL((k_lists_dense<R>), dim3(g.ncell * g.dsplit), dim3(kDenseBlock), 0, s,
-                       d, a.box, g,
-                       a.pc.r2_list_b, cap_b, thr);
+    if (g.dls == 2)
+      hipLaunchKernelGGL((k_lists_dense<R, 2>), dim3(g.ncell * g.dsplit), dim3(kDenseBlock), 0,
+                         s, d, a.box, g, a.pc.r2_list_b, cap_b, thr);
+    else
+      hipLaunchKernelGGL((k_lists_dense<R, 4>), dim3(g.ncell * g.dsplit), dim3(kDenseBlock), 0,
+                         s, d, a.box, g, a.pc.r2_list_b, cap_b, thr);
   return hipGetLastError();
 }
 
