@@ -806,7 +806,10 @@ constexpr int kStagePad = 8;  // stage entries the unrolled tests may read past 
 // its atom's entries as it accepts them (16-bit stores).  count_only
 // (cap 0): no writes.  Neighbourhood positions come from the LDS stage when
 // STAGED, else from the sorted arrays.
-template <typename R, bool STAGED, bool MI>
+// One lane per atom (PACK): a group of 8 entries is collected in registers and
+// stored at once, which takes half the instructions of a 16-bit store per entry
+// (and those of one 64-bit address each).
+template <typename R, bool STAGED, bool MI, bool PACK>
 __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
                                              const Grid& g, const Neigh& h,
                                              const SlotTables<kMaxSlots>& t,
@@ -816,7 +819,7 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
   const int i0 = d.key_start[2 * h.cell0], i1 = d.key_start[2 * h.cell1];
   // 2^lsh adjacent lanes per atom, each a contiguous range of the stencil
   // rows: they count their entries first, and their offsets in the row follow
-  const int lsh = g.lsh, sub = (int)threadIdx.x & ((1 << lsh) - 1);
+  const int lsh = PACK ? 0 : g.lsh, sub = (int)threadIdx.x & ((1 << lsh) - 1);
   for (int ii = threadIdx.x; ii < (i1 - i0) << lsh; ii += blockDim.x) {
     const int i = i0 + (ii >> lsh);
     int c[3];
@@ -834,7 +837,23 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
     const size_t n8 = (size_t)d.n * 8;
     constexpr int sh = StageShift<R>::value;
     size_t wo = 0;  // (count >> 3) * n8 + (count & 7), kept as entries are added
+    uint4* gp = reinterpret_cast<uint4*>(row);  // PACK: the current group
+    unsigned w[4] = {0u, 0u, 0u, 0u};           // and its entries, the last on top
+    auto push = [&](unsigned e) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[q] = __builtin_amdgcn_alignbit(w[q + 1], w[q], 16);
+      w[3] = __builtin_amdgcn_alignbit(e, w[3], 16);
+    };
     auto accept = [&](int l) {
+      if (PACK) {
+        push((unsigned)l << sh);
+        ++count;
+        if ((count & 7) == 0) {
+          if (count <= lcap) *gp = make_uint4(w[0], w[1], w[2], w[3]);
+          gp += d.n;
+        }
+        return;
+      }
       if (count < lcap) row[wo] = (uint16_t)(l << sh);
       ++count;
       wo += (count & 7) ? 1 : n8 - 7;
@@ -928,8 +947,13 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
     if ((count & 7) && count <= lcap) {
       // the rest of the last group: the pair kernel's sentinel entry
       const uint16_t sent = (uint16_t)((StageCap<R>::value - 1) << sh);
-      uint16_t* gp = row + (size_t)(count >> 3) * n8;
-      for (int s8 = count & 7; s8 < 8; ++s8) gp[s8] = sent;
+      if (PACK) {
+        for (int s8 = count & 7; s8 < 8; ++s8) push(sent);
+        *gp = make_uint4(w[0], w[1], w[2], w[3]);
+      } else {
+        uint16_t* sp = row + (size_t)(count >> 3) * n8;
+        for (int s8 = count & 7; s8 < 8; ++s8) sp[s8] = sent;
+      }
     }
     d.cnt_a[i] = (lcap == 0 && cap > 0) ? cap + 1 + count : count;
     mx = max(mx, count);
@@ -964,12 +988,19 @@ __device__ __forceinline__ void list_a_brick(const Dev<R>& d, const Box<R>& b,
   // neighbourhoods beyond 16-bit byte offsets are left to the direct scan
   const int lcap = total > (65536 >> StageShift<R>::value) ? 0 : cap;
   int mx = 0, sum = 0;
-  if (staged && !h.mi)
-    list_a_atoms<R, true, false>(d, b, g, h, t, stage, r2, split, lcap, cap, mx, sum);
-  else if (staged)
-    list_a_atoms<R, true, true>(d, b, g, h, t, stage, r2, split, lcap, cap, mx, sum);
+  auto build = [&](auto pack) {
+    constexpr bool P = decltype(pack)::value;
+    if (staged && !h.mi)
+      list_a_atoms<R, true, false, P>(d, b, g, h, t, stage, r2, split, lcap, cap, mx, sum);
+    else if (staged)
+      list_a_atoms<R, true, true, P>(d, b, g, h, t, stage, r2, split, lcap, cap, mx, sum);
+    else
+      list_a_atoms<R, false, true, P>(d, b, g, h, t, stage, r2, split, lcap, cap, mx, sum);
+  };
+  if (g.lsh == 0)
+    build(std::true_type());
   else
-    list_a_atoms<R, false, true>(d, b, g, h, t, stage, r2, split, lcap, cap, mx, sum);
+    build(std::false_type());
   // per-block statistics (folded by k_reduce)
   __shared__ int s_red[2 * 8];
   mx = wave_max_i(mx);
