@@ -189,17 +189,23 @@ __device__ __forceinline__ SpecRow batch_spec_row(const BatchDev& d, int ms, int
 //   Coulomb: per-lane lists of accepted charged atoms [kQList][block];
 //   k-space: the atom tile, per-k coefficients and rho, and partial sums.
 constexpr int kEvalBlock = 256;
-constexpr int kLjList = 44;
+// Accepted stage positions per lane between two evaluations of the list: the
+// force pass, whose registers allow 4 waves per SIMD, takes as few as let a
+// fourth workgroup into a CU's LDS; with energies or CVFF registers allow 3.
+template <bool LEAN>
+struct LjList {
+  static constexpr int value = LEAN ? 24 : 44;
+  static constexpr size_t bytes = (size_t)value * 256 * sizeof(unsigned short);
+};
 constexpr int kStagePad = 64;
 constexpr int kQList = 8;
 constexpr int kKsTile = 256;
 constexpr size_t kStageBytes = (size_t)(kBatchStageCap + kStagePad) * sizeof(float4);
-constexpr size_t kListBytes = (size_t)kLjList * kEvalBlock * sizeof(unsigned short);
 constexpr size_t kGidBytes = (size_t)kBatchStageCap * sizeof(int);
 constexpr size_t kKsBytes = kKsTile * sizeof(float4) + 2 * (size_t)kBatchMaxK * sizeof(float4) +
                             (size_t)kBatchMaxK * sizeof(double2) +
                             2 * (size_t)kEvalBlock * sizeof(double);
-static_assert(kKsBytes <= kStageBytes + kListBytes, "k-space LDS");
+static_assert(kEvalBlock == 256 && kKsBytes <= kStageBytes + LjList<true>::bytes, "k-space LDS");
 
 // r^2 with room for the rounding of a test that shifts another operand across
 // the box edge than the evaluation does: coordinates are within |lo| + L of 0,
@@ -354,12 +360,25 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
         m &= (unsigned)(0xffffffff00000000ull >> rem);
         const int so = li - b0 - k0;
         if ((unsigned)so < 32u) m &= ~(0x80000000u >> so);
-        if (__any(cnt + __popc(m) > kLjList)) drain();
-        while (m) {
-          const int u = __clz((int)m);
-          m &= ~(0x80000000u >> u);
-          list[cnt * T] = (unsigned short)(b0 + k0 + u);
-          ++cnt;
+        auto take = [&](int room) {
+          while (m && cnt < room) {
+            const int u = __clz((int)m);
+            m &= ~(0x80000000u >> u);
+            list[cnt * T] = (unsigned short)(b0 + k0 + u);
+            ++cnt;
+          }
+        };
+        constexpr int kRoom = LjList<!EFLAG && !GEN>::value;
+        if (kRoom >= 32) {
+          if (__any(cnt + __popc(m) > kRoom)) drain();
+          take(kRoom);
+        } else {
+          // evaluated when some lane's list is full
+          for (;;) {
+            take(kRoom);
+            if (!__any(m != 0)) break;
+            drain();
+          }
         }
       }
     }
@@ -374,7 +393,7 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
                                          float fs[3], Acc<float>& a) {
   float4* sx = reinterpret_cast<float4*>(buf);
   unsigned short* list = reinterpret_cast<unsigned short*>(buf + kStageBytes) + threadIdx.x;
-  int* sgid = reinterpret_cast<int*>(buf + kStageBytes + kListBytes);
+  int* sgid = reinterpret_cast<int*>(buf + kStageBytes + LjList<!EFLAG && !GEN>::bytes);
   const Box<float> b = p.box;
   const BrickNb h = batch_brick(p, brick);
   if (threadIdx.x < 64) {
@@ -811,7 +830,8 @@ template <bool RBL, bool EFLAG, bool GEN>
 __global__ __launch_bounds__(kEvalBlock) void kb_eval(BatchDev d, PairConst<float> pc_arg,
                                                       BatchRange rg, int nk, int npg,
                                                       int qlanes) {
-  __shared__ __align__(16) char buf[kStageBytes + kListBytes + (GEN ? kGidBytes : 0)];
+  __shared__ __align__(16) char buf[kStageBytes + LjList<!EFLAG && !GEN>::bytes +
+                                      (GEN ? kGidBytes : 0)];
   __shared__ int soff[kBatchMaxSlots + 1];
   __shared__ int sfirst[kBatchMaxSlots];
   __shared__ int sedge[kBatchMaxSlots];
