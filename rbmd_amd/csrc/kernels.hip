@@ -3060,17 +3060,18 @@ hipError_t launch_export(const Dev<R>& d, const StepArgs<R>& a, int candidates,
 // last bits may vary between runs); everything else is deterministic.
 // ---------------------------------------------------------------------------
 
-// LJ scalars of one pair from its adjoint table row (-24 eps, sigma^2, eps,
-// 1/sigma or 0): f = -24 eps (2 s6 - 1) s6 / u (= eps df/deps), fp = df/du,
-// fs = df/d sigma_ij.
+// LJ scalars of one pair from its adjoint table row (-24 eps, sigma^2, 48 eps,
+// -72 eps / sigma or 0): f = -24 eps (2 s6 - 1) s6 / u (= eps df/deps),
+// fp2 = 2 df/du, fsh = (df/d sigma_ij) / 2.
 template <typename R>
-__device__ __forceinline__ void lj_vjp(const R* row, R u, R& f, R& fp, R& fs) {
+__device__ __forceinline__ void lj_vjp(const R* row, R u, R& f, R& fp2, R& fsh) {
   const R inv = pair_rcp(u);
   const R s2 = row[1] * inv;
   const R s6 = s2 * s2 * s2;
-  f = row[0] * (R(2) * s6 - R(1)) * s6 * inv;
-  fp = R(24) * row[2] * (R(14) * s6 * s6 - R(4) * s6) * inv * inv;
-  fs = R(-144) * row[2] * (R(4) * s6 - R(1)) * s6 * inv * row[3];
+  const R t = s6 * inv;
+  f = row[0] * (R(2) * s6 - R(1)) * t;
+  fp2 = row[2] * (R(14) * s6 - R(4)) * (t * inv);
+  fsh = row[3] * (R(4) * s6 - R(1)) * t;
 }
 
 // erfc Coulomb without the charges: f_C = -qqr2e q_i q_j h(u),
@@ -3131,7 +3132,7 @@ struct VjpAcc {
 template <typename R>
 __device__ __forceinline__ void vjp_flush(float* tab, int nt, int a, const R* s_lj,
                                           const VjpAcc& c) {
-  const R ea = s_lj[4 * (a * nt + a) + 2];
+  const R ea = s_lj[4 * (a * nt + a)] / R(-24);
   if (c.dq != 0.f) atomicAdd(&tab[a], c.dq);
   if (c.de != 0.f && ea > R(0)) atomicAdd(&tab[nt + a], (float)(c.de / (R(2) * ea)));
   if (c.ds != 0.f) atomicAdd(&tab[2 * nt + a], c.ds);
@@ -3185,30 +3186,30 @@ __device__ __forceinline__ void vjp_pair(R dx, R dy, R dz, R u, const R* row,
                                          const R gi[3], const R gj[3], R r[3],
                                          VjpAcc& acc, R ws = R(1), R cij = R(0),
                                          R cji = R(0)) {
-  R flj = 0, fp = 0, fs = 0;
-  if (row) lj_vjp<R>(row, u, flj, fp, fs);
+  R flj = 0, fp2 = 0, fsh = 0;
+  if (row) lj_vjp<R>(row, u, flj, fp2, fsh);
   if (ws != R(1)) {
     flj *= ws;
-    fp *= ws;
-    fs *= ws;
+    fp2 *= ws;
+    fsh *= ws;
   }
   R f = flj, gqb = 0;
   if (coul) {
     R h, hp;
     coul_vjp<R>(pc, u, h, hp);
     f += -pc.qqr2e * qi * qj * h;
-    fp += -pc.qqr2e * qi * qj * hp;
+    fp2 += R(-2) * pc.qqr2e * qi * qj * hp;
     gqb = -pc.qqr2e * h;
   }
   const R hx = wji * gj[0] - wij * gi[0], hy = wji * gj[1] - wij * gi[1],
           hz = wji * gj[2] - wij * gi[2];
   const R hd = hx * dx + hy * dy + hz * dz;
-  r[0] += f * hx + R(2) * fp * hd * dx;
-  r[1] += f * hy + R(2) * fp * hd * dy;
-  r[2] += f * hz + R(2) * fp * hd * dz;
+  r[0] += f * hx + fp2 * hd * dx;
+  r[1] += f * hy + fp2 * hd * dy;
+  r[2] += f * hz + fp2 * hd * dz;
   if (row) {
     acc.de -= (float)(flj * hd);
-    acc.ds -= (float)(R(0.5) * fs * hd);
+    acc.ds -= (float)(fsh * hd);
   }
   if (coul) acc.dq -= (float)(qj * gqb * hd);
   if (coul && ws != R(1)) {
@@ -3240,10 +3241,12 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
   extern __shared__ char dyn_lds[];
   const int nt = pc.ntypes;
   R* s_lj = reinterpret_cast<R*>(dyn_lds);
-  // the LJ table with 1/sigma_ab in place of sigma_ab
+  // the LJ table with 48 eps_ab and -72 eps_ab / sigma_ab (lj_vjp)
   for (int q = threadIdx.x; q < 4 * nt * nt; q += blockDim.x) {
     const R x = lj_tab[q];
-    s_lj[q] = (q & 3) == 3 ? (x > R(0) ? R(1) / x : R(0)) : x;
+    s_lj[q] = (q & 3) == 3   ? (x > R(0) ? R(-72) * lj_tab[q - 1] / x : R(0))
+              : (q & 3) == 2 ? R(48) * x
+                             : x;
   }
   for (int q = threadIdx.x; q < 3 * nt; q += blockDim.x) tab[q] = 0.f;
   const R gm[3] = {(R)v.gmean[0], (R)v.gmean[1], (R)v.gmean[2]};
@@ -3308,7 +3311,7 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
     // Without special bonds or list-A shell pairs, an entry's weight both
     // ways is the force window a_lo < u < a_hi: the entries (and the
     // sentinels that pad the last group) go without branches, a masked one
-    // with finite stand-ins (u = 1, G'_j = 0, weights 0) that add exact zeros.
+    // with finite stand-ins (u = 1, H = 0) that add exact zeros.
     const bool flat = !SPECIAL && (!RBL || !(pc.rclj2 > pc.rs2));
     if (flat && staged && cnt <= d.cap_a) {
       auto run = [&](auto mi) {
@@ -3325,11 +3328,19 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
             R dx, dy, dz;
             const R u = pair_d2<R, MI>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
             const bool in = (u > pc.a_lo) & (u < pc.a_hi);
-            const R w = in ? R(1) : R(0);
-            const R gj[3] = {in ? gq.x : R(0), in ? gq.y : R(0), in ? gq.z : R(0)};
-            const int tj = pair_woff(xj.w) / (4 * (int)sizeof(R));
-            vjp_pair<R>(dx, dy, dz, in ? u : R(1), lrow + 4 * tj, false, pc, R(0), R(0), w,
-                        w, gi, gj, r, acc, R(1));
+            const R hx = in ? gq.x - gi[0] : R(0), hy = in ? gq.y - gi[1] : R(0),
+                    hz = in ? gq.z - gi[2] : R(0);
+            const R* row = reinterpret_cast<const R*>(reinterpret_cast<const char*>(lrow) +
+                                                      pair_woff(xj.w));
+            R f, fp2, fsh;
+            lj_vjp<R>(row, in ? u : R(1), f, fp2, fsh);
+            const R hd = fma_r(hx, dx, fma_r(hy, dy, hz * dz));
+            const R td = fp2 * hd;
+            r[0] = fma_r(f, hx, fma_r(td, dx, r[0]));
+            r[1] = fma_r(f, hy, fma_r(td, dy, r[1]));
+            r[2] = fma_r(f, hz, fma_r(td, dz, r[2]));
+            acc.de -= (float)(f * hd);
+            acc.ds -= (float)(fsh * hd);
           }
         }
       };

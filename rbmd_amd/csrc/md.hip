@@ -227,7 +227,7 @@ __global__ __launch_bounds__(1024) void k_md_thermostat(
     st.ke = st.ke * st.scale * st.scale;
   }
   *out = st;
-  // the next step's opening half, ready for its k_md_first
+  // the next step's opening half, ready for its first kernel
   open_step(st, p, step + 1);
   *open = st;
 }
