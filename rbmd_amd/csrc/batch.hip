@@ -184,8 +184,9 @@ __device__ __forceinline__ SpecRow batch_spec_row(const BatchDev& d, int ms, int
 
 // LDS of kb_eval's workgroups: one buffer for the three roles.
 //   LJ: the stage (position and LJ-row offset), 64 entries of padding that
-//       the unrolled tests may read past a row, then the per-lane lists of accepted stage positions [kLjList][block] and, with
-//       GEN, the staged global ids;
+//       the unrolled tests may read past a row, then the per-lane lists of
+//       accepted stage positions [LjList][block] and, with GEN, the staged
+//       global ids;
 //   Coulomb: per-lane lists of accepted charged atoms [kQList][block];
 //   k-space: the atom tile, per-k coefficients and rho, and partial sums.
 constexpr int kEvalBlock = 256;
@@ -216,6 +217,23 @@ __device__ __forceinline__ float test_r2(const Box<float>& b, float r2) {
   return r2 + 1e-6f * sqrtf(r2) * s;
 }
 
+// Dimensions (a bit each) across whose edge a pair of charged atoms, the first
+// in cell `own`, takes its image as r_j shifted by L before the subtraction;
+// in the others L comes off r_j - r_i, which rounds differently: the last bit
+// decides the class of a pair at a cutoff.  Shifted: the dimensions that a
+// two-cell brick widened by ext_c on both sides does not cover, if that
+// neighbourhood has at most 512 cells.
+__device__ __forceinline__ int coul_shifted(const RepInfo& p, const int own[3]) {
+  int m = 0, cells = 1;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const int w = min(2, p.nc[q] - (own[q] & ~1)) + 2 * p.ext_c[q];
+    if (w < p.nc[q]) m |= 1 << q;
+    cells *= min(w, p.nc[q]);
+  }
+  return cells <= 512 ? m : 0;
+}
+
 // Where an owner's rows wrap (MODE 2 of lj_lane): per dimension the first
 // neighbourhood cell, and the cell count of a dimension of three or four cells
 // (0: its neighbourhood is staged shifted).
@@ -225,6 +243,33 @@ struct WrapLane {
   __device__ __forceinline__ float shift(int q, int k, const Box<float>& b) const {
     const int u = rs[q] + k;
     return nc[q] == 0 ? 0.f : (u < 0 ? -b.L[q] : (u >= nc[q] ? b.L[q] : 0.f));
+  }
+};
+
+// A charged owner near a box edge: dimensions (bits) staged in shifted images
+// in which its pairs with charged atoms take L off r_j - r_i (coul_shifted).
+// Only a distance within rounding of a cutoff is affected, so the stage stays
+// as it is and such a pair, about one in a million, is looked up again.
+struct QEdge {
+  int mask, nslots;
+  const int *soff, *sfirst;
+  const float4* xs;
+  const int* perm;
+  const float* charge;
+  // d^2 and d of the pair with the neighbourhood's atom l
+  __device__ float image(const float4& xi, int l, const Box<float>& b, float& dx, float& dy,
+                         float& dz) const {
+    int s = 0;
+    for (int k = 1; k < nslots; ++k) s = soff[k] <= l ? k : s;
+    const int j = sfirst[s] + (l - soff[s]);
+    if (charge[perm[j]] != 0.f) {
+      const float4 x = xs[j];
+      const float tx = x.x - xi.x, ty = x.y - xi.y, tz = x.z - xi.z;
+      if (mask & 1) dx = fma_r(-rint(tx * b.invL[0]), b.L[0], tx);
+      if (mask & 2) dy = fma_r(-rint(ty * b.invL[1]), b.L[1], ty);
+      if (mask & 4) dz = fma_r(-rint(tz * b.invL[2]), b.L[2], tz);
+    }
+    return fma_r(dz, dz, fma_r(dy, dy, mul_rn(dx, dx)));
   }
 };
 
@@ -243,8 +288,9 @@ struct WrapLane {
 // minimum image as one subtraction of L from r_j - r_i, so that a pair at a
 // cutoff falls on the side the single-box path puts it; the tests shift the
 // owner instead (per row, and in x per side of the wrapped cell: two
-// instructions a test) against test_r2, and the evaluation decides.  MODE 1: some dimension has fewer than three cells, and
-// the tests take the minimum image as well.
+// instructions a test) against test_r2, and the evaluation decides.  MODE 1:
+// some dimension has fewer than three cells, and the tests take the minimum
+// image as well.
 template <bool RBL, bool EFLAG, bool GEN, int MODE>
 __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<float>& b,
                                         const float* s_lj, const float4* sx,
@@ -252,13 +298,15 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
                                         unsigned short* list, int T, const int lo3[3],
                                         const int hi3[3], int rn0, int rn1, int w0, int w1,
                                         bool live, const float4& xi, int li,
-                                        const WrapLane& wl, int sub, int lsh, bool shell, unsigned long long hi,
-                                        const SpecRow& sr, float& fx, float& fy, float& fz,
-                                        Acc<float>& a) {
+                                        const WrapLane& wl, const QEdge& qe, int sub, int lsh,
+                                        bool shell, unsigned long long hi, const SpecRow& sr,
+                                        float& fx, float& fy, float& fz, Acc<float>& a) {
   const float r2 = (EFLAG || GEN) ? fminf(pc.rclj2, pc.rc2) : pc.a_hi;
   const char* lj_row =
       reinterpret_cast<const char*>(s_lj) + (__float_as_int(xi.w) * pc.ntypes);
-  const float r2t = MODE == 2 ? test_r2(b, r2) : r2;
+  const float r2t = test_r2(b, r2);
+  // distances within rounding of a class boundary (none unless qe says so)
+  const float near = qe.mask ? r2t - r2 : -1.f;
   auto d2_of = [&](const float4& xj, float& dx, float& dy, float& dz) {
     return MODE ? pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz)
                 : pair_d2<float, false>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz);
@@ -271,7 +319,10 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
     const int l = on ? list[k * T] : 0;
     const float4 xj = sx[l];
     float dx, dy, dz;
-    const float d2 = d2_of(xj, dx, dy, dz);
+    float d2 = d2_of(xj, dx, dy, dz);
+    bool edge = fabsf(d2 - r2) <= near;
+    if (RBL && (EFLAG || GEN)) edge = edge || fabsf(d2 - pc.rs2) <= near;
+    if (__builtin_expect(edge, 0)) d2 = qe.image(xi, l + w0, b, dx, dy, dz);
     const float2 lj = *reinterpret_cast<const float2*>(lj_row + __float_as_int(xj.w));
     const float inv = pair_rcp(d2);
     const float s2 = lj.y * inv;
@@ -479,6 +530,12 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
     const int ci = d.perm[i];
     const unsigned long long hi = (RBL && GEN) ? rbl_hi(d.gid_s[i]) : 0ull;
     const SpecRow sr = batch_spec_row<GEN>(d, pc.ms, ci);
+    QEdge qe{0, h.nslots, soff, sfirst, d.xs, d.perm, d.charge};
+    if (d.charge[ci] != 0.f) {
+      const int own[3] = {h.o[0] + k[0], h.o[1] + k[1], h.o[2] + k[2]};
+      qe.mask = ~coul_shifted(p, own) &
+                ((p.nc[0] < 5 ? 0 : 1) | (p.nc[1] < 5 ? 0 : 2) | (p.nc[2] < 5 ? 0 : 4));
+    }
     float fx = 0.f, fy = 0.f, fz = 0.f;
     for (int w0 = 0; w0 < total; w0 += kBatchStageCap) {
       const int w1 = min(total, w0 + kBatchStageCap);
@@ -507,16 +564,16 @@ __device__ __forceinline__ void lj_brick(const BatchDev& d, const PairConst<floa
       }
       if (h.mi)
         lj_lane<RBL, EFLAG, GEN, 1>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3, hi3,
-                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, sub,
-                                     lsh, shell, hi, sr, fx, fy, fz, a);
+                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, qe,
+                                     sub, lsh, shell, hi, sr, fx, fy, fz, a);
       else if (unsh)
         lj_lane<RBL, EFLAG, GEN, 2>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3, hi3,
-                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, sub,
-                                     lsh, shell, hi, sr, fx, fy, fz, a);
+                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, qe,
+                                     sub, lsh, shell, hi, sr, fx, fy, fz, a);
       else
         lj_lane<RBL, EFLAG, GEN, 0>(pc, b, s_lj, sx, sgid, soff, list, blockDim.x, lo3, hi3,
-                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, sub,
-                                     lsh, shell, hi, sr, fx, fy, fz, a);
+                                     h.rn[0], h.rn[1], w0, w1, live, xi, li - w0, wl, qe,
+                                     sub, lsh, shell, hi, sr, fx, fy, fz, a);
     }
     fs[0] += fx;
     fs[1] += fy;
@@ -571,16 +628,11 @@ __device__ __forceinline__ void coul_run(const BatchDev& d, const PairConst<floa
   const int rw = qlanes / cw, rl = gl / cw, ql = gl % cw;
   float fx = 0.f, fy = 0.f, fz = 0.f;
   int cnt = 0;
-  // The nearest image of r_j - r_i: across the edge of a dimension that the
-  // two-cell brick widened by ext_c on both sides does not cover, r_j is
-  // shifted by L before the subtraction, else r_j - r_i after it.  The last
-  // bit decides the class of a pair at a cutoff; the tests, which always
+  // The nearest image of r_j - r_i (coul_shifted); the tests, which always
   // shift r_j - r_i, go against test_r2.
   const int own[3] = {cx, cy, cz};
-  bool shifted[3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-    shifted[q] = min(2, p.nc[q] - (own[q] & ~1)) + 2 * p.ext_c[q] < p.nc[q];
+  const int sm = coul_shifted(p, own);
+  const bool shifted[3] = {(sm & 1) != 0, (sm & 2) != 0, (sm & 4) != 0};
   auto image = [&](int q, float x, float y) {
     const float t = y - x, k = rint(t * b.invL[q]);
     return fma_r(-k, b.L[q], shifted[q] ? y : t) - (shifted[q] ? x : 0.f);
