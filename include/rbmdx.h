@@ -238,12 +238,12 @@ int rbmdx_force(rbmdx_ctx* ctx, int64_t step, const void* px, const void* py,
  * the same and are launched one by one on `stream` (no graph instantiation).
  * The per-evaluation scratch (per-block reduction partials, S(k) chunk
  * partials, rho and the per-k coefficients) lives in a static per-device
- * array of 4 MiB (held by every device the library runs on until the
+ * array of 16.1 MiB (held by every device the library runs on until the
  * process ends) instead of the context's buffers; the neighbour lists and
  * sorted arrays are the context's, allocated by rbmdx_set_system and the
  * first rbmdx_force call, and are never grown here (an overflowed list is
  * still evaluated exactly; the next rbmdx_force grows it).
- * Errors: RBMDX_E_CAPACITY when the system's scratch exceeds 4 MiB (the
+ * Errors: RBMDX_E_CAPACITY when the system's scratch exceeds 16.1 MiB (the
  * 200,000-atom electrolyte at P = 200 needs about 0.23 MiB, 2,000,000 atoms
  * at P = 400 about 2.9 MiB), RBMDX_E_STATE before the context's first
  * rbmdx_force call, or with m_samples NULL before the seeded k-sample stream
