@@ -281,7 +281,8 @@ struct QEdge {
 // evaluated at the end of the window (or when it would overflow).  The lpo
 // lanes of an owner each take a contiguous part of every row.
 // Bound by VALU issue.  256 electrolytes (777,841 atoms): 3352 us with every
-// candidate's terms evaluated in one pass at the default shape.
+// candidate's terms evaluated in one pass at the default shape, 512 to 537 us
+// for the whole of kb_eval (Coulomb and k-space blocks beside it) with the lists.
 //
 // MODE 0: every dimension is staged in shifted images.  MODE 2: some dimension
 // has three or four cells.  It is staged unshifted and its pairs take the
