@@ -306,7 +306,8 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
   const char* lj_row =
       reinterpret_cast<const char*>(s_lj) + (__float_as_int(xi.w) * pc.ntypes);
   const float r2t = test_r2(b, r2);
-  // distances within rounding of a class boundary (none unless qe says so)
+  // distances within rounding of a class boundary (none unless qe says so): the
+  // cutoff, which without energies is the core's, and otherwise the core's as well
   const float near = qe.mask ? r2t - r2 : -1.f;
   auto d2_of = [&](const float4& xj, float& dx, float& dy, float& dz) {
     return MODE ? pair_d2_list<float>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, dx, dy, dz)
@@ -322,7 +323,9 @@ __device__ __forceinline__ void lj_lane(const PairConst<float>& pc, const Box<fl
     float dx, dy, dz;
     float d2 = d2_of(xj, dx, dy, dz);
     bool edge = fabsf(d2 - r2) <= near;
-    if (RBL && (EFLAG || GEN)) edge = edge || fabsf(d2 - pc.rs2) <= near;
+    if (RBL && (EFLAG || GEN)) edge = edge || fabsf(d2 - pc.t_core) <= near;
+    if (RBL && GEN)  // the shell's bounds
+      edge = edge || fabsf(d2 - pc.rs2) <= near || fabsf(d2 - pc.t_shell) <= near;
     if (__builtin_expect(edge, 0)) d2 = qe.image(xi, l + w0, b, dx, dy, dz);
     const float2 lj = *reinterpret_cast<const float2*>(lj_row + __float_as_int(xj.w));
     const float inv = pair_rcp(d2);

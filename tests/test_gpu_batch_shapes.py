@@ -124,6 +124,52 @@ def test_pairs_at_the_cutoff_across_an_edge(device, q, rc, cells):
         assert float((t - te).abs().max()) < 1e-5
 
 
+@pytest.mark.parametrize("lj_cut", [2.5, 3.2])
+def test_core_pairs_across_an_edge(device, lj_cut):
+    """RBL: pairs of two (weakly charged) ions across an edge of five or six cells,
+    within rounding of the core's bound r_core^2 - 1e-4: the LJ force is there exactly
+    when the FP32 square of the minimum image is below it, in the pass with energies
+    as in the one without.  Beyond it, up to r_core, no class holds the pair."""
+    import torch
+
+    f32 = np.float32
+    rng = np.random.default_rng(11)
+    t_core = f32(f32(2.5) * f32(2.5) - f32(1e-4))
+    reps, want = [], []
+    for r in range(192):
+        L = float(f32(rng.uniform(5.05 * lj_cut, 5.4 * lj_cut)))
+        u = rng.normal(size=3)
+        u[r % 3] = 3.0 * np.sign(u[r % 3])
+        u /= np.linalg.norm(u)
+        x0 = rng.uniform(0.3, 0.7, 3) * L
+        x0[r % 3] = L - 0.3 if u[r % 3] > 0 else 0.3
+        x1 = x0 + u * (np.sqrt(float(t_core)) + rng.uniform(-6e-7, 6e-7))
+        x0, x1 = x0.astype(f32), (x1 - L * np.floor(x1 / L)).astype(f32)
+        d = x1 - x0
+        d = np.where(np.abs(d) > f32(0.5) * f32(L), d - np.copysign(f32(L), d), d)
+        t = f32(d[0] * d[0])
+        for k in (1, 2):  # fused: one rounding
+            t = f32(np.float64(d[k]) * np.float64(d[k]) + np.float64(t))
+        want.append(bool(t < t_core))
+        s = _pair_box(L, np.stack([x0, x1]), 1)
+        s.charges = 1e-3 * s.charges
+        reps.append(s)
+    assert 40 < sum(want) < 152
+    b = BatchContext(systems.ljsalt_config(P=8, lj_cut_off=lj_cut), device=0)
+    b.set_systems(reps)
+    p = torch.tensor(np.concatenate([s.pos for s in reps]).astype(f32), device=device)
+    px, py, pz = (p[:, d].contiguous() for d in range(3))
+    m = torch.zeros(3 * 8 * len(reps), dtype=torch.int32, device=device)
+    m[0::3] = 1
+    f = [torch.zeros(b.n, dtype=torch.float32, device=device) for _ in range(3)]
+    for energy in (False, True):
+        b.force(1, px, py, pz, *f, m_samples=m, energy=energy, sync=True)
+        # the LJ force at the bound is 0.039, all charged terms are below 1e-5
+        F = torch.stack(f, 1).norm(dim=1).cpu().numpy().reshape(-1, 2)
+        got = F > 0.02
+        assert got[:, 0].tolist() == got[:, 1].tolist() == want
+
+
 def test_box_edge_of_a_power_of_two(device):
     """Fewer than three cells per dimension (minimum image per pair), edges a
     power of two, full lists, as many atoms as leave lanes idle."""
