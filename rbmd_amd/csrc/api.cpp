@@ -158,10 +158,14 @@ class Engine : public EngineBase {
         throw Error(RBMDX_E_ARG,
                     "set_charges may not change which atoms are charged");
     (void)any;
+    HIPCHK(hipSetDevice(device_));
+    // evaluations in flight read the current values, type parameters in flight
+    // (set_type_params) would overwrite the new ones
+    HIPCHK(hipDeviceSynchronize());
     q_ = nq;
     upload_charges();
     charge_sums();
-    hipDeviceSynchronize();
+    HIPCHK(hipDeviceSynchronize());
   }
 
   // The charge of every atom as its type's, with the types' LJ parameters
@@ -178,7 +182,8 @@ class Engine : public EngineBase {
           throw Error(RBMDX_E_ARG,
                       "set_charges may not change which atoms are charged");
     HIPCHK(hipSetDevice(device_));
-    // evaluations in flight on another stream read the current values
+    // evaluations in flight on another stream read the current values, and type
+    // parameters in flight there would overwrite the new ones
     if (last_stream_set_ && last_stream_ != s) HIPCHK(hipDeviceSynchronize());
     eps_.assign(eps, eps + ntypes_);
     sig_.assign(sig, sig + ntypes_);
@@ -195,6 +200,9 @@ class Engine : public EngineBase {
     if (!split_)
       for (int i = 0; i < n_; ++i) q_[i] = q[type_[i]];
     HIPCHK(launch_type_params<R>(tp, ntypes_, d_.type, d_.charge, n_, lj_tab_, s));
+    // what is ordered after the last evaluation is ordered after this kernel
+    last_stream_ = s;
+    last_stream_set_ = true;
     self_energy();
   }
 

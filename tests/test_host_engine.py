@@ -1,0 +1,104 @@
+"""The engine's host logic over a stand-in for the HIP runtime (host/hip_stub.cpp, built
+here from the library's own sources): orders of launches and copies, and failures
+half-way, without a GPU."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import rbmd_amd
+from rbmd_amd import RbmdxError, build, systems
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host") / "libhost.so")
+    src = [os.path.join(build.CSRC, f) for f in ("api.cpp", "batch.cpp", "sampler.cpp", "sog.cpp",
+                                                 "data_api.cpp", "lammps_data.cpp", "output.cpp")]
+    flags = ["-O0" if f == "-O2" else f for f in build.CXX_FLAGS]
+    # -Bsymbolic: the stand-in, not the HIP runtime that torch has loaded
+    subprocess.run(["g++", *flags, "-shared", "-Wl,-Bsymbolic", "-Wno-unused-result", "-o", out, *src,
+                    os.path.join(HERE, "host", "hip_stub.cpp"), "-lpthread"], check=True)
+    h = rbmd_amd.load_library(out)
+    h.stub_log.restype = ctypes.c_char_p
+    return h
+
+
+@pytest.fixture
+def stub(lib, monkeypatch):
+    monkeypatch.setattr(rbmd_amd, "_lib", lib)
+    lib.stub_counts(0)
+    lib.stub_clear()
+
+    class Stub:
+        def log(self):
+            out = lib.stub_log().decode().split("\n")[:-1]
+            lib.stub_clear()
+            return out
+
+        fail = staticmethod(lambda name, after: lib.stub_fail(name.encode(), after))
+        counts = staticmethod(lib.stub_counts)
+
+    return Stub()
+
+
+class _Row(np.ndarray):
+    """A host array that the bindings take as a device tensor."""
+
+    def data_ptr(self):
+        return self.ctypes.data
+
+
+def _rows(n, dtype=np.float32):
+    return [np.zeros(n, dtype).view(_Row) for _ in range(3)]
+
+
+def _ctx(n=600, **md):
+    s = systems.electrolyte(n, seed=3)
+    cfg = systems.ljsalt_config(P=8)
+    if md:
+        cfg["execution"] = md
+    ctx = rbmd_amd.ForceContext(cfg, device=0)
+    ctx.set_system(s.box_lo, s.box_len, s.types, s.ids, s.charges, s.eps, s.sigma)
+    return s, ctx
+
+
+A, B = 16, 32  # two streams
+
+
+def _ordered(log, first, then):
+    """Whether every `then` that follows a `first` has a wait in between."""
+    pending = False
+    for e in log:
+        if e.startswith("sync"):
+            pending = False
+        elif e.startswith(then) and pending:
+            return False
+        if e.startswith(first):
+            pending = True
+    return True
+
+
+def test_type_parameters_and_what_follows_them(stub):
+    """The parameters set on a stream are in place before charges copied from the host,
+    or parameters set on another stream."""
+    s, ctx = _ctx()
+    p = (np.array([1.1, -1.1, 0.0]), np.ones(3), np.ones(3))
+    stub.log()
+    ctx.set_type_params(*p, A)
+    ctx.set_charges(1.2 * s.charges)
+    assert _ordered(stub.log(), "type_params", "h2d")
+    ctx.set_type_params(*p, A)
+    ctx.set_lj(np.ones(3), np.ones(3))
+    assert _ordered(stub.log(), "type_params", "h2d")
+    ctx.set_type_params(*p, A)
+    ctx.set_type_params(*p, B)
+    log = stub.log()
+    assert log.index("type_params s16") < log.index("sync") < log.index("type_params s32")
+    # on one stream nothing waits
+    ctx.set_type_params(*p, B)
+    assert stub.log() == ["type_params s32"]
