@@ -312,7 +312,9 @@ int rbmdx_thermo(rbmdx_ctx* ctx, rbmdx_thermo_t* out);
  * rbmdx_md_run: nsteps steps; positions, velocities, image flags and forces
  * are updated in place, the force of the last step is left in fx..fz.  flags:
  * RBMDX_FLAG_ENERGY computes energies every step (always on with the
- * energy-stable rescale); other force flags pass through.
+ * energy-stable rescale); other force flags pass through.  A run that fails
+ * at a step leaves the steps before it done (arrays and thermostat state),
+ * and a later run goes on from there.
  * rbmdx_md_state: synchronise and read the thermostat state.
  */
 int rbmdx_md_init(rbmdx_ctx* ctx, void* px, void* py, void* pz, void* vx,

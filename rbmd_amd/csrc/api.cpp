@@ -386,13 +386,19 @@ class Engine : public EngineBase {
       d_.ix = d_.iy = d_.iz = nullptr;
       md_kick_ = false;
     };
+    int32_t k = 0;
     try {
-      for (int32_t k = 0; k < nsteps; ++k) {
+      for (; k < nsteps; ++k) {
         force(md_step_ + 1, c.px, c.py, c.pz, c.fx, c.fy, c.fz, nullptr, 0, ff, s);
         ++md_step_;
       }
     } catch (...) {
       unbind();
+      // the steps done stay done: closed as at the end of a run, so that a later
+      // run goes on from here (a device that refuses this needs a new start)
+      if (k > 0 &&
+          md_launch_apply(a, md_state_ + kMdStep, md_state_ + kMdClosed, s) != hipSuccess)
+        md_ready_ = false;
       throw;
     }
     unbind();

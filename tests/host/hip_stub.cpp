@@ -25,7 +25,7 @@ std::map<char*, size_t> g_live;     // device allocations
 int g_count_a = 0;                  // list-A count that an evaluation reports
 float g_us = 1.f;                   // what an event pair measures
 struct Graph {
-  std::vector<std::function<void()>> ops;
+  std::vector<std::function<void(hipStream_t)>> ops;  // the launching stream
 };
 Graph* g_capture = nullptr;
 
@@ -42,14 +42,14 @@ std::string on(hipStream_t s) { return " s" + std::to_string((size_t)s); }
 
 hipError_t launch(const std::string& name, hipStream_t s, std::function<void()> f = [] {}) {
   if (fails(name.c_str())) return hipErrorOutOfMemory;
-  auto op = [=] {
-    note(name + on(s));
+  auto op = [=](hipStream_t q) {
+    note(name + on(q));
     f();
   };
   if (g_capture)
     g_capture->ops.push_back(op);
   else
-    op();
+    op(s);
   return hipSuccess;
 }
 
@@ -167,9 +167,9 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t x) {
   delete (Graph*)x;
   return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t) {
+hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t s) {
   if (fails("hipGraphLaunch")) return hipErrorOutOfMemory;
-  for (auto& op : ((Graph*)x)->ops) op();
+  for (auto& op : ((Graph*)x)->ops) op(s);
   return hipSuccess;
 }
 }  // extern "C"

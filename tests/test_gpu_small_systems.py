@@ -108,6 +108,34 @@ def test_md_runs_split_anywhere(device):
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
 
 
+def test_thermostatted_runs_split_anywhere(device):
+    """NVT: a run's end applies the factor that the next step would have taken into its
+    opening one, which rounds each velocity once more (1.1e-16, FP64) per split; nine
+    steps of a liquid multiply a difference by less than ten."""
+    import torch
+
+    s = systems.electrolyte(700, frac_ion=0.0, seed=4)
+    cfg = systems.lj_config()
+    cfg["execution"] = {"ensemble": "NVT", "temp_ctrl_type": "NOSE_HOOVER", "timestep": 0.004,
+                        "temperature": [1.5, 1.2, 0.1], "integration_type": "vv",
+                        "num_steps": 9}
+    out, st = [], []
+    for runs in ((9,), (0, 4, 1, 4)):
+        ctx = _ctx(s, cfg)
+        ctx.set_masses(np.ones(len(s.eps)))
+        x, v = (_rows(a, device, torch.float64) for a in (s.pos, s.vel))
+        f = [torch.zeros_like(t) for t in x]
+        ctx.md_init(x, v, f)
+        for k in runs:
+            ctx.md_run(k, x, v, f)
+        st.append(ctx.md_state())
+        out.append(torch.stack([*x, *v]))
+    assert st[0]["step"] == st[1]["step"] == 9
+    for q in ("temperature", "ke", "t_target", "eta", "eta_dot", "thermostat_energy"):
+        np.testing.assert_allclose(st[1][q], st[0][q], rtol=1e-13, atol=1e-15)
+    assert float((out[1] - out[0]).abs().max()) < 1e-13
+
+
 def test_type_parameters_on_the_stream(device):
     """The parameters of a training step: forces bit for bit those of set_charges
     and set_lj, the energies too (the charge sums per type), and a type may not

@@ -102,3 +102,43 @@ def test_type_parameters_and_what_follows_them(stub):
     # on one stream nothing waits
     ctx.set_type_params(*p, B)
     assert stub.log() == ["type_params s32"]
+
+
+@pytest.mark.parametrize("ensemble", ["NVT", "NVE"])
+def test_md_run_that_fails_half_way(stub, ensemble):
+    """A step that fails (its graph's launch) leaves the completed steps: their state is
+    closed with its factor applied, step and thermostat agree, and a later run goes on."""
+    md = dict(ensemble=ensemble, timestep=0.002, integration_type="vv")
+    if ensemble == "NVT":
+        md.update(temp_ctrl_type="NOSE_HOOVER", temperature=[1.0, 1.0, 0.1])
+    s, ctx = _ctx(**md)
+    ctx.set_masses(np.ones(3))
+    x, v, f = _rows(s.n), _rows(s.n), _rows(s.n)
+    ctx.md_init(x, v, f, stream=A)
+    ctx.md_run(2, x, v, f, stream=A)
+    st = ctx.md_state()
+    assert (st["step"], st["temperature"]) == (2, 2.0)
+    stub.log()
+    stub.fail("hipGraphLaunch", 3)
+    with pytest.raises(RbmdxError):
+        ctx.md_run(5, x, v, f, stream=A)
+    log = stub.log()
+    assert log.count("md_thermostat s16") == 3 and log[-1] == "md_apply s16"
+    st = ctx.md_state()
+    assert (st["step"], st["temperature"]) == (5, 5.0)
+    # before its first step: nothing done, nothing pending
+    stub.log()
+    stub.fail("hipGraphLaunch", 0)
+    with pytest.raises(RbmdxError):
+        ctx.md_run(5, x, v, f, stream=A)
+    assert "md_apply s16" not in stub.log()
+    ctx.md_run(2, x, v, f, stream=A)
+    st = ctx.md_state()
+    assert (st["step"], st["temperature"]) == (7, 7.0)
+    # a state that cannot be closed is not taken for one
+    stub.fail("hipGraphLaunch", 1)
+    stub.fail("md_apply", 0)
+    with pytest.raises(RbmdxError):
+        ctx.md_run(5, x, v, f, stream=A)
+    with pytest.raises(RbmdxError, match="md_init first"):
+        ctx.md_run(1, x, v, f, stream=A)
