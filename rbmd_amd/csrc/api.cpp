@@ -497,7 +497,6 @@ class Engine : public EngineBase {
     grow_if_needed(s);
     int force_rebuild = (flags & RBMDX_FLAG_REBUILD) ? 1 : 0;
     if (lists_stale_) force_rebuild = 1;
-    lists_stale_ = false;
     alloc_vjp();
     StepArgs<R> a = args(step, 0);
     a.force_rebuild = force_rebuild;
@@ -516,6 +515,7 @@ class Engine : public EngineBase {
     a.p.num_k = last_num_k_;
     // the evaluation's lists and sorted tiles (as the forward path builds them)
     HIPCHK(launch_skin_build<R>(d_, a, s));
+    lists_stale_ = false;
     HIPCHK(launch_vjp<R>(d_, vjp_, a, s));
     HIPCHK(hipEventRecord(slot_events_[slot], s));
     slot_used_[slot] = true;
@@ -691,9 +691,9 @@ class Engine : public EngineBase {
     } else {
       grow_if_needed(s);
     }
-    // freshly (re)allocated lists hold no entries yet: rebuild before use
+    // freshly (re)allocated lists hold no entries yet: rebuild before use (they
+    // stay stale until an evaluation that rebuilds them is launched)
     if (lists_stale_) force_rebuild = 1;
-    lists_stale_ = false;
     StepArgs<R> a = args(step, flags);
     a.force_rebuild = force_rebuild;
     // this evaluation's slot of the host-mapped rings: step parameters and,
@@ -800,6 +800,7 @@ class Engine : public EngineBase {
       }
       HIPCHK(launch_step(d_, a, s));
     }
+    lists_stale_ = false;
     HIPCHK(hipEventRecord(slot_events_[slot], s));
     slot_used_[slot] = true;
     last_stream_ = s;
@@ -1753,16 +1754,18 @@ class Engine : public EngineBase {
     if (d_.list_a) release(d_.list_a);
     if (d_.list_b) release(d_.list_b);
     if (d_.list_t) release(d_.list_t);
+    // without lists until all of them are there again (an allocation may fail)
+    d_.list_a = nullptr;
+    d_.list_b = nullptr;
     d_.list_t = nullptr;
+    d_.cap_a = d_.cap_b = 0;
     d_.list_a = alloc<uint16_t>((size_t)cap_a * n_);
-    d_.cap_a = cap_a;
     if (d_.nc > 0) {
       d_.list_b = alloc<int>((size_t)cap_b * d_.nc);
-      d_.cap_b = cap_b;
       if (grid_.qblocks) d_.list_t = alloc<unsigned char>((size_t)cap_b * d_.nc);
-    } else {
-      d_.cap_b = 0;
+      d_.cap_b = cap_b;
     }
+    d_.cap_a = cap_a;
   }
 
   void release(void* p) {

@@ -176,7 +176,10 @@ hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t s) {
 
 namespace rbmdx {
 hipError_t noalloc_scratch_init(int) { return hipSuccess; }
-void* noalloc_scratch(int) { return nullptr; }
+void* noalloc_scratch(int) {
+  static std::vector<char> buf(kNoAllocScratchBytes);
+  return buf.data();
+}
 
 template <typename R>
 hipError_t launch_force(const Dev<R>& d, const StepArgs<R>&, hipStream_t s) {

@@ -142,3 +142,32 @@ def test_md_run_that_fails_half_way(stub, ensemble):
         ctx.md_run(5, x, v, f, stream=A)
     with pytest.raises(RbmdxError, match="md_init first"):
         ctx.md_run(1, x, v, f, stream=A)
+
+
+def test_lists_that_cannot_grow(stub):
+    """Lists that an evaluation outgrew are replaced by the next one; if that fails
+    (allocation, or the capture after it), no later evaluation reads freed lists, and
+    none reads new ones before they are built."""
+    s, ctx = _ctx()
+    x, f = _rows(s.n), _rows(s.n)
+    stub.counts(100)
+    ctx.force(0, *x, *f, stream=A)
+    ctx.force(1, *x, *f, stream=A)
+    stub.log()
+    for k, call in enumerate(("hipMalloc", "hipGraphInstantiate", "hipGraphLaunch")):
+        stub.counts(200 << k)
+        ctx.force(2, *x, *f, stream=A)  # outgrown: the next call allocates
+        stub.fail(call, 0)
+        with pytest.raises(RbmdxError):
+            ctx.force(3, *x, *f, stream=A)
+        assert "force s16" not in stub.log()[2:]
+        with pytest.raises(RbmdxError, match="no lists built yet|neighbour lists"):
+            if call == "hipMalloc":
+                ctx.force_noalloc(3, *x, *f, stream=A)
+            else:
+                ctx.export_candidates()
+        for step in (4, 5):
+            ctx.force(step, *x, *f, stream=A)
+        log = stub.log()
+        assert "force reads freed lists" not in log and log.count("rebuild") == 1
+        assert log.index("rebuild") == log.index("force s16") + 1
