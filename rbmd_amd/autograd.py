@@ -25,8 +25,9 @@ class _ForceFn(torch.autograd.Function):
     @staticmethod
     def forward(fctx, pos, Q, eps, sigma, model, step, m_samples, num_k):
         model._apply(Q, eps, sigma, pos.device)
-        # one transposing copy each way; the rows are the SoA arrays
-        x = pos.t().contiguous()
+        # one transposing copy each way; the rows are the SoA arrays (a copy in any
+        # memory order: the caller may change pos before the backward pass)
+        x = pos.transpose(0, 1).clone(memory_format=torch.contiguous_format)
         f = torch.empty_like(x)
         model.ctx.force(step, *x.unbind()[:3], *f.unbind()[:3], m_samples=m_samples,
                         num_k=num_k)
@@ -35,19 +36,19 @@ class _ForceFn(torch.autograd.Function):
         fctx.step = step
         fctx.pdev = (Q.device, eps.device, sigma.device)
         fctx.pdtype = (Q.dtype, eps.dtype, sigma.dtype)
-        return f[:3].t().contiguous()
+        return f[:3].transpose(0, 1).contiguous()
 
     @staticmethod
     def backward(fctx, gF):
         x, = fctx.saved_tensors
         model = fctx.model
-        g = gF.to(x.dtype).t().contiguous()
+        g = gF.to(x.dtype).transpose(0, 1).contiguous()
         d = torch.empty_like(g)
         nt = model.ntypes
         dparam = torch.empty(3 * nt, dtype=torch.float64, device=x.device)
         model.ctx.force_vjp(fctx.step, *x.unbind()[:3], *g.unbind(), *d.unbind(), dparam,
                             neutral_q=model.neutral_charge_grad)
-        dpos = d.t().contiguous()
+        dpos = d.transpose(0, 1).contiguous()
         grads = [dparam[k * nt:(k + 1) * nt].to(device=dev, dtype=dt)
                  for k, (dev, dt) in enumerate(zip(fctx.pdev, fctx.pdtype))]
         return (dpos, *grads, None, None, None, None)

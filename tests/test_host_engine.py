@@ -171,3 +171,30 @@ def test_lists_that_cannot_grow(stub):
         log = stub.log()
         assert "force reads freed lists" not in log and log.count("rebuild") == 1
         assert log.index("rebuild") == log.index("force s16") + 1
+
+
+@pytest.mark.parametrize("order", ["rows", "columns", "column of one", "one atom"])
+def test_positions_changed_between_forward_and_backward(stub, monkeypatch, order):
+    """The positions of the backward pass are the forward pass's in any memory order of
+    the argument, also when the caller changes its array in between."""
+    import torch
+
+    from rbmd_amd import autograd
+
+    for m in (rbmd_amd, autograd):
+        monkeypatch.setattr(m, "_current_stream", lambda device: A)
+    s = systems.electrolyte(600, frac_ion=0.05, seed=3)
+    model = autograd.DifferentiableForce(systems.ljsalt_config(P=8), s)
+    seen = []
+    monkeypatch.setattr(model.ctx, "force_vjp", lambda step, *a, **k: (
+        seen.extend(t.clone() for t in a[:3]), [t.zero_() for t in (*a[6:9], a[9])]))
+    p = torch.tensor(s.pos.astype(np.float32))
+    base, pos = {"rows": (p, p), "columns": (q := p.t().contiguous(), q.t()),
+                 "column of one": (p, p.unsqueeze(2)), "one atom": (p, p[:1])}[order]
+    want = pos.clone()
+    par = [torch.tensor(a, requires_grad=True) for a in ([1.0, -1.0, 0.0], s.eps, s.sigma)]
+    F = model(pos, *par)
+    assert F.shape == pos.shape
+    base += 1.0
+    F.sum().backward()
+    assert torch.equal(torch.stack(seen, 1), want)
