@@ -475,8 +475,8 @@ int rbmdx_batch_energies(rbmdx_batch* ctx, double* out);
 /* Launch shape (brick width in cells, threads per pair workgroup, persistent
  * pair workgroups per CU, lanes per charged atom): measured on the caller's
  * inputs by coordinate descent over {1, 2} x {64, 128, 256}, {1, 2, 4, 8},
- * {4, 8, 16} and kept; with cache_path, a choice stored for this device and
- * batch shape is reused without measuring and a new one is written there
+ * {4, 8, 16} and kept; with cache_path, a choice stored for this device,
+ * batch shape and version of the kernels is reused without measuring and a new one is written there
  * (JSON).  us_out (may be null) receives the chosen evaluation time in
  * microseconds, 0 when it came from the cache.  The forces written are those
  * of step. */

@@ -645,7 +645,7 @@ class Batch {
     std::ostringstream k;
     k << arch_ << "|cu" << num_cu_ << "|R" << R_ << "|N" << N_ << "|NQ" << NQ_ << "|P"
       << P_ << "|rc" << cfg_.cut_off << "|rl" << cfg_.lj_cut_off << "|" << cfg_.neighbor_type
-      << "|t" << ntypes_ << "|k" << d_.kmode << "|s" << special_;
+      << "|t" << ntypes_ << "|k" << d_.kmode << "|s" << special_ << "|v" << kBatchKernels;
     return k.str();
   }
 

@@ -95,7 +95,12 @@ struct BatchDev {
   long long* epoch = nullptr;     // [1] RBL sampling epoch of the evaluation
 };
 
-// Launch shapes chosen by the autotuner.
+// Launch shapes chosen by the autotuner.  A stored choice holds for the kernels it
+// was measured on: kBatchKernels is part of its key and goes up with every change
+// that moves the best shape (256 boxes of 500 to 8000 atoms: 128 threads, 2
+// workgroups per CU and 8 lanes, once the default, take 1404 us on these kernels,
+// their own best 531).
+constexpr int kBatchKernels = 2;
 struct BatchTune {
   int bw = 2;            // brick width in cells (1 or 2)
   int pair_block = 256;  // threads per pair workgroup

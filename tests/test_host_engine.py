@@ -2,7 +2,9 @@
 here from the library's own sources): orders of launches and copies, and failures
 half-way, without a GPU."""
 import ctypes
+import json
 import os
+import re
 import subprocess
 
 import numpy as np
@@ -198,3 +200,31 @@ def test_positions_changed_between_forward_and_backward(stub, monkeypatch, order
     base += 1.0
     F.sum().backward()
     assert torch.equal(torch.stack(seen, 1), want)
+
+
+def test_stored_launch_shapes_are_those_of_the_kernels(stub, tmp_path):
+    """A shape stored for other kernels (a key without this version) is measured again;
+    one stored for these is taken."""
+    path = tmp_path / "tune.json"
+
+    def tuned():
+        b = rbmd_amd.BatchContext(systems.ljsalt_config(P=8), device=0)
+        b.set_systems([systems.electrolyte(600, seed=3)])
+        x, f = _rows(b.n), _rows(b.n)
+        stub.log()
+        out = b.autotune(0, *x, *f, m_samples=np.ones(24, np.int32).view(_Row),
+                         cache_path=path, stream=A)
+        return out, "batch s16" in stub.log()
+
+    (_, us), measured = tuned()
+    assert measured and us > 0
+    (_, us), measured = tuned()
+    assert not measured and us == 0
+    entries = json.loads(path.read_text())
+    (key, shape), = entries.items()
+    other = re.sub(r"\|v\d+$", "", key)
+    shape.update(pair_block=64, grid_per_cu=1)
+    path.write_text(json.dumps({other: shape, re.sub(r"\|v\d+$", "|v1", key): shape}))
+    (shape, us), measured = tuned()
+    assert measured and us > 0 and shape["grid_per_cu"] > 1
+    assert set(entries) < set(json.loads(path.read_text()))
