@@ -1684,8 +1684,11 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
         else
           list_a_atom<R, RBL, EFLAG, SHELL, false, true, SPECIAL>(
               d, b, pc, s_lj, t, h.nslots, stage, i, cnt, sub_l, lsh, xi, ti, hi, a, sr, sgid);
-      } else if (sub_l == 0) {
-        // list overflow since the last rebuild: scan the 27 cells directly
+      } else {
+        // list overflow since the last rebuild, or a neighbourhood beyond 16-bit
+        // offsets: scan the 27 cells directly, each lane every 2^lsh-th atom of a
+        // cell (16,000 LJ atoms, cutoff 6 sigma: 8129 us with
+        // one of eight lanes, 1027 with all)
         int c[3];
         unpack_coord(g.coord_of_cell[d.cell_s[i]], c);
         const Stencil st = atom_stencil(g, h, c);
@@ -1697,7 +1700,7 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
               const int sl = (st.at(2, kz) * h.cnt[1] + st.at(1, ky)) * h.cnt[0] +
                              st.at(0, kx);
               const int len = t.off[sl + 1] - t.off[sl];
-              for (int k = qi ? t.nq[sl] : 0; k < len; ++k) {
+              for (int k = (qi ? t.nq[sl] : 0) + sub_l; k < len; k += 1 << lsh) {
                 const int jg = t.first[sl] + k;
                 if (jg == i) continue;
                 interact_a<R, RBL, EFLAG, SPECIAL>(pc, b, s_lj, ti, xi, hi, d.xs[jg],
@@ -3367,8 +3370,10 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
           one(dx, dy, dz, u, tj, gj, gidj);
         }
       }
-    } else if (sub == 0) {
-      // unstaged brick or list overflow: scan the 27 cells directly
+    } else {
+      // unstaged brick or list overflow: scan the 27 cells directly, each lane every
+      // 2^lsh-th atom of a cell (16,000 LJ atoms, cutoff 6 sigma, forward and adjoint:
+      // 16.2 ms with one of four lanes, 3.0 with all)
       int c[3];
       unpack_coord(g.coord_of_cell[d.cell_s[i]], c);
       const Stencil st = atom_stencil(g, h, c);
@@ -3380,7 +3385,7 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
             const int sl_ = (st.at(2, kz) * h.cnt[1] + st.at(1, ky)) * h.cnt[0] +
                             st.at(0, kx);
             const int len = t.off[sl_ + 1] - t.off[sl_];
-            for (int kk = qi ? t.nq[sl_] : 0; kk < len; ++kk) {
+            for (int kk = (qi ? t.nq[sl_] : 0) + sub; kk < len; kk += 1 << lsh) {
               const int jg = t.first[sl_] + kk;
               if (jg == i) continue;
               const R4T<R> xj = d.xs[jg];

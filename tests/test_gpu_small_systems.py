@@ -11,6 +11,7 @@ import pytest
 
 from rbmd_amd import ForceContext, RbmdxError, rbe_sample_host, systems
 from tests.refs import reference_force, rel_rms
+from tests.test_gpu_vjp import _oracle as adjoint_oracle, _run as adjoint
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +60,39 @@ def test_forces_where_the_launch_rules_change(device, n):
             w = np.asarray(vir) + np.asarray(vk)
             np.testing.assert_allclose(th["virial"], w, rtol=1e-5, atol=1e-5 * np.abs(w).max())
     assert ctx.thermo()["rebuilds"] >= 2
+
+
+@pytest.mark.parametrize("n,precision", [(2600, "fp32"), (5000, "fp32"), (2600, "fp64")])
+def test_neighbourhoods_beyond_the_stage(device, n, precision):
+    """Long cutoffs: neighbourhoods beyond the LDS stage, with lists (2,600 atoms in
+    FP32) and beyond the lists' 16-bit offsets (direct scans over an atom's lanes).
+    Forces and energies as above, the adjoint as in test_gpu_vjp."""
+    import torch
+
+    s = systems.electrolyte(n, frac_ion=0.1, seed=12)
+    s.sigma = np.array([1.0, 0.95, 1.05])
+    cfg = systems.ljsalt_config(P=40, cut_off=6.0, lj_cut_off=6.0, precision=precision)
+    m = rbe_sample_host(0.09, s.box_len, 40, 5, 0)
+    mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
+    ctx = _ctx(s, cfg)
+    dt = torch.float32 if precision == "fp32" else torch.float64
+    p32 = _wrap32(s.pos, s.box_len)
+    p = _rows(p32, device, dt)
+    f = [torch.zeros_like(t) for t in p]
+    Fo, en, _, _, _ = reference_force(s, p32, cfg, 2, m)
+    for energy in (False, True):
+        ctx.force(2, *p, *f, m_samples=mt, energy=energy, sync=True)
+        assert rel_rms(torch.stack(f, 1).double().cpu().numpy(), Fo) < 2e-5
+    assert ctx.thermo()["e_vdwl"] == pytest.approx(en[0], rel=1e-5)
+    if precision == "fp32":
+        s.pos = p32.astype(np.float64)
+        G = np.random.default_rng(7).normal(size=(n, 3))
+        _, dr, dp = adjoint(ctx, s, device, 2, m, G)
+        _, (dro, *dpo) = adjoint_oracle(s, cfg, 2, m, G)
+        assert rel_rms(dr, dro) < 1e-4
+        for k, want in enumerate(dpo):
+            np.testing.assert_allclose(dp[3 * k:3 * k + 3], want, rtol=0,
+                                       atol=1e-4 * np.abs(want).max())
 
 
 @pytest.mark.parametrize("samples", [1000, 40, 30, 20])
