@@ -817,8 +817,8 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
                                              int split, int lcap, int cap,
                                              int& mx, int& sum) {
   const int i0 = d.key_start[2 * h.cell0], i1 = d.key_start[2 * h.cell1];
-  // 2^lsh adjacent lanes per atom, each a contiguous range of the stencil
-  // rows: they count their entries first, and their offsets in the row follow
+  // 2^lsh adjacent lanes per atom.  Staged, each takes a contiguous range of the
+  // stencil rows: they count their entries first, and their offsets in the row follow
   const int lsh = PACK ? 0 : g.lsh, sub = (int)threadIdx.x & ((1 << lsh) - 1);
   for (int ii = threadIdx.x; ii < (i1 - i0) << lsh; ii += blockDim.x) {
     const int i = i0 + (ii >> lsh);
@@ -858,13 +858,47 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
       ++count;
       wo += (count & 7) ? 1 : n8 - 7;
     };
+    // Unstaged neighbourhoods: the lanes test adjacent candidates of a cell, and a
+    // ballot gives each accepted one its place, so that one pass over the candidates
+    // fills the row in their order.  Counting first and storing in a second pass, a
+    // range of rows per lane, left most of eight lanes waiting for the longest (16,000
+    // LJ atoms with a cutoff of 4 sigma, us per rebuilding evaluation: 576, now 270;
+    // one lane per atom 603).
+    if (!STAGED && !PACK) {
+      const unsigned gm = (1u << (1 << lsh)) - 1u;
+      const int g0 = (int)(threadIdx.x & 63) - sub;
+      for (int kz = 0; kz < st.n[2]; ++kz)
+        for (int ky = 0; ky < st.n[1]; ++ky)
+          for (int kx = 0; kx < st.n[0]; ++kx) {
+            const int sl = (st.at(2, kz) * h.cnt[1] + st.at(1, ky)) * h.cnt[0] + st.at(0, kx);
+            const int l0 = t.off[sl], l1 = t.off[sl + 1], jf = t.first[sl] - l0;
+            constexpr int kBatch = 4;
+            for (int l = (qi ? l0 + t.nq[sl] : l0) + sub; l - sub < l1; l += kBatch << lsh) {
+              R4T<R> xj[kBatch];
+#pragma unroll
+              for (int u = 0; u < kBatch; ++u) xj[u] = d.xs[jf + min(l + (u << lsh), l1 - 1)];
+#pragma unroll
+              for (int u = 0; u < kBatch; ++u) {
+                const int lu = l + (u << lsh);
+                R dx, dy, dz;
+                const R d2 = pair_d2<R>(b, xi.x, xi.y, xi.z, xj[u].x, xj[u].y, xj[u].z, dx,
+                                        dy, dz);
+                const bool ok = lu < l1 && d2 < r2 && lu != self;
+                const unsigned bits = (unsigned)(__ballot(ok) >> g0) & gm;
+                const int e = count + __popc(bits & ((1u << sub) - 1u));
+                if (ok && e < lcap) row[(size_t)(e >> 3) * n8 + (e & 7)] = (uint16_t)(lu << sh);
+                count += __popc(bits);
+              }
+            }
+          }
+    }
     // Staged neighbourhoods scan a stencil row (its x cells are consecutive
     // slots, hence one contiguous stage range) as one run; the charged atoms of
     // each cell are skipped for a charged i.
     const bool rows = STAGED && st.mode[0] != 1;
     const int runlen = rows ? st.n[0] : 1;
     const int nrow = st.n[2] * st.n[1];
-    for (int pass = lsh > 0 ? 0 : 1; pass < 2; ++pass) {
+    for (int pass = !STAGED && !PACK ? 2 : (lsh > 0 ? 0 : 1); pass < 2; ++pass) {
       const bool count_pass = pass == 0;
       for (int row_ = (nrow * sub) >> lsh; row_ < (nrow * (sub + 1)) >> lsh; ++row_) {
         const int kz = row_ / st.n[1], ky = row_ - kz * st.n[1];
@@ -920,12 +954,7 @@ __device__ __forceinline__ void list_a_atoms(const Dev<R>& d, const Box<R>& b,
               R dx, dy, dz;
               const R d2 = pair_d2<R>(b, xi.x, xi.y, xi.z, xj.x, xj.y, xj.z,
                                       dx, dy, dz);
-              if (d2 < r2 && l != self) {
-                if (count_pass)
-                  ++count;
-                else
-                  accept(l);
-              }
+              if (d2 < r2 && l != self) accept(l);
             }
           }
         }
