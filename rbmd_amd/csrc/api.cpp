@@ -1247,6 +1247,11 @@ class Engine : public EngineBase {
       // threads 1636 us, 2 in 320 1856, 4 in 256 1542).
       grid_.vsh = 2;
       grid_.vblock = threads(per * (1 << grid_.vsh), 256);
+      // lanes that stage a cell: as many as it has atoms, with margin (200,000 LJ
+      // atoms, us per evaluation with 8, 16, 32 lanes: 2.2 atoms a cell 106, 119, 146,
+      // 4.4 75, 81, 95, 9 62.4, 61.0, 65.5; 18 57 with 16 or 32)
+      grid_.ssl = 3;
+      while (grid_.ssl < 5 && (1 << grid_.ssl) < 1.25 * apc) ++grid_.ssl;
       // mostly charged systems put nearly all pairs in list B: kernels of
       // their own take them, one wave per charged atom, with one resident
       // round (contiguous runs of atoms per wave): the FP32 force pass runs 6

@@ -91,6 +91,7 @@ struct Grid {
   int lsh = 0;     // log2 of the lanes per atom over list A (build and pair kernel)
   int vsh = 0;     // the same in the adjoint's pair pass, and its threads per block
   int vblock = 64;
+  int ssl = 5;     // log2 of the lanes that stage a cell (stage_rows)
   // a wave of the pair kernel's brick block that takes the brick's charged
   // pairs while the others take list A (0 or 64 threads; mostly neutral
   // systems with one workgroup per brick)

@@ -217,18 +217,18 @@ __device__ __forceinline__ int pair_woff(float w) { return __float_as_int(w); }
 __device__ __forceinline__ int pair_woff(double w) { return (int)w; }
 
 // Visit the neighbourhood's atoms in slot order: load(source row) for every
-// atom, then put(stage position, slot, loaded row).  Half a wave per slot (a
-// cell of a liquid holds about 18 atoms), in batches of 8 slots: the slots'
-// rows first, then all their loads, then the stores, so that a thread waits
+// atom, then put(stage position, slot, loaded row).  2^ssl lanes per slot (half a
+// wave in a liquid, whose cells hold about 18 atoms), in batches of 8 slots: the
+// slots' rows first, then all their loads, then the stores, so that a thread waits
 // for memory once per batch.  No entry looks its slot up: the search of the
 // offsets that lanes over the whole stage need took 24 % of the pair kernel's
 // instructions (200,000 atoms 31.7 -> 30.1 us, 2,000,000 250 -> 225 us).
 template <int NS, typename Load, typename Put>
-__device__ __forceinline__ void stage_rows(const Neigh& h, const SlotTables<NS>& t, Load load,
-                                           Put put) {
+__device__ __forceinline__ void stage_rows(const Neigh& h, const SlotTables<NS>& t, int ssl,
+                                           Load load, Put put) {
   constexpr int kBatch = 8;
-  const int hl = (int)threadIdx.x & 31, nhw = (int)blockDim.x >> 5;
-  for (int s0 = (int)threadIdx.x >> 5; s0 < h.nslots; s0 += kBatch * nhw) {
+  const int w = 1 << ssl, hl = (int)threadIdx.x & (w - 1), nhw = (int)blockDim.x >> ssl;
+  for (int s0 = (int)threadIdx.x >> ssl; s0 < h.nslots; s0 += kBatch * nhw) {
     int off[kBatch], len[kBatch];
     decltype(load(0)) p[kBatch];
 #pragma unroll
@@ -242,7 +242,7 @@ __device__ __forceinline__ void stage_rows(const Neigh& h, const SlotTables<NS>&
     for (int u = 0; u < kBatch; ++u) {
       const int sc = min(s0 + u * nhw, h.nslots - 1);
       if (hl < len[u]) put(off[u] + hl, sc, p[u]);
-      for (int k = hl + 32; k < len[u]; k += 32) put(off[u] + k, sc, load(t.first[sc] + k));
+      for (int k = hl + w; k < len[u]; k += w) put(off[u] + k, sc, load(t.first[sc] + k));
     }
   }
 }
@@ -270,7 +270,7 @@ __device__ __forceinline__ void stage_atoms(const Grid& g, const Box<R>& b,
                                             int* sgid = nullptr) {
   constexpr int kInside = 1 | 1 << 2 | 1 << 4;  // edge code of an unshifted cell
   stage_rows(
-      h, t, [&](int src) { return RowGid<R>{xs[src], sgid ? gid_s[src] : 0}; },
+      h, t, g.ssl, [&](int src) { return RowGid<R>{xs[src], sgid ? gid_s[src] : 0}; },
       [&](int l, int slot, const RowGid<R>& r) {
         R4T<R> v = r.v;
         const int e = t.edge[slot];
@@ -3294,7 +3294,7 @@ __global__ __launch_bounds__(512) void k_pair_vjp(Dev<R> d, VjpDev<R> v, Box<R> 
   if (staged) {
     stage_atoms<R, true>(g, b, h, t, d.xs, stage);
     stage_rows(
-        h, t, [&](int src) { return RowGid<R>{v.gs[src], d.gid_s[src]}; },
+        h, t, g.ssl, [&](int src) { return RowGid<R>{v.gs[src], d.gid_s[src]}; },
         [&](int l, int, const RowGid<R>& r) {
           R4T<R> w;
           w.x = r.v.x - gm[0];

@@ -62,6 +62,28 @@ def test_forces_where_the_launch_rules_change(device, n):
     assert ctx.thermo()["rebuilds"] >= 2
 
 
+@pytest.mark.parametrize("rho", [0.08, 0.3, 0.5])
+def test_sparse_cells(device, rho):
+    """Cells of 2, 7 and 11 atoms on average (8 and 16 lanes stage a cell, some cells
+    holding more), with lists shorter than a group of entries per lane."""
+    import torch
+
+    n = 5000
+    s = systems.electrolyte(n, rho=rho, frac_ion=0.1, seed=13)
+    cfg = systems.ljsalt_config(P=40)
+    m = rbe_sample_host(0.09, s.box_len, 40, 5, 0)
+    mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
+    ctx = _ctx(s, cfg)
+    p32 = _wrap32(s.pos, s.box_len)
+    p = _rows(p32, device, torch.float32)
+    f = [torch.zeros_like(t) for t in p]
+    Fo, en, _, _, _ = reference_force(s, p32, cfg, 2, m)
+    for energy in (False, True):
+        ctx.force(2, *p, *f, m_samples=mt, energy=energy, sync=True)
+        assert rel_rms(torch.stack(f, 1).double().cpu().numpy(), Fo) < 2e-5
+    assert ctx.thermo()["e_vdwl"] == pytest.approx(en[0], rel=1e-5)
+
+
 @pytest.mark.parametrize("n,precision", [(2600, "fp32"), (5000, "fp32"), (2600, "fp64")])
 def test_neighbourhoods_beyond_the_stage(device, n, precision):
     """Long cutoffs: neighbourhoods beyond the LDS stage, with lists (2,600 atoms in
