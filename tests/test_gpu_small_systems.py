@@ -65,11 +65,13 @@ def test_forces_where_the_launch_rules_change(device, n):
 @pytest.mark.parametrize("rho", [0.08, 0.3, 0.5])
 def test_sparse_cells(device, rho):
     """Cells of 2, 7 and 11 atoms on average (8 and 16 lanes stage a cell, some cells
-    holding more), with lists shorter than a group of entries per lane."""
+    holding more), with lists shorter than a group of entries per lane.  No pair is
+    closer than sigma, where rounding a coordinate shifted across the edge (4e-6)
+    would move the energy by 12 times as much as r."""
     import torch
 
     n = 5000
-    s = systems.electrolyte(n, rho=rho, frac_ion=0.1, seed=13)
+    s = systems.electrolyte(n, rho=rho, frac_ion=0.1, d_min=1.0, seed=13)
     cfg = systems.ljsalt_config(P=40)
     m = rbe_sample_host(0.09, s.box_len, 40, 5, 0)
     mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
