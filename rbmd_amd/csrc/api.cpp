@@ -1228,14 +1228,34 @@ class Engine : public EngineBase {
       // up to 8 lanes, which fills waves that the few atoms leave empty; beyond
       // about one wave per SIMD the split costs more (partial groups, the list
       // build's counting pass) than it hides.  LJ fluids, whose blocks have no
-      // list-B wave beside them, gain up to four waves per SIMD.
+      // list-B wave beside them, gain up to four waves per SIMD; two lanes alone pay in
+      // FP64 only.
       // Per step: 4,000 LJ atoms in FP64 66 -> 50 us, a 4,001-atom electrolyte
       // 62 -> 55, 27,000 atoms 61 -> 60, 45,000 66 (67 with two lanes), 200,000 92
-      // (105 with two); 50,000 LJ atoms with energies 104 -> 78, in FP64 115 -> 97.
+      // (105 with two).  LJ with 1, 2, 4 lanes, without / with energies: FP32 50,000
+      // atoms 41/50, 39/55, 39/54, 130,000 48/60, 52/90, 54/89; FP64 50,000 81/96,
+      // 67/77, 59/70, 130,000 148/178, 120/139, 103/132.
       const int64_t lanes = split_ ? 65536 : 262144;
-      grid_.lsh = 0;
-      while (grid_.lsh < 3 && ((int64_t)n_ << (grid_.lsh + 1)) <= lanes) ++grid_.lsh;
-      const double per = 1.25 * apc * grid_.bw * grid_.bw * grid_.bw;
+      const double mean = apc * grid_.bw * grid_.bw * grid_.bw;  // atoms of a brick
+      // atoms of its neighbourhood, and entries of an atom's list
+      double hood = apc;
+      for (int d = 0; d < 3; ++d) hood *= std::min(grid_.nc[d], grid_.bw + 2);
+      const double entries = (double)n_ / V * 4.0 / 3.0 * M_PI * ra * ra * ra;
+      auto shared = [&](int lsh) {  // 2^lsh lanes per atom pay
+        int64_t most = lanes;
+        if (!split_ && sizeof(R) == 4 && lsh == 1) most = 131072;
+        // eight lanes want a group of 8 entries each (16,000 LJ atoms in FP64, cutoff
+        // 1.5 sigma, 19 entries: 42/46 us, with four lanes 36/38)
+        if (!split_ && lsh == 3 && entries < 64) most = 65536;
+        // beyond the lists' 16-bit offsets atoms scan their cells: more lanes than
+        // the block holds only repeat its passes (60,000 LJ atoms, 480 a brick,
+        // cutoff 8 sigma: 3107 us with one lane, 3591 with four)
+        const bool scans = hood > 65536 / (int)sizeof(R4);
+        return ((int64_t)n_ << lsh) <= most && (!scans || mean * (1 << lsh) <= 512);
+      };
+      grid_.lsh = 3;
+      while (grid_.lsh > 0 && !shared(grid_.lsh)) --grid_.lsh;
+      const double per = 1.25 * mean;
       auto threads = [&](double lanes, int most) {
         return std::min(most, std::max(64, ((int)std::ceil(lanes) + 63) / 64 * 64));
       };
