@@ -1261,12 +1261,19 @@ class Engine : public EngineBase {
       };
       // (a shared list leaves the list-B wave its place in the block)
       grid_.block = threads(per * (1 << grid_.lsh), split_ && grid_.lsh > 0 ? 448 : 512);
-      // The adjoint's blocks hold 50 KB of LDS and 118 VGPRs a thread: three
-      // blocks of four waves fill a CU, and five or six waves per block leave it
-      // half empty (2,000,000 atoms, forward and adjoint: 1 lane per atom in 192
-      // threads 1636 us, 2 in 320 1856, 4 in 256 1542).
+      // The adjoint's blocks hold 50 KB of LDS, three of them a CU: with four waves
+      // each they fill it, with five or six they leave it half empty (2,000,000 atoms,
+      // forward and adjoint: 1 lane per atom in 192 threads 1636 us, 2 in 320 1856, 4
+      // in 256 1542).  Where a CU gets at most two, each takes up to eight waves
+      // (24,000 water atoms 1170 us with four, 748 with eight; 90,000 LJ atoms in 729
+      // bricks 110 and 120); beyond the LDS stage, where atoms scan their cells,
+      // lanes that such a block does not hold only repeat its passes (4,000 LJ atoms
+      // in 8 bricks, cutoff 6 sigma: 1652 us with one lane, 1725 with four).
+      const bool wide = nb <= 2 * num_cu_;
       grid_.vsh = 2;
-      grid_.vblock = threads(per * (1 << grid_.vsh), 256);
+      while (wide && hood >= stage_cap && grid_.vsh > 0 && mean * (1 << grid_.vsh) > 512)
+        --grid_.vsh;
+      grid_.vblock = threads(per * (1 << grid_.vsh), wide ? 512 : 256);
       // lanes that stage a cell: as many as it has atoms, with margin (200,000 LJ
       // atoms, us per evaluation with 8, 16, 32 lanes: 2.2 atoms a cell 106, 119, 146,
       // 4.4 75, 81, 95, 9 62.4, 61.0, 65.5; 18 57 with 16 or 32)
