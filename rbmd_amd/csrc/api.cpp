@@ -1297,12 +1297,21 @@ class Engine : public EngineBase {
         // the list build's groups of 64 charged atoms per cell, with margin
         // for cells above the mean
         const double qpc = (double)nc / grid_.ncell;
+        // (for sixteen lanes 1.6 sqrt(n) at least: a cell of one atom more than its
+        // blocks hold takes a second pass)
         auto split = [&](int atoms, int most) {
-          return std::max(1, std::min(most, (int)std::ceil(1.25 * qpc / atoms)));
+          const double more = atoms < 64 ? 1.6 * std::sqrt(qpc) : 0.0;
+          return std::max(1, std::min(most, (int)std::ceil(std::max(1.25 * qpc, qpc + more) /
+                                                           atoms)));
         };
+        // Sixteen lanes per atom while the blocks of four lanes leave CUs without a
+        // second one.  us per rebuilding evaluation with four / sixteen: water 9,000
+        // (189 blocks of four lanes) 415 / 306, 24,000 (500) 309 / 285, 27,000 (625)
+        // 379 / 423; ions 8,000 (343) 254 / 249, 9,000 (512) 256 / 286, 16,000 (729)
+        // 291 / 370.
         grid_.dls = 2;
         grid_.dsplit = split(64, 16);
-        if ((int64_t)grid_.ncell * grid_.dsplit < 4 * num_cu_) {
+        if ((int64_t)grid_.ncell * grid_.dsplit < 2 * num_cu_) {
           grid_.dls = 4;
           grid_.dsplit = split(16, 64);
         }
