@@ -17,6 +17,8 @@ constexpr int kMaxSpecial = 64;  // CVFF special partners per atom
 constexpr int kSkTile = 8;       // k-vectors per S(k) block
 constexpr int kSmallAtoms = 16384;  // small_rebuild: at most this many atoms
 constexpr int kSmallKeys = 4096;    // and cell keys (LDS counters)
+constexpr int kSmallBlock = 1024;   // threads of its block
+constexpr int kSmallSk = 1024;      // and S(k) blocks beside it
 constexpr int kSkChunk = 1024;   // charged atoms per S(k) block
 constexpr int kVjpSkBlocks = 1024;  // adjoint structure-sum blocks wanted before a chunk grows
 constexpr int kRbeBlocks = 1024; // RBE-force blocks wanted before a block takes more atoms

@@ -509,19 +509,19 @@ __device__ __forceinline__ int cell_key(const Dev<R>& d, const Box<R>& b, const 
   return 2 * cell + ((!split || d.charge[i] == R(0)) ? 1 : 0);
 }
 
-// The rebuild decision, part 2: a block of 256 threads folds the skin-check
-// maxima (every binning block for itself; `first` publishes the result).
+// The rebuild decision, part 2: a block folds the skin-check maxima (every
+// binning block for itself; `first` publishes the result).
 template <typename R>
 __device__ __forceinline__ bool rebuild_decision(const Dev<R>& d, unsigned thr, int nskin,
                                                  bool first) {
-  __shared__ float s_max[4];
+  __shared__ float s_max[16];
   float m = 0.f;
   for (int k = threadIdx.x; k < nskin; k += blockDim.x)
     m = fmaxf(m, d.skin_part[k]);
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
   __syncthreads();
-  m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+  for (int w = 0; w < (int)blockDim.x >> 6; ++w) m = fmaxf(m, s_max[w]);
   if (first && threadIdx.x == 0) d.ctrl->maxdisp_bits = __float_as_uint(m);
   return __float_as_uint(m) > thr;
 }
@@ -539,24 +539,39 @@ __device__ __forceinline__ void bin_block(const Dev<R>& d, const Box<R>& b,
 }
 
 // Binning, cell scans and sorted-order scatter of a small system (at most
-// kSmallAtoms atoms and kSmallKeys keys) in one block of 256 threads, the
-// counters in LDS.  Two launches fewer per evaluation, most of which do not
-// rebuild: 4,000 LJ atoms 47.2 -> 45.8 us per step,
-// 13,824 ions 86.5 -> 84.5.
+// kSmallAtoms atoms and kSmallKeys keys) in one block of kSmallBlock threads, the
+// counters in LDS and every atom's key and slot in registers.  Two launches fewer
+// per evaluation, most of which do not rebuild.  Bound by latency: the positions of
+// 4 atoms a thread are in flight at once.  us per evaluation of an electrolyte
+// without a rebuild / with one, here / with the four launches: 1,500
+// atoms 37.3, 71.2 / 40.9, 75.3; 4,000 37.9, 82.9 / 41.2, 85.1; 8,000 38.2, 79.0 /
+// 41.8, 77.3; 16,384 39.3, 98.4 / 42.7, 87.6 (a run rebuilds every 10 to 20 steps; one
+// that rebuilds on more than a quarter of its evaluations would gain from a limit of
+// 8,192).
 template <typename R>
 __device__ __forceinline__ void small_rebuild(const Dev<R>& d, const Box<R>& b, const Grid& g,
                                               int split, unsigned thr, int nskin) {
   __shared__ int cnt[kSmallKeys];
   __shared__ int smem[33];
   if (!rebuild_decision(d, thr, nskin, true)) return;
-  const int t = threadIdx.x, nt = blockDim.x, ncell = g.ncell;
+  const int t = threadIdx.x, ncell = g.ncell;
+  constexpr int nt = kSmallBlock, kMost = kSmallAtoms / nt, kBatch = 4;
+  static_assert(kSmallAtoms % nt == 0 && kMost % kBatch == 0 && kSmallAtoms <= 1 << 14 &&
+                    kSmallKeys <= 1 << 16,
+                "atoms per thread; key and slot in one word");
+  int ks[kMost];  // slot and, above it, key
   for (int k = t; k < 2 * ncell; k += nt) cnt[k] = 0;
   __syncthreads();
-#pragma unroll 4
-  for (int i = t; i < d.n; i += nt) {
-    const int key = cell_key(d, b, g, split, i);
-    d.key[i] = key;
-    d.slot[i] = atomicAdd(&cnt[key], 1);
+#pragma unroll
+  for (int u0 = 0; u0 < kMost; u0 += kBatch) {
+    if (u0 * nt >= d.n) break;
+    int key[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      key[u] = cell_key(d, b, g, split, min(t + (u0 + u) * nt, d.n - 1));
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (t + (u0 + u) * nt < d.n) ks[u0 + u] = key[u] << 14 | atomicAdd(&cnt[key[u]], 1);
   }
   __syncthreads();
   const int per = (ncell + nt - 1) / nt;  // consecutive cells per thread
@@ -583,8 +598,11 @@ __device__ __forceinline__ void small_rebuild(const Dev<R>& d, const Box<R>& b, 
     d.ctrl->rebuild_count += 1;
   }
   __syncthreads();
-#pragma unroll 4
-  for (int i = t; i < d.n; i += nt) d.perm[cnt[d.key[i]] + d.slot[i]] = i;
+#pragma unroll
+  for (int u = 0; u < kMost; ++u) {
+    const int i = t + u * nt;
+    if (i < d.n) d.perm[cnt[ks[u] >> 14] + (ks[u] & 0x3fff)] = i;
+  }
 }
 
 // Exclusive scans in one block of 1024 threads: key_start over all 2 ncell
@@ -2259,21 +2277,23 @@ __global__ __launch_bounds__(1024) void k_sk_exact(Dev<R> d, Box<R> b, int nchun
   if (threadIdx.x == 0) d.thermo[24] = p.qqr2e * two_pi / p.volume * e[0];
 }
 
-// S(k) partial sums of one block, one lane per k-vector: the kSkAtoms
+// S(k) partial sums of one block of NW waves, one lane per k-vector: the kSkAtoms
 // charged atoms of chunk `chunk` (in the fixed order of xqs) are staged in
-// LDS as fractional coordinates and charge, each wave takes 64 of them with
-// broadcast reads, and lane l of every wave accumulates k = tile * kSkK + l
-// in FP32 over its atoms (two alternating accumulators); the four waves'
+// LDS as fractional coordinates and charge, each wave takes kSkAtoms / NW of them
+// with broadcast reads, and lane l of every wave accumulates k = tile * kSkK + l
+// in FP32 over its atoms (two alternating accumulators); the waves'
 // sums are added in FP64 in wave order into sk_part[chunk][k].  The K
 // integer k-vectors are m_arg (device memory) or, for the sampled stream,
 // the step's ring slot, which k_skin has copied to m_dev.
-template <typename R>
+template <typename R, int NW>
 __device__ __forceinline__ void sk2_block(const Dev<R>& d, const Box<R>& b,
                                           const int* __restrict__ m_arg, int from_ring,
                                           int K, int chunk, int tile) {
+  constexpr int kPer = kSkAtoms / NW;  // atoms per wave
+  static_assert(kPer % 2 == 0 && 64 * NW >= kSkAtoms, "waves of an S(k) block");
   const int* m_src = from_ring ? d.m_dev : m_arg;
   __shared__ float4 s_a[kSkAtoms];
-  __shared__ double s_p[kSkAtoms / 64][2][kSkK];
+  __shared__ double s_p[NW][2][kSkK];
   const int t = (int)threadIdx.x, lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int k0 = tile * kSkK;
@@ -2284,7 +2304,7 @@ __device__ __forceinline__ void sk2_block(const Dev<R>& d, const Box<R>& b,
     float sx, sy, sz;
     frac_coords<R>(b, pp, sx, sy, sz);
     s_a[t] = make_float4(sx, sy, sz, (float)pp.w);
-  } else {
+  } else if (t < kSkAtoms) {
     s_a[t] = make_float4(0.f, 0.f, 0.f, 0.f);  // charge 0 adds nothing
   }
   const int kl = k0 + min(lane, kn - 1);
@@ -2292,9 +2312,9 @@ __device__ __forceinline__ void sk2_block(const Dev<R>& d, const Box<R>& b,
               mz = (float)m_src[3 * kl + 2];
   __syncthreads();
   float re0 = 0.f, im0 = 0.f, re1 = 0.f, im1 = 0.f;
-  const float4* sa = s_a + 64 * wv;
+  const float4* sa = s_a + kPer * wv;
 #pragma unroll 4
-  for (int a = 0; a < 64; a += 2) {
+  for (int a = 0; a < kPer; a += 2) {
     const float4 u = sa[a], v = sa[a + 1];
     float sn, cs, sn1, cs1;
     sincos_rev(fma_r(mx, u.x, fma_r(my, u.y, mz * u.z)), sn, cs);
@@ -2310,7 +2330,7 @@ __device__ __forceinline__ void sk2_block(const Dev<R>& d, const Box<R>& b,
   if (t < kn) {
     double sre = 0.0, sim = 0.0;
 #pragma unroll
-    for (int w = 0; w < kSkAtoms / 64; ++w) {
+    for (int w = 0; w < NW; ++w) {
       sre += s_p[w][0][t];
       sim += s_p[w][1][t];
     }
@@ -2493,17 +2513,18 @@ __global__ __launch_bounds__(256) void k_cellsort_fin(Dev<R> d, Box<R> b, int nc
                     buf);
 }
 
-// A small system's rebuild up to the cell sort (block 0) and the S(k)
-// partials (the blocks after).
+// A small system's rebuild up to the cell sort (block 0) and the S(k) partials
+// (the blocks after, 16 waves each).
 template <typename R>
-__global__ __launch_bounds__(256) void k_small_sk(Dev<R> d, Box<R> b, Grid g, int split,
-                                                  unsigned thr, int nskin, KsArgs ks) {
+__global__ __launch_bounds__(kSmallBlock) void k_small_sk(Dev<R> d, Box<R> b, Grid g, int split,
+                                                          unsigned thr, int nskin, KsArgs ks) {
   if (blockIdx.x == 0) {
     small_rebuild<R>(d, b, g, split, thr, nskin);
     return;
   }
   const int q = (int)blockIdx.x - 1;
-  sk2_block<R>(d, b, ks.m_arg, ks.from_ring, ks.K, q % ks.nchunks, q / ks.nchunks);
+  sk2_block<R, kSmallBlock / 64>(d, b, ks.m_arg, ks.from_ring, ks.K, q % ks.nchunks,
+                                 q / ks.nchunks);
 }
 
 // Binning (blocks [0, nbin)) and the S(k) partials (the blocks after).
@@ -2516,7 +2537,8 @@ __global__ __launch_bounds__(256) void k_bin_sk(Dev<R> d, Box<R> b, Grid g, int 
     return;
   }
   const int q = (int)blockIdx.x - nbin;
-  sk2_block<R>(d, b, ks.m_arg, ks.from_ring, ks.K, q % ks.nchunks, q / ks.nchunks);
+  sk2_block<R, kBlock / 64>(d, b, ks.m_arg, ks.from_ring, ks.K, q % ks.nchunks,
+                            q / ks.nchunks);
 }
 
 // The cell scans (block 0) and the FP64 S(k) reduction (blocks 1 .. ntiles,
@@ -2798,8 +2820,11 @@ hipError_t build_part(const Dev<R>& d, const StepArgs<R>& a, int nskin,
   const bool kon = ks.K > 0;
   const int nsk = kon ? ks.nchunks * ks.ntiles : 0, nfin = kon ? ks.ntiles : 0;
   const int ncb = blocks_for(g.ncell * 64, kBlock);
-  if (d.n <= kSmallAtoms && 2 * g.ncell <= kSmallKeys) {
-    hipLaunchKernelGGL((k_small_sk<R>), dim3(1 + nsk), dim3(kBlock), 0, s, d, a.box, g,
+  // (one block rebuilds a small system, unless its workgroups of 1,024 threads would
+  // carry many S(k) blocks, which run better as 256: 16,384 ions, 2,196 k's with exact
+  // Ewald, 93.8 and 91.2 us per evaluation)
+  if (d.n <= kSmallAtoms && 2 * g.ncell <= kSmallKeys && nsk <= kSmallSk) {
+    hipLaunchKernelGGL((k_small_sk<R>), dim3(1 + nsk), dim3(kSmallBlock), 0, s, d, a.box, g,
                        a.p.split, thr, nskin, ks);
     hipLaunchKernelGGL((k_cellsort_fin<R>), dim3(ncb + nfin), dim3(kBlock), 0, s, d, a.box,
                        g.ncell, thr, a.pc.ms, ncb, ks);

@@ -34,14 +34,17 @@ def _wrap32(pos, L):
     return np.where(p >= L.astype(np.float32), np.float32(0), p)
 
 
-@pytest.mark.parametrize("n", [130, 1500, 4100, 8193, 16384, 16385, 33000])
-def test_forces_where_the_launch_rules_change(device, n):
+@pytest.mark.parametrize("n,ions,P", [(130, 0.1, 60), (1500, 0.1, 60), (4100, 0.1, 60),
+                                      (8193, 0.1, 60), (16384, 0.1, 60), (16385, 0.1, 60),
+                                      (33000, 0.1, 60), (16384, 0.5, 1000), (16384, 0.5, 1040)])
+def test_forces_where_the_launch_rules_change(device, n, ions, P):
+    """Also around 1,024 S(k) blocks (every atom charged, 1,000 and 1,040 k's)."""
     import torch
 
-    s = systems.electrolyte(n, frac_ion=0.1, seed=21)
-    cfg = systems.ljsalt_config(P=60, cut_off=2.4 if n < 500 else 3.5,
+    s = systems.electrolyte(n, frac_ion=ions, seed=21)
+    cfg = systems.ljsalt_config(P=P, cut_off=2.4 if n < 500 else 3.5,
                                 lj_cut_off=2.2, r_core=2.2, skin=0.2)
-    m = rbe_sample_host(0.09, s.box_len, 60, 5, 0)
+    m = rbe_sample_host(0.09, s.box_len, P, 5, 0)
     mt = torch.tensor(m.reshape(-1).astype(np.int32), device=device)
     ctx = _ctx(s, cfg)
     rng = np.random.default_rng(n)
