@@ -1244,9 +1244,10 @@ class Engine : public EngineBase {
       auto shared = [&](int lsh) {  // 2^lsh lanes per atom pay
         int64_t most = lanes;
         if (!split_ && sizeof(R) == 4 && lsh == 1) most = 131072;
-        // eight lanes want a group of 8 entries each (16,000 LJ atoms in FP64, cutoff
-        // 1.5 sigma, 19 entries: 42/46 us, with four lanes 36/38)
-        if (!split_ && lsh == 3 && entries < 64) most = 65536;
+        // eight lanes want three groups of 8 entries among them (16,000 LJ atoms in
+        // FP64, cutoff 1.5 sigma, 19 entries: 42/46 us, with four lanes 36/38; 30,000 at
+        // density 0.4, 37 entries: 45/50 with either, a rebuild 102 and 106)
+        if (!split_ && lsh == 3 && entries < 24) most = 65536;
         // beyond the lists' 16-bit offsets atoms scan their cells: more lanes than
         // the block holds only repeat its passes (60,000 LJ atoms, 480 a brick,
         // cutoff 8 sigma: 3107 us with one lane, 3591 with four)
