@@ -2619,25 +2619,22 @@ __global__ __launch_bounds__(256) void k_scatter(Dev<R> d, unsigned thr) {
 // With md_kick (the molecular-dynamics step) it applies the closing half-kick
 // v += 0.5 F / m dt ftm2v instead and writes the workgroup's FP64 sum of
 // m v^2 to d.md_part[blockIdx.x].
-// SUMS: k_reduce's sums ride here.  The blocks from nasm on take a component
-// each, block 0 the list statistics of a rebuild, and with mean_fix every block
+// SUMS (no k-space): k_reduce's sums ride here.  The blocks from nasm on take a
+// component each, block 0 the list statistics of a rebuild, and with mean_fix every block
 // adds up the force partials for itself (the same order, so the same mean),
 // which costs less than a launch up to kMeanParts of them.
 template <typename R, bool SUMS>
 __global__ __launch_bounds__(256) void k_assemble(Dev<R> d, int mean_fix, int has_a,
                                                   int has_k, int has_b, R dt,
                                                   R dt_ftm, int md_kick, R ftm2v,
-                                                  RedArgs ra, int ncp, int nasm) {
+                                                  RedArgs ra, int nasm) {
   __shared__ double smem[6 * 4];
   __shared__ double s_mean[3];
   if (SUMS) {
     const int blk = (int)blockIdx.x - nasm;
     if (blk >= 0) {
-      if (blk < ncp)
-        reduce_pair(ra.pair_part, ra.npair, ra.part2, ra.npair2, ra.eflag, blk, ra.thermo,
-                    ra.mean, mean_fix, ra.n_global, smem);
-      else
-        reduce_kspace(ra.ks, blk - ncp, ra.thermo, smem);
+      reduce_pair(ra.pair_part, ra.npair, ra.part2, ra.npair2, ra.eflag, blk, ra.thermo,
+                  ra.mean, mean_fix, ra.n_global, smem);
       return;
     }
     if (blockIdx.x == 0) {
@@ -3035,10 +3032,10 @@ hipError_t launch_force(const Dev<R>& d, const StepArgs<R>& a, hipStream_t s) {
   ra.ks = ksum;
   const int nasm = blocks_for(d.n), ncp = ra.ncp(), nck = ra.nck();
 #define RBMDX_ASSEMBLE(SUMSv)                                                             \
-  hipLaunchKernelGGL((k_assemble<R, SUMSv>), dim3(nasm + (SUMSv ? ncp + nck : 0)),       \
+  hipLaunchKernelGGL((k_assemble<R, SUMSv>), dim3(nasm + (SUMSv ? ncp : 0)),             \
                      dim3(kBlock), 0, s, d, p.mean_fix, has_a ? 1 : 0, ks_on ? 1 : 0,    \
                      p.split ? 1 : 0, (R)a.dt, (R)a.dt_ftm, a.md_kick, (R)a.ftm2v, ra,   \
-                     ncp, nasm)
+                     nasm)
   if (sums) {
     RBMDX_ASSEMBLE(true);
   } else {
