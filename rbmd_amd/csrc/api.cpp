@@ -837,7 +837,7 @@ class Engine : public EngineBase {
   };
   GraphKey graph_key(const StepArgs<R>& a) const {
     GraphKey g;
-    std::memset(&g, 0, sizeof g);
+    std::memset((void*)&g, 0, sizeof g);
     const void* p[15] = {d_.px, d_.py, d_.pz, d_.fx, d_.fy, d_.fz, d_.vx, d_.vy,
                          d_.vz, d_.xw, d_.yw, d_.zw, d_.ix, d_.iy, d_.iz};
     for (int q = 0; q < 15; ++q) g.ptr[q] = p[q];

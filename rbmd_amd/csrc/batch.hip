@@ -222,7 +222,12 @@ __device__ __forceinline__ float test_r2(const Box<float>& b, float r2) {
 // in the others L comes off r_j - r_i, which rounds differently: the last bit
 // decides the class of a pair at a cutoff.  Shifted: the dimensions that a
 // two-cell brick widened by ext_c on both sides does not cover, if that
-// neighbourhood has at most 512 cells.
+// neighbourhood has at most kCoulImageCells cells.  Nothing here stages such a
+// neighbourhood: the rule only fixes the rounding of an image, in the form in which
+// stored results and trajectories have it, so that a pair at a cutoff keeps its
+// class.  It follows the owner's cell, so the two directions of a pair within
+// rounding of a boundary (about one in a million) may differ in class.
+constexpr int kCoulImageCells = 512;
 __device__ __forceinline__ int coul_shifted(const RepInfo& p, const int own[3]) {
   int m = 0, cells = 1;
 #pragma unroll
@@ -231,7 +236,7 @@ __device__ __forceinline__ int coul_shifted(const RepInfo& p, const int own[3]) 
     if (w < p.nc[q]) m |= 1 << q;
     cells *= min(w, p.nc[q]);
   }
-  return cells <= 512 ? m : 0;
+  return cells <= kCoulImageCells ? m : 0;
 }
 
 // Where an owner's rows wrap (MODE 2 of lj_lane): per dimension the first

@@ -24,7 +24,7 @@ constexpr int kVjpSkBlocks = 1024;  // adjoint structure-sum blocks wanted befor
 constexpr int kRbeBlocks = 1024; // RBE-force blocks wanted before a block takes more atoms
 constexpr int kMeanParts = 512;  // force partials that every assembly block adds up
 constexpr int kRbeStage = 256;   // k coefficients per LDS stage of the RBE force
-constexpr int kSkAtoms = 256;    // charged atoms per S(k) block (4 waves of 64)
+constexpr int kSkAtoms = 256;    // charged atoms per S(k) block
 constexpr int kSkK = 64;         // k-vectors per S(k) block and per reduction block
 constexpr int kMaxK = 1 << 20;   // k-vector capacity bound
 constexpr int kMaxSlots = 64;    // neighbourhood cells staged per brick

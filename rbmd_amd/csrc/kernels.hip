@@ -11,6 +11,9 @@
 //                 S(k) reduction per k tile (rho_k, per-k energy terms and
 //                 force coefficients)
 //   k_scatter     on a rebuild the scatter into cell order
+//   k_small_sk    small systems, in place of these three: one block does a
+//                 rebuild up to the cell sort beside the S(k) partials, whose
+//                 reduction rides on the sort (k_cellsort_fin)
 //   k_cellsort,   on a rebuild only (early exit otherwise): deterministic
 //   k_lists,      in-cell order and the gather in it; brick-local all-atom
 //   k_lists_dense candidate lists from LDS-staged neighbourhoods and the
@@ -349,28 +352,6 @@ __device__ __forceinline__ void unpack_coord(int packed, int c[3]) {
   c[2] = (packed >> 20) & 1023;
 }
 
-// ---------------------------------------------------------------------------
-// Every evaluation, one thread per caller atom (coalesced reads, scattered
-// writes): the rebuild decision, part 1, and the gather of positions into
-// the cell-sorted tiles in the order of the last rebuild.
-//   * per-block max |r - r_ref|^2 (minimum image), +inf when a rebuild is
-//     forced; k_bin folds the block maxima (the kernel boundary makes them
-//     visible to every block) into ctrl->maxdisp_bits;
-//   * xs[inv_perm[i]] = (r, type + 1/2 if charged), and the charged copy;
-//   * xqs[qpos[i]] = (r, q): the charged atoms in a fixed order (ascending
-//     caller index) for the k-space kernels.
-// When k_bin then decides to rebuild, k_cellsort gathers again in the new
-// order.  The gather runs also when the step ring asks for a rebuild: the
-// order maps always hold a valid order (the identity, without charged
-// copies, until the first rebuild), and k_cellsort overwrites its result.
-// With ctl, the last block is the control block and reads no atoms: it
-// takes the step ring's header (host memory), publishes the sampling epoch,
-// reports a requested rebuild as an infinite block maximum and copies the
-// step's k-sample (kcopy vectors, then with_src their virial-chain sources)
-// from the host-mapped ring slot to HBM for the k-space kernels, all beside
-// the gather.  force (an explicit rebuild of the list builder alone) skips
-// the sorted gather.
-// ---------------------------------------------------------------------------
 // v + 0.5 F / m dt ftm2v evaluated left to right, as RBMD's UpdateVelocity
 // (update_velocity_op.hip.cu:19-21), without contraction into FMA.
 template <typename R>
@@ -399,6 +380,28 @@ __device__ __forceinline__ void md_open_coord(R& x, R& v, R f, R sc, R m, R dt, 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Every evaluation, one thread per caller atom (coalesced reads, scattered
+// writes): the rebuild decision, part 1, and the gather of positions into
+// the cell-sorted tiles in the order of the last rebuild.
+//   * per-block max |r - r_ref|^2 (minimum image), +inf when a rebuild is
+//     forced; k_bin folds the block maxima (the kernel boundary makes them
+//     visible to every block) into ctrl->maxdisp_bits;
+//   * xs[inv_perm[i]] = (r, type + 1/2 if charged), and the charged copy;
+//   * xqs[qpos[i]] = (r, q): the charged atoms in a fixed order (ascending
+//     caller index) for the k-space kernels.
+// When k_bin then decides to rebuild, k_cellsort gathers again in the new
+// order.  The gather runs also when the step ring asks for a rebuild: the
+// order maps always hold a valid order (the identity, without charged
+// copies, until the first rebuild), and k_cellsort overwrites its result.
+// With ctl, the last block is the control block and reads no atoms: it
+// takes the step ring's header (host memory), publishes the sampling epoch,
+// reports a requested rebuild as an infinite block maximum and copies the
+// step's k-sample (kcopy vectors, then with_src their virial-chain sources)
+// from the host-mapped ring slot to HBM for the k-space kernels, all beside
+// the gather.  force (an explicit rebuild of the list builder alone) skips
+// the sorted gather.
+// ---------------------------------------------------------------------------
 // MD: the evaluation of a molecular-dynamics step.  The step's opening (kick,
 // drift, wrap) rides on this pass over the atoms (4.3 us as a kernel of its
 // own at 200,000 atoms).
@@ -672,10 +675,10 @@ __device__ __forceinline__ void scatter_block(const Dev<R>& d, unsigned thr, int
 }
 
 // One wave per cell: both key segments are sorted by caller index (by rank up
-// to 512 atoms, from the lanes' registers, serial by lane 0 beyond), then the cell's atoms are gathered into the sorted tiles:
-// positions (and the charged copy), reference positions for the skin check,
-// sorted ids, RBL hashes and cells, the charged map, inv_perm, and the CVFF
-// special-bond rows (ms per atom).  A cell of at most 64 atoms is gathered in
+// to 512 atoms, from the lanes' registers, serial by lane 0 beyond), then the
+// cell's atoms are gathered into the sorted tiles: positions (and the charged
+// copy), reference positions for the skin check, sorted ids, RBL hashes and cells,
+// the charged map, inv_perm, and the CVFF special-bond rows (ms per atom).  A cell of at most 64 atoms is gathered in
 // one pass with the caller indices taken from the sort's registers.
 template <typename R>
 __device__ __forceinline__ void cellsort_block(const Dev<R>& d, const Box<R>& b, int ncell,
@@ -820,8 +823,8 @@ constexpr int kStagePad = 8;  // stage entries the unrolled tests may read past 
 // All-atom candidate list of one brick: every j != i within r2 among the 27
 // cells around i, except charged-charged pairs when the work is split (those
 // go to list B).  Entries are 16-bit positions in the brick's staged
-// neighbourhood in the interleaved layout of list_a_index; each lane stores
-// its atom's entries as it accepts them (16-bit stores).  count_only
+// neighbourhood in the interleaved layout of list_a_index; lanes that share an
+// atom store its entries as they accept them (16-bit stores).  count_only
 // (cap 0): no writes.  Neighbourhood positions come from the LDS stage when
 // STAGED, else from the sorted arrays.
 // One lane per atom (PACK): a group of 8 entries is collected in registers and
@@ -1670,15 +1673,14 @@ struct kPairWaves {
 };
 
 // Pair forces of one brick.  Phase 1: LJ over list A for every atom of the
-// brick (one lane per atom, neighbours from the LDS stage).  Phase 2: the
+// brick (2^lsh lanes per atom, neighbours from the LDS stage).  Phase 2: the
 // brick's charged atoms add LJ + Coulomb over list B, kChargedLanes lanes per
 // atom.  fa[i] receives the total pair force of atom i.
 // SPECIAL: CVFF special-bond weights (partners looked up by global id).
 template <typename R, bool RBL, bool EFLAG, bool SHELL, bool SPECIAL>
 __global__ __launch_bounds__(512)
-__attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value))) void k_pair(Dev<R> d, Box<R> b, Grid g,
-                                              PairConst<R> pc_arg,
-                                              const R* lj_tab, int split) {
+__attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value))) void k_pair(
+    Dev<R> d, Box<R> b, Grid g, PairConst<R> pc_arg, const R* lj_tab, int split) {
   // the sampling epoch of this evaluation comes from the step ring (k_skin)
   PairConst<R> pc = pc_arg;
   if (RBL) pc.epoch = d.ctrl->epoch;
@@ -1873,14 +1875,15 @@ __attribute__((amdgpu_waves_per_eu(kPairWaves<R, EFLAG, SHELL || SPECIAL>::value
 // j.  Every 64 packed pairs then take LJ, the Coulomb term and the
 // special-bond weight on a full wave without further gathers (but j's global
 // id for special bonds), so with RBL at r_c + skin only the core and the
-// selected shell (about a quarter of a row) reach that part.  Per-atom sums: each lane's terms in ring order, then
-// a fixed tree over the wave; block partials of the thermo sums in `part`
-// (k_reduce's second segment).  Each wave takes a contiguous run of atoms,
+// selected shell (about a quarter of a row) reach that part.  Per-atom sums: each
+// lane's terms in ring order, then a fixed tree over the wave; block partials of
+// the thermo sums in `part` (k_reduce's second segment).  Each wave takes a contiguous run of atoms,
 // and the runs of one XCD are contiguous, so an XCD's L2 holds one region's
 // neighbours.  Bound by the latency of the gathers (TD busy 89 %, VALU 77 %):
 // 72,981 water atoms take 295, 238, 222 and 208 us with 2.5, 4, 5 and 6 waves per
-// SIMD, and 236 with 8, where registers spill; so the force pass is held to 80
-// registers (6 waves) and the grid to one resident round.
+// SIMD, and 236 with 8; so the force pass is held to 80 registers (6 waves, where
+// with RBL and special bonds one register spills, 8 bytes a lane; at 8 waves many do)
+// and the grid to one resident round.
 // ---------------------------------------------------------------------------
 constexpr int kQBatch = 3;  // list steps of 64 entries per load batch
 constexpr int kRing = 256;  // ring entries per wave (>= 63 + 64 * kQBatch)
@@ -1888,9 +1891,8 @@ static_assert(kRing >= 63 + 64 * kQBatch && (kRing & (kRing - 1)) == 0, "ring si
 
 template <typename R, bool RBL, bool EFLAG, bool SPECIAL>
 __global__ __launch_bounds__(64 * kQWaves)
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !EFLAG ? 6 : 4))) void k_pair_b(Dev<R> d, Box<R> b, Grid g,
-                                                      PairConst<R> pc_arg,
-                                                      const R* lj_tab, double* part) {
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !EFLAG ? 6 : 4))) void k_pair_b(
+    Dev<R> d, Box<R> b, Grid g, PairConst<R> pc_arg, const R* lj_tab, double* part) {
   PairConst<R> pc = pc_arg;
   if (RBL) pc.epoch = d.ctrl->epoch;
   __shared__ R4T<R> r_d[kQWaves][kRing];         // (dx, dy, dz, d^2)
