@@ -334,7 +334,7 @@ class ForceContext:
         sigma = np.ascontiguousarray(sigma, dtype=np.float64)
         lo = np.ascontiguousarray(box_lo, dtype=np.float64)
         L = np.ascontiguousarray(box_len, dtype=np.float64)
-        self.n = len(types)
+        self.n, self.ntypes = len(types), len(eps)
         self._check(self.lib.rbmdx_set_system(
             self._h, self.n, _dptr(lo), _dptr(L), _iptr(types), _iptr(ids),
             _dptr(charges), len(eps), _dptr(eps), _dptr(sigma)))
@@ -398,6 +398,8 @@ class ForceContext:
         """Charge, eps and sigma per type (set_charges of charges[type] and
         set_lj) ordered on the stream of the evaluations, without a wait."""
         q, e, s = (np.ascontiguousarray(a, dtype=np.float64) for a in (charges, eps, sigma))
+        if self.n and not q.size == e.size == s.size == self.ntypes:
+            raise ValueError(f"set_type_params takes {self.ntypes} values each, one per type")
         self._check(self.lib.rbmdx_set_type_params(self._h, _dptr(q), _dptr(e), _dptr(s),
                                                    ctypes.c_void_p(stream)))
 

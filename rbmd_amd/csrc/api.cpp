@@ -1963,6 +1963,7 @@ int rbmdx_set_type_params(rbmdx_ctx* ctx, const double* charge, const double* ep
                           const double* sigma, void* stream) {
   if (!ctx) return RBMDX_E_ARG;
   return guarded(ctx, [&] {
+    if (!ctx->eng) throw Error(RBMDX_E_STATE, "context was not created");
     ctx->eng->set_type_params(charge, eps, sigma, (hipStream_t)stream);
   });
 }

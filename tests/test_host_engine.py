@@ -106,6 +106,23 @@ def test_type_parameters_and_what_follows_them(stub):
     assert stub.log() == ["type_params s32"]
 
 
+def test_type_parameters_are_checked(stub, lib):
+    """One value per type; no system and no context are errors."""
+    s, ctx = _ctx()
+    for bad in ((s.charges, s.eps, s.sigma), ([1.0, -1.0], s.eps, s.sigma)):
+        with pytest.raises(ValueError, match="one per type"):
+            ctx.set_type_params(*bad, A)
+    new = rbmd_amd.ForceContext(systems.ljsalt_config(P=8), device=0)
+    with pytest.raises(RbmdxError, match="set_system first"):
+        new.set_type_params([1.0, -1.0, 0.0], s.eps, s.sigma, A)
+    h = ctypes.c_void_p()
+    assert lib.rbmdx_create(b"{", 0, ctypes.byref(h)) != 0
+    one = (ctypes.c_double * 1)(1.0)
+    assert lib.rbmdx_set_type_params(h, one, one, one, None) != 0
+    assert b"not created" in lib.rbmdx_last_error(h)
+    lib.rbmdx_destroy(h)
+
+
 @pytest.mark.parametrize("ensemble", ["NVT", "NVE"])
 def test_md_run_that_fails_half_way(stub, ensemble):
     """A step that fails (its graph's launch) leaves the completed steps: their state is
